@@ -41,6 +41,7 @@ EXPORTED = (
     "fb_gemv_mx_presplit", "fb_mx_presplit_workspace_bytes",
     "fb_jenks2_ssd_host", "fb_jenks2_ssd_workspace", "fb_jenks2_ssd_gpu",
     "fb_jenks2_ssd_filters_host", "fb_jenks2_ssd_filters_gpu",
+    "fb_gemm", "fb_gemm_workspace_bytes",
 )
 
 
@@ -79,6 +80,8 @@ def lib() -> ctypes.CDLL:
         "fb_from_device": (ctypes.c_int, [vp, vp, vp, sp]),
         "fb_dequant_host": (ctypes.c_int, [vp, vp, vp, sp]),
         "fb_gemv": (ctypes.c_int, [vp, vp, vp, sp, vp, sz, vp]),
+        "fb_gemm": (ctypes.c_int, [vp, vp, vp, sp, vp, sz, vp]),
+        "fb_gemm_workspace_bytes": (sz, [sp]),
         "fb_dequant": (ctypes.c_int, [vp, vp, i32, sp, vp]),
         "fb_quantize_gf4_gpu": (ctypes.c_int, [vp, vp, i32, i32, vp, vp, vp]),
         "fb_quantize_e2m1_gpu": (ctypes.c_int, [vp, i32, i32, vp, vp, vp]),
@@ -291,6 +294,19 @@ def _check_gemv_operands(name, wdev, x, y, shape):
                          f"(B={shape.B}, K={shape.K}, N={shape.N})")
     if wdev.numel() < device_bytes(shape):
         raise ValueError("weight stream is smaller than fb_device_bytes(shape)")
+
+
+def gemm(wdev: torch.Tensor, x: torch.Tensor, y: torch.Tensor, shape: FbShape) -> torch.Tensor:
+    """y[B,N] = x'[B,K] . W^T on the GPU for any number of rows (asynchronous on the current
+    stream).  The workspace is the allocator's, for this call only: rotated x and part sums
+    of a long prompt are too large to keep per layer."""
+    _check_gemv_operands("fb_gemm", wdev, x, y, shape)
+    need = lib().fb_gemm_workspace_bytes(ctypes.byref(shape))
+    with torch.cuda.device(x.device):
+        ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
+        check(lib().fb_gemm(_ptr(wdev), _ptr(x), _ptr(y), ctypes.byref(shape),
+                            _ptr(ws) if need else None, need, _stream(x.device)))
+    return y
 
 
 def _mx_refuse(shape: FbShape) -> None:

@@ -1,0 +1,500 @@
+// The 4-bit linear layer on many rows of x (prompts, training batches): y[M, N] = x[M, K] .
+// W^T, one launch over all of x, where 16-row GEMV calls would read and decode the whole
+// weight once per 16 rows.
+//
+// Workgroup tile: (64 RT rows of W) x (16 CT rows of x), 4 waves, one per SIMD; each wave owns
+// RT 16-row weight tiles and all CT column tiles, RT * CT * 4 fp32 accumulators per lane.
+//  - W goes from the device stream straight into MFMA A operands, as in the GEMV: lane L's 16
+//    bytes of a block are row L % 16, item L / 16, so no weight passes through LDS.  Every
+//    weight is decoded once per workgroup.
+//  - x goes through LDS in chunks of 128 K-values: the 32 values of each of a span's four
+//    128-value items that the four k-steps of one 16-byte nibble chunk multiply.  The loads
+//    write LDS directly (no VGPRs, no ds_write); the 16-byte units of an x row are permuted by
+//    unit ^ (row % 16) on the load's source side, which leaves the MFMA B reads (16 rows, 256
+//    bytes apart) without a bank conflict.
+//  - Nibbles and x are requested kBufs - 1 chunks ahead (3 where four chunks fit the LDS that
+//    the occupancy allows, else 1), with one barrier per chunk.
+//  - Each k-step's decode (21 VALU instructions per GF4 row tile, 8 codes per lane) is written
+//    between the MFMAs of the step before it, a half decode per column tile, and the column
+//    tiles are separate scheduling regions: with one or two waves per SIMD the decode only
+//    hides behind the MFMAs if the instruction stream alternates them.
+// What bounds it: E2M1 runs at the matrix cores' power-limited rate (8192 -> 28672, M = 2048:
+// 737 us, 1305 TFLOP/s; the library's bf16 GEMM of 8192^3 reaches 1418 on the same card);
+// GF4 issues as many cycles of decode and MFMA instructions as its MFMAs take (1006 us, 956
+// TFLOP/s; 16-row GEMV calls: 4840 us).  Small M is bound by latency and the x fill of each
+// CU; the K range is then cut into P parts whose fp32 sums gemm_sum adds in part order.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <atomic>
+#include <cstdint>
+
+#include "fourbit.h"
+#include "fourbit_decode.h"
+#include "fourbit_layout.h"
+
+// Host helpers of fourbit_gemv.hip.  Not part of the library's ABI.
+namespace fb_gpu {
+__attribute__((visibility("hidden"))) int cu_count();
+__attribute__((visibility("hidden"))) int rotate_rows(const void* x, void* xo, int rows, int K,
+                                                      int block, hipStream_t hs);
+}  // namespace fb_gpu
+
+namespace {
+
+constexpr int kGemmWaves = 4;
+constexpr int kRowBytes = 256;  // one x row of a chunk: 128 K-values, 32 of each item of a span
+
+typedef __attribute__((address_space(3))) uint8_t lds_byte;
+
+// workgroup barrier once this wave has at most N vector memory operations in flight and has
+// received every LDS read
+template <int N>
+__device__ __forceinline__ void wait_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+struct GemmArgs {
+  const uint8_t* w;
+  const void* x;
+  void* y;
+  float* part;  // P > 1: the parts' fp32 sums [P, M, N]; else null
+  int M, N, K;
+  int GS;       // spans per row
+  int tiles_n, tiles_m;
+  int spp;      // spans per K-part
+  int ydt;
+  int vec;      // y (and part) rows take 4-value stores: N % 4 == 0, 16-byte aligned y
+};
+
+template <int RT, int CT>
+struct GemmTile {
+  static constexpr int kRows = RT * 16 * kGemmWaves;  // rows of W
+  static constexpr int kCols = CT * 16;               // rows of x
+  static constexpr int kBuf = kCols * kRowBytes;      // one staged chunk
+  // CT <= 4: four chunks in at most 64 KiB, so two workgroups share a CU; CT = 8: four chunks
+  // in 128 KiB, one workgroup; CT = 6: two or four would both leave one workgroup per CU
+  static constexpr int kBufs = kBuf * 4 <= 128 * 1024 ? 4 : 2;
+  static constexpr int kOcc = kBuf * kBufs <= 80 * 1024 ? 2 : 1;
+};
+
+template <int FMT, int XDT, int RT, int CT>
+__global__ __launch_bounds__(kGemmWaves * 64, (GemmTile<RT, CT>::kOcc)) void gemm_kernel(GemmArgs a) {
+  using T = GemmTile<RT, CT>;
+  constexpr int BB = FMT == FB_FMT_GF4 ? fb::kGf4BlockBytes : fb::kE2m1BlockBytes;
+  constexpr int NB = T::kBufs, D = NB - 1;
+  constexpr int XD = T::kBuf / (kGemmWaves * 1024);  // 1 KiB x requests of one wave per chunk
+  __shared__ __align__(1024) uint8_t xb0[T::kBuf], xb1[T::kBuf];
+  __shared__ __align__(1024) uint8_t xb2[NB == 4 ? T::kBuf : 16], xb3[NB == 4 ? T::kBuf : 16];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  // Tile of this workgroup.  Workgroups go round-robin over the 8 XCDs: each XCD takes a
+  // contiguous run of tiles, 4 x-tiles by many weight tiles at a time, so that the tiles in
+  // flight on an XCD share x and weights in its L2.
+  const int per = a.tiles_n * a.tiles_m;
+  const int total = gridDim.x;
+  int id = blockIdx.x;
+  {
+    const int q = total >> 3, r = total & 7, xcd = id & 7, k = id >> 3;
+    id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + k;
+  }
+  const int p = id / per;
+  id -= p * per;
+  const int gsz = 4 * a.tiles_n;
+  const int g = id / gsz, gm = min(4, a.tiles_m - g * 4);
+  const int rem = id - g * gsz;
+  const int tn = rem / gm, tm = g * 4 + (rem - tn * gm);
+
+  const int sp0 = p * a.spp, sp1 = min(a.GS, sp0 + a.spp);
+  const int nsp = sp1 - sp0;
+  const int m0 = tm * T::kCols;
+  const int rows = min(T::kCols, a.M - m0);
+  const int row_tiles = (a.N + 15) >> 4;
+  const int t0 = tn * (RT * kGemmWaves) + wave * RT;
+
+  const rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(static_cast<const uint8_t*>(a.x)) + (int64_t)m0 * a.K * 2, (short)0,
+      rows * a.K * 2, kRsrcWord3);
+  rsrc_t wrs[RT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+    const int t = min(t0 + r, row_tiles - 1);
+    wrs[r] = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(a.w) + (int64_t)t * a.GS * BB, (short)0, a.GS * BB, kRsrcWord3);
+  }
+
+  // Request j of a wave fills 4 x rows of a chunk (1 KiB, lane order): this lane's row and the
+  // 16-byte unit whose place in that row it fills.  Rows past M are out of the resource's
+  // range and read zeros; so do K-values past K (the weight stream is zero there).
+  unsigned xoff[4];
+  int xk[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int row = (wave * XD + j) * 4 + (lane >> 4);
+    const int u = (lane & 15) ^ (row & 15);
+    xoff[j] = (unsigned)row * (unsigned)a.K * 2u + (u >> 2) * 256 + (u & 3) * 16;
+    xk[j] = (u >> 2) * 128;
+  }
+  auto stage = [&](int sp, int c, uint8_t* buf) {
+    const int kleft = a.K - sp * 512;
+    const unsigned so = (unsigned)sp * 1024u + (unsigned)c * 64u;
+#pragma unroll
+    for (int j = 0; j < XD; ++j) {
+      const unsigned off = xk[j & 3] < kleft
+                               ? xoff[j & 3] + (unsigned)((j >> 2) * 16) * (unsigned)a.K * 2u + so
+                               : kXOutOfRange;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          xrs, (lds_byte*)(buf + (wave * XD + j) * 1024), 16, off, 0, 0, 0);
+    }
+  };
+
+  u32x4 nib[NB][RT];
+  u32x4 tb[RT][2], tbn[RT][2];
+  auto load_nib = [&](int sp, int c, u32x4 (&d)[RT]) {
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+      d[r] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                           wrs[r], lane * 16 + c * 1024, sp * BB, 0));
+  };
+  auto load_tab = [&](int sp, u32x4 (&d)[RT][2]) {
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      if constexpr (FMT == FB_FMT_GF4) {
+        d[r][0] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                wrs[r], lane * 16 + 4096, sp * BB, 0));
+        d[r][1] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                wrs[r], lane * 16 + 5120, sp * BB, 0));
+      } else {
+        d[r][0].x = __builtin_amdgcn_raw_buffer_load_b32(wrs[r], lane * 4 + 4096, sp * BB, 0);
+      }
+    }
+  };
+
+  f32x4 acc[RT][CT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int c = 0; c < CT; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // B operand of column tile ct, k-step s: x row lane % 16, unit 4 (lane / 16) + s
+  const unsigned rbase = (lane & 15) * kRowBytes + ((((lane >> 4) * 4) ^ (lane & 15)) << 4);
+
+  // Half h of the A operand of k-step s of chunk c (words 2h, 2h + 1 of 4), from nibbles nb
+  // and tables tt.
+  auto decode_half = [&](u32x4& A, const u32x4& nb, const u32x4 (&tt)[2], int c, int s, int h) {
+    if constexpr (FMT == FB_FMT_GF4) {
+      const unsigned sel = (h ? nb[s] >> 4 : nb[s]) & 0x0F0F0F0Fu;
+      const unsigned sel8 = sel ^ 0x08080808u;
+      const unsigned lo = perm(tt[0].y, tt[0].x, sel) ^ perm(tt[0].w, tt[0].z, sel8);
+      const unsigned hi = perm(tt[1].y, tt[1].x, sel) ^ perm(tt[1].w, tt[1].z, sel8);
+      A[2 * h] = perm(hi, lo, 0x05010400u);
+      A[2 * h + 1] = perm(hi, lo, 0x07030602u);
+    } else {
+      const float sc = __builtin_bit_cast(float, ((tt[0].x >> (8 * c)) & 0xFFu) << 23);
+      const u32x4 v = e2m1_decode8<XDT>(nb[s], sc);
+      A[2 * h] = v[2 * h];
+      A[2 * h + 1] = v[2 * h + 1];
+    }
+  };
+  u32x4 A[2][RT];  // this k-step's operands and the next one's
+  // One chunk: 4 k-steps of RT x CT MFMAs.  B operands are read two column tiles ahead.
+  auto compute = [&](const uint8_t* buf, const u32x4 (&nb)[RT], const u32x4 (&nbn)[RT], int c) {
+    u32x4 B[3];
+    auto readb = [&](int i) {
+      return *reinterpret_cast<const u32x4*>(buf + (rbase ^ ((i / CT) * 16)) +
+                                             (i % CT) * 16 * kRowBytes);
+    };
+    B[0] = readb(0);
+    B[1] = readb(1);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        const int i = s * CT + ct;
+        if (i + 2 < 4 * CT) B[(i + 2) % 3] = readb(i + 2);
+        // this step's share of the next k-step's 2 RT half decodes
+#pragma unroll
+        for (int q = ct * 2 * RT / CT; q < (ct + 1) * 2 * RT / CT; ++q) {
+          const int r = q >> 1, h = q & 1;
+          if (s < 3)
+            decode_half(A[(s + 1) & 1][r], nb[r], tb[r], c, s + 1, h);
+          else if (c < 3)
+            decode_half(A[0][r], nbn[r], tb[r], c + 1, 0, h);
+          else
+            decode_half(A[0][r], nbn[r], tbn[r], 0, 0, h);
+        }
+#pragma unroll
+        for (int r = 0; r < RT; ++r) acc[r][ct] = mfma<XDT>(A[s & 1][r], B[i % 3], acc[r][ct]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+
+  uint8_t* const bufs[4] = {xb0, xb1, NB == 4 ? xb2 : xb0, NB == 4 ? xb3 : xb1};
+  if (nsp > 0) {
+    load_tab(sp0, tb);
+#pragma unroll
+    for (int c = 0; c < D; ++c) {
+      load_nib(sp0, c, nib[c]);
+      stage(sp0, c, bufs[c]);
+    }
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      decode_half(A[0][r], nib[0][r], tb[r], 0, 0, 0);
+      decode_half(A[0][r], nib[0][r], tb[r], 0, 0, 1);
+    }
+    for (int sp = sp0; sp < sp1; ++sp) {
+      const int spn = min(sp + 1, sp1 - 1);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        // The x of chunk c was requested D chunks ago; each of the D - 1 chunks since then
+        // requested XD pieces of x and RT nibble chunks (and sometimes tables), so at most that
+        // many younger requests in flight means it has arrived.  Past the barrier every
+        // wave's part of it has, and every wave has read the chunk before.
+        wait_barrier<(D - 1) * (XD + RT)>();
+        const int cn = (c + D) & 3;
+        const int spx = c + D >= 4 ? spn : sp;
+        load_nib(spx, cn, nib[cn % NB]);
+        if (cn == 0) load_tab(spx, tbn);
+        stage(spx, cn, bufs[cn]);
+        compute(bufs[c], nib[c % NB], nib[(c + 1) % NB], c);
+      }
+#pragma unroll
+      for (int r = 0; r < RT; ++r) {
+        tb[r][0] = tbn[r][0];
+        tb[r][1] = tbn[r][1];
+      }
+    }
+  }
+
+  // lane: x row 16 ct + lane % 16, weight rows 4 (lane / 16) .. + 3 of each row tile
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) {
+    const int m = ct * 16 + (lane & 15);
+    if (m >= rows) continue;
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      const int n = (t0 + r) * 16 + (lane >> 4) * 4;
+      const f32x4 v = acc[r][ct];
+      const int64_t o = (int64_t)(m0 + m) * a.N + n;
+      if (a.part) {
+        float* dst = a.part + (int64_t)p * a.M * a.N + o;
+        if (a.vec && n + 4 <= a.N) {
+          *reinterpret_cast<f32x4*>(dst) = v;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < a.N) dst[e] = v[e];
+        }
+      } else if (a.vec && n + 4 <= a.N) {
+        if (a.ydt == FB_DT_F32) {
+          *reinterpret_cast<f32x4*>(static_cast<float*>(a.y) + o) = v;
+        } else {
+          unsigned h[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            h[e] = a.ydt == FB_DT_F16 ? __builtin_bit_cast(unsigned short, (_Float16)v[e])
+                                      : __builtin_bit_cast(unsigned short, (__bf16)v[e]);
+          *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.y) + o) =
+              make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < a.N) store_y(a.y, o + e, v[e], a.ydt);
+      }
+    }
+  }
+}
+
+// y = the P parts' sums added in part order (deterministic), four outputs per thread.
+__global__ __launch_bounds__(256) void gemm_sum(const float* __restrict__ part, int P, int64_t n,
+                                                void* __restrict__ y, int ydt, int vec) {
+  const int64_t i0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i0 >= n) return;
+  if (vec) {
+    f32x4 a = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(part + i0));
+#pragma unroll 4
+    for (int p = 1; p < P; ++p)
+      a += __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(part + (int64_t)p * n + i0));
+    if (ydt == FB_DT_F32) {
+      *reinterpret_cast<f32x4*>(static_cast<float*>(y) + i0) = a;
+    } else {
+      unsigned h[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        h[e] = ydt == FB_DT_F16 ? __builtin_bit_cast(unsigned short, (_Float16)a[e])
+                                : __builtin_bit_cast(unsigned short, (__bf16)a[e]);
+      *reinterpret_cast<uint2*>(static_cast<uint16_t*>(y) + i0) =
+          make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+    }
+  } else {
+    for (int64_t i = i0; i < min(n, i0 + 4); ++i) {
+      float a = part[i];
+      for (int p = 1; p < P; ++p) a += part[(int64_t)p * n + i];
+      store_y(y, i, a, ydt);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------
+// host side
+// ---------------------------------------------------------------------------------
+// Tile shapes the plan chooses from, with the time in us that a span (512 K-values) of one
+// tile takes on a CU when one workgroup runs there (one) and when two do (two, both done;
+// 0: LDS holds one workgroup).  Fitted to 2,300 timings of every shape and part count over
+// M = 17..1024 on 4096^2, 8192^2, 4096 -> 11008, 11008 -> 4096 and 8192 -> 28672; the plan it
+// picks is within 2% (geometric mean; 17% at worst) of the best one timed.  A table rather
+// than a formula because the costs follow no simple one: small tiles are bound by latency
+// and the x fill, large GF4 tiles by instruction issue, large E2M1 tiles by the MFMAs.
+struct GemmShape {
+  int rt, ct;
+  float one[2], two[2];  // [GF4, E2M1]
+};
+constexpr GemmShape kGemmShapes[] = {
+    {4, 8, {7.12f, 5.37f}, {0, 0}},         {4, 4, {5.10f, 2.76f}, {8.24f, 4.55f}},
+    {3, 6, {4.82f, 3.23f}, {0, 0}},         {2, 6, {3.47f, 2.33f}, {0, 0}},
+    {2, 4, {2.65f, 1.51f}, {4.48f, 2.84f}}, {2, 3, {2.34f, 1.26f}, {3.79f, 2.23f}},
+    {2, 2, {1.92f, 1.07f}, {3.21f, 1.73f}},
+};
+constexpr int kMaxParts = 8;
+constexpr int64_t kMaxPartBytes = 256ll << 20;
+
+struct GemmPlan {
+  int rt = 0, ct = 0, P = 1;
+};
+
+GemmPlan gemm_plan(const fb_shape_t* s, int cus) {
+  const int GS = (s->K / 128 + 3) / 4;
+  const int f = s->fmt == FB_FMT_GF4 ? 0 : 1;
+  const double mn = 1e-6 * s->B * (double)s->N;
+  // the same fit's cost of a part-sum launch, and of its traffic per million fp32 sums
+  const double sum0 = f ? 2.23 : 1.79, sum1 = f ? 1.70 : 1.83;
+  GemmPlan best;
+  double bt = 0;
+  for (const GemmShape& c : kGemmShapes) {
+    const int64_t T = (int64_t)((s->N + c.rt * 64 - 1) / (c.rt * 64)) *
+                      ((s->B + c.ct * 16 - 1) / (c.ct * 16));
+    const int occ = c.two[f] > 0 ? 2 : 1;
+    for (int P = 1; P <= kMaxParts && P <= GS; ++P) {
+      const int S = (GS + P - 1) / P;
+      if (S * (P - 1) >= GS) continue;  // an empty part
+      if (P > 1 && 4 * (int64_t)P * s->B * s->N > kMaxPartBytes) break;
+      const int64_t slots = (int64_t)cus * occ, full = T * P / slots, rem = T * P % slots;
+      double t = S * (full * (occ == 2 ? c.two[f] : c.one[f]) +
+                      (rem == 0 ? 0.0 : rem <= cus ? c.one[f] : c.two[f]));
+      if (P > 1) t += sum0 + sum1 * mn * P;
+      if (!best.rt || t < bt) {
+        bt = t;
+        best.rt = c.rt;
+        best.ct = c.ct;
+        best.P = P;
+      }
+    }
+  }
+  return best;
+}
+
+template <int FMT, int XDT, int RT, int CT>
+int launch_gemm(GemmArgs a, int P, hipStream_t hs) {
+  using T = GemmTile<RT, CT>;
+  a.tiles_n = (a.N + T::kRows - 1) / T::kRows;
+  a.tiles_m = (a.M + T::kCols - 1) / T::kCols;
+  a.spp = (a.GS + P - 1) / P;
+  const int64_t grid = (int64_t)a.tiles_n * a.tiles_m * P;
+  if (grid > INT32_MAX) return FB_ERR_SHAPE;
+  hipLaunchKernelGGL((gemm_kernel<FMT, XDT, RT, CT>), dim3((unsigned)grid),
+                     dim3(kGemmWaves * 64), 0, hs, a);
+  return hipGetLastError() == hipSuccess ? FB_OK : FB_ERR_HIP;
+}
+
+template <int FMT, int XDT>
+int launch_gemm_tile(const GemmArgs& a, const GemmPlan& pl, hipStream_t hs) {
+  switch (pl.rt * 100 + pl.ct) {
+    case 408: return launch_gemm<FMT, XDT, 4, 8>(a, pl.P, hs);
+    case 404: return launch_gemm<FMT, XDT, 4, 4>(a, pl.P, hs);
+    case 306: return launch_gemm<FMT, XDT, 3, 6>(a, pl.P, hs);
+    case 206: return launch_gemm<FMT, XDT, 2, 6>(a, pl.P, hs);
+    case 204: return launch_gemm<FMT, XDT, 2, 4>(a, pl.P, hs);
+    case 203: return launch_gemm<FMT, XDT, 2, 3>(a, pl.P, hs);
+    default: return launch_gemm<FMT, XDT, 2, 2>(a, pl.P, hs);
+  }
+}
+
+// x (rotated already where the layer is) times W^T with the parts' sums in ws (pl.P > 1).
+int gemm_run(const void* wdev, const void* x, void* y, const fb_shape_t* s, const GemmPlan& pl,
+             void* ws, hipStream_t hs) {
+  GemmArgs a{};
+  a.w = static_cast<const uint8_t*>(wdev);
+  a.x = x;
+  a.y = y;
+  a.part = pl.P > 1 ? static_cast<float*>(ws) : nullptr;
+  a.M = s->B;
+  a.N = s->N;
+  a.K = s->K;
+  a.GS = (s->K / 128 + 3) / 4;
+  a.ydt = s->y_dtype;
+  a.vec = (s->N & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
+  int st;
+  if (s->fmt == FB_FMT_GF4)
+    st = launch_gemm_tile<FB_FMT_GF4, FB_DT_F16>(a, pl, hs);
+  else if (s->x_dtype == FB_DT_BF16)
+    st = launch_gemm_tile<FB_FMT_E2M1, FB_DT_BF16>(a, pl, hs);
+  else
+    st = launch_gemm_tile<FB_FMT_E2M1, FB_DT_F16>(a, pl, hs);
+  if (st != FB_OK || pl.P == 1) return st;
+  const int64_t n = (int64_t)s->B * s->N;
+  if ((n + 1023) / 1024 > INT32_MAX) return FB_ERR_SHAPE;
+  hipLaunchKernelGGL(gemm_sum, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, hs, a.part,
+                     pl.P, n, y, s->y_dtype, a.vec);
+  return hipGetLastError() == hipSuccess ? FB_OK : FB_ERR_HIP;
+}
+
+size_t rot_bytes(const fb_shape_t* s) {
+  return s->fwht_block ? ((size_t)s->B * s->K * 2 + 255) & ~size_t(255) : 0;
+}
+
+// A tile's x rows and a weight tile's stream are addressed with 32-bit byte offsets.
+int gemm_check(const fb_shape_t* s) {
+  const int st = fb_validate(s);
+  if (st != FB_OK) return st;
+  if (s->K > (1 << 22) || s->B > (1 << 24)) return FB_ERR_SHAPE;
+  if (s->fwht_block && s->x_dtype != FB_DT_F16) return FB_ERR_DTYPE;
+  return FB_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+size_t fb_gemm_workspace_bytes(const fb_shape_t* s) {
+  if (!s || gemm_check(s) != FB_OK) return 0;
+  const GemmPlan pl = gemm_plan(s, fb_gpu::cu_count());
+  return rot_bytes(s) + (pl.P > 1 ? ((size_t)pl.P * s->B * s->N * 4 + 255) & ~size_t(255) : 0);
+}
+
+int fb_gemm(const void* wdev, const void* x, void* y, const fb_shape_t* s, void* ws,
+            size_t ws_bytes, void* stream) {
+  if (!s || !wdev || !x || !y) return FB_ERR_NULL;
+  const int st = gemm_check(s);
+  if (st != FB_OK) return st;
+  if ((reinterpret_cast<uintptr_t>(wdev) & 15u) || (reinterpret_cast<uintptr_t>(x) & 15u) ||
+      (reinterpret_cast<uintptr_t>(y) & 3u))
+    return FB_ERR_ALIGN;
+  hipStream_t hs = static_cast<hipStream_t>(stream);
+  GemmPlan pl = gemm_plan(s, fb_gpu::cu_count());
+  const size_t rot = rot_bytes(s);
+  const size_t need = rot + (pl.P > 1 ? (size_t)pl.P * s->B * s->N * 4 : 0);
+  if (need && !ws) return FB_ERR_NULL;
+  if (need && (reinterpret_cast<uintptr_t>(ws) & 255u)) return FB_ERR_ALIGN;
+  if (need > ws_bytes) return FB_ERR_WORKSPACE;
+  if (rot) {
+    const int rc = fb_gpu::rotate_rows(x, ws, s->B, s->K, s->fwht_block, hs);
+    if (rc != FB_OK) return rc;
+    x = ws;
+  }
+  return gemm_run(wdev, x, y, s, pl, static_cast<uint8_t*>(ws) + rot, hs);
+}
+
+}  // extern "C"

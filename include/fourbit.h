@@ -169,6 +169,22 @@ int fb_dequant_host(const uint8_t* codes, const void* meta, float* w_out, const 
 int fb_gemv(const void* wdev, const void* x, void* y, const fb_shape_t* s, void* ws,
             size_t ws_bytes, void* stream);
 
+/* The same product for any number of rows B of x (prompts, training batches), decoding the
+ * weight once per 32 to 128 rows: y = x' . W^T with x' = FWHT_b(x) when fwht_block.  Operands,
+ * layout and rotation as fb_gemv's; replaces the same reference interface
+ * (QuantLinear.forward, layers.py:33-38) where its input has many rows.  fb_gemv is the faster
+ * one for B <= 16.  K <= 2^22, B <= 2^24 (FB_ERR_SHAPE).
+ * ws: device workspace, 256-byte aligned, of at least fb_gemm_workspace_bytes(s) bytes (the
+ * rotated x, and the fp32 sums of K-parts for shapes that leave CUs idle otherwise; required
+ * where that is not 0: FB_ERR_NULL / FB_ERR_ALIGN / FB_ERR_WORKSPACE).  Its contents need no
+ * initialisation; calls that share it must not overlap. */
+int fb_gemm(const void* wdev, const void* x, void* y, const fb_shape_t* s, void* ws,
+            size_t ws_bytes, void* stream);
+
+/* Workspace bytes of fb_gemm for this shape on the current device (0: none, or a shape it does
+ * not take). */
+size_t fb_gemm_workspace_bytes(const fb_shape_t* s);
+
 /* fb_gemv that allocates nothing and takes no workspace.  No counterpart in the reference:
  * it is for callers that cannot allocate device memory around a call (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  The once-per-call
