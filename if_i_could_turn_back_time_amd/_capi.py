@@ -41,7 +41,7 @@ EXPORTED = (
     "fb_gemv_mx_presplit", "fb_mx_presplit_workspace_bytes",
     "fb_jenks2_ssd_host", "fb_jenks2_ssd_workspace", "fb_jenks2_ssd_gpu",
     "fb_jenks2_ssd_filters_host", "fb_jenks2_ssd_filters_gpu",
-    "fb_gemm", "fb_gemm_workspace_bytes",
+    "fb_gemm", "fb_gemm_workspace_bytes", "fb_grad_x", "fb_grad_x_workspace_bytes",
 )
 
 
@@ -82,6 +82,8 @@ def lib() -> ctypes.CDLL:
         "fb_gemv": (ctypes.c_int, [vp, vp, vp, sp, vp, sz, vp]),
         "fb_gemm": (ctypes.c_int, [vp, vp, vp, sp, vp, sz, vp]),
         "fb_gemm_workspace_bytes": (sz, [sp]),
+        "fb_grad_x": (ctypes.c_int, [vp, vp, vp, sp, i32, i32, vp, sz, vp]),
+        "fb_grad_x_workspace_bytes": (sz, [sp, i32]),
         "fb_dequant": (ctypes.c_int, [vp, vp, i32, sp, vp]),
         "fb_quantize_gf4_gpu": (ctypes.c_int, [vp, vp, i32, i32, vp, vp, vp]),
         "fb_quantize_e2m1_gpu": (ctypes.c_int, [vp, i32, i32, vp, vp, vp]),
@@ -307,6 +309,32 @@ def gemm(wdev: torch.Tensor, x: torch.Tensor, y: torch.Tensor, shape: FbShape) -
         check(lib().fb_gemm(_ptr(wdev), _ptr(x), _ptr(y), ctypes.byref(shape),
                             _ptr(ws) if need else None, need, _stream(x.device)))
     return y
+
+
+def grad_x(wdev: torch.Tensor, gy: torch.Tensor, gx: torch.Tensor, shape: FbShape,
+           f16_exact: bool) -> torch.Tensor:
+    """gx[B,K] = (gy[B,N] . W) H on the GPU (fb_grad_x; asynchronous on the current stream):
+    the gradient of gemm's x.  ``shape`` has gy's dtype as its y_dtype; gx may be float16,
+    bfloat16 or float32."""
+    if not (wdev.is_cuda and gy.is_cuda and gx.is_cuda):
+        raise RuntimeError("fb_grad_x needs device tensors (ROCm GPU)")
+    if not (wdev.device == gy.device == gx.device):
+        raise ValueError("fb_grad_x operands are on different devices")
+    if not (gy.is_contiguous() and gx.is_contiguous()):
+        raise ValueError("gy and gx must be contiguous")
+    if DTYPE_CODE.get(gy.dtype) != shape.y_dtype or gx.dtype not in DTYPE_CODE:
+        raise ValueError("gy / gx dtypes do not match the shape")
+    if tuple(gy.shape) != (shape.B, shape.N) or tuple(gx.shape) != (shape.B, shape.K):
+        raise ValueError("gy / gx do not match the shape")
+    if wdev.numel() < device_bytes(shape):
+        raise ValueError("weight stream is smaller than fb_device_bytes(shape)")
+    with torch.cuda.device(gy.device):
+        need = lib().fb_grad_x_workspace_bytes(ctypes.byref(shape), int(f16_exact))
+        ws = torch.empty(max(need, 1), dtype=torch.uint8, device=gy.device)
+        check(lib().fb_grad_x(_ptr(wdev), _ptr(gy), _ptr(gx), ctypes.byref(shape),
+                              DTYPE_CODE[gx.dtype], int(f16_exact), _ptr(ws), need,
+                              _stream(gy.device)))
+    return gx
 
 
 def _mx_refuse(shape: FbShape) -> None:

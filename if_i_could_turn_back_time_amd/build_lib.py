@@ -67,6 +67,7 @@ def build(verbose: bool = False) -> Path:
     gemv_o = BUILD / "fourbit_gemv.o"
     ilp_o = BUILD / "fourbit_gemv_ilp.o"
     gemm_o = BUILD / "fourbit_gemm.o"
+    grad_o = BUILD / "fourbit_grad.o"
     pack_o = BUILD / "fourbit_pack.o"
     jenks2_o = BUILD / "fourbit_jenks2.o"
     trace_o = BUILD / "fourbit_gemv_trace.o"
@@ -79,6 +80,7 @@ def build(verbose: bool = False) -> Path:
         [_hipcc(), *HIP_FLAGS, "-mllvm", "-amdgpu-sched-strategy=max-ilp", *inc, "-c",
          str(CSRC / "fourbit_gemv_ilp.hip"), "-o", str(ilp_o)],
         [_hipcc(), *HIP_FLAGS, *inc, "-c", str(CSRC / "fourbit_gemm.hip"), "-o", str(gemm_o)],
+        [_hipcc(), *HIP_FLAGS, *inc, "-c", str(CSRC / "fourbit_grad.hip"), "-o", str(grad_o)],
         # the GPU packer must round every fp64 operation as the host packer does
         [_hipcc(), *HIP_FLAGS, "-ffp-contract=off", *inc, "-c", str(CSRC / "fourbit_pack.hip"),
          "-o", str(pack_o)],
@@ -100,7 +102,7 @@ def build(verbose: bool = False) -> Path:
     for lib, kern_os in ((LIB, (gemv_o, ilp_o)), (TRACE_LIB, (trace_o, trace_ilp_o))):
         tmp = lib.with_suffix(".so.tmp")
         link = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", str(host_o),
-                *map(str, kern_os), str(gemm_o), str(pack_o), str(jenks2_o), "-o", str(tmp), "-lpthread"]
+                *map(str, kern_os), str(gemm_o), str(grad_o), str(pack_o), str(jenks2_o), "-o", str(tmp), "-lpthread"]
         if verbose:
             print(" ".join(link), flush=True)
         _run(link)

@@ -35,6 +35,30 @@ __device__ __forceinline__ void store_y(void* y, int64_t idx, float v, int ydt) 
   }
 }
 
+// Four outputs at idx, which 16-byte alignment of y and idx % 4 == 0 make one store.
+__device__ __forceinline__ void store4(void* y, int64_t idx, const f32x4& v, int ydt) {
+  if (ydt == FB_DT_F32) {
+    *reinterpret_cast<f32x4*>(static_cast<float*>(y) + idx) = v;
+  } else {
+    unsigned h[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      h[e] = ydt == FB_DT_F16 ? __builtin_bit_cast(unsigned short, (_Float16)v[e])
+                              : __builtin_bit_cast(unsigned short, (__bf16)v[e]);
+    *reinterpret_cast<uint2*>(static_cast<uint16_t*>(y) + idx) =
+        make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+  }
+}
+
+typedef __attribute__((address_space(3))) uint8_t lds_byte;
+
+// Workgroup barrier once this wave has at most N vector memory operations in flight (of which
+// loads into LDS are some) and has received every LDS read.
+template <int N>
+__device__ __forceinline__ void wait_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
 // GF4 decode of one 32-bit word (8 codes, layout order) into 4 fp16 pairs in element
 // order (e0,e1) (e2,e3) (e4,e5) (e6,e7).  tl/th: lo/hi byte-plane tables
 // {A'[0..3], A'[4..7], B'[0..3], B'[4..7]}.

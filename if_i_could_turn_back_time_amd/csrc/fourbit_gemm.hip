@@ -33,26 +33,19 @@
 #include "fourbit_decode.h"
 #include "fourbit_layout.h"
 
-// Host helpers of fourbit_gemv.hip.  Not part of the library's ABI.
+// Host helpers shared by the GPU units.  Not part of the library's ABI.
 namespace fb_gpu {
 __attribute__((visibility("hidden"))) int cu_count();
 __attribute__((visibility("hidden"))) int rotate_rows(const void* x, void* xo, int rows, int K,
                                                       int block, hipStream_t hs);
+__attribute__((visibility("hidden"))) int sum_parts(const float* part, int P, int64_t n, void* y,
+                                                    int ydt, int vec, hipStream_t hs);
 }  // namespace fb_gpu
 
 namespace {
 
 constexpr int kGemmWaves = 4;
 constexpr int kRowBytes = 256;  // one x row of a chunk: 128 K-values, 32 of each item of a span
-
-typedef __attribute__((address_space(3))) uint8_t lds_byte;
-
-// workgroup barrier once this wave has at most N vector memory operations in flight and has
-// received every LDS read
-template <int N>
-__device__ __forceinline__ void wait_barrier() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
-}
 
 struct GemmArgs {
   const uint8_t* w;
@@ -288,17 +281,7 @@ __global__ __launch_bounds__(kGemmWaves * 64, (GemmTile<RT, CT>::kOcc)) void gem
             if (n + e < a.N) dst[e] = v[e];
         }
       } else if (a.vec && n + 4 <= a.N) {
-        if (a.ydt == FB_DT_F32) {
-          *reinterpret_cast<f32x4*>(static_cast<float*>(a.y) + o) = v;
-        } else {
-          unsigned h[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            h[e] = a.ydt == FB_DT_F16 ? __builtin_bit_cast(unsigned short, (_Float16)v[e])
-                                      : __builtin_bit_cast(unsigned short, (__bf16)v[e]);
-          *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.y) + o) =
-              make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-        }
+        store4(a.y, o, v, a.ydt);
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
@@ -318,17 +301,7 @@ __global__ __launch_bounds__(256) void gemm_sum(const float* __restrict__ part, 
 #pragma unroll 4
     for (int p = 1; p < P; ++p)
       a += __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(part + (int64_t)p * n + i0));
-    if (ydt == FB_DT_F32) {
-      *reinterpret_cast<f32x4*>(static_cast<float*>(y) + i0) = a;
-    } else {
-      unsigned h[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        h[e] = ydt == FB_DT_F16 ? __builtin_bit_cast(unsigned short, (_Float16)a[e])
-                                : __builtin_bit_cast(unsigned short, (__bf16)a[e]);
-      *reinterpret_cast<uint2*>(static_cast<uint16_t*>(y) + i0) =
-          make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-    }
+    store4(y, i0, a, ydt);
   } else {
     for (int64_t i = i0; i < min(n, i0 + 4); ++i) {
       float a = part[i];
@@ -444,11 +417,7 @@ int gemm_run(const void* wdev, const void* x, void* y, const fb_shape_t* s, cons
   else
     st = launch_gemm_tile<FB_FMT_E2M1, FB_DT_F16>(a, pl, hs);
   if (st != FB_OK || pl.P == 1) return st;
-  const int64_t n = (int64_t)s->B * s->N;
-  if ((n + 1023) / 1024 > INT32_MAX) return FB_ERR_SHAPE;
-  hipLaunchKernelGGL(gemm_sum, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, hs, a.part,
-                     pl.P, n, y, s->y_dtype, a.vec);
-  return hipGetLastError() == hipSuccess ? FB_OK : FB_ERR_HIP;
+  return fb_gpu::sum_parts(a.part, pl.P, (int64_t)s->B * s->N, y, s->y_dtype, a.vec, hs);
 }
 
 size_t rot_bytes(const fb_shape_t* s) {
@@ -465,6 +434,15 @@ int gemm_check(const fb_shape_t* s) {
 }
 
 }  // namespace
+
+// y[i] = part 0's + part 1's + ... sum i, for n sums (vec: n % 4 == 0 and y 16-byte aligned)
+int fb_gpu::sum_parts(const float* part, int P, int64_t n, void* y, int ydt, int vec,
+                      hipStream_t hs) {
+  if ((n + 1023) / 1024 > INT32_MAX) return FB_ERR_SHAPE;
+  hipLaunchKernelGGL(gemm_sum, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, hs, part, P, n,
+                     y, ydt, vec);
+  return hipGetLastError() == hipSuccess ? FB_OK : FB_ERR_HIP;
+}
 
 extern "C" {
 

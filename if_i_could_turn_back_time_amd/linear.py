@@ -122,7 +122,9 @@ def _gemv_chunks(wdev, N, kp, fmt, fwht_block, xk, y, fp4_mfma=False, ws_cache=N
             C.gemv(wdev, xk[b0:b1], y[b0:b1], shape, ws)
 
 
-# Most bytes of fp32 weight the backward pass decodes at once (a chunk of 16-row tiles).
+# fb_grad_x addresses a row of grad_y with 32-bit offsets.
+MAX_GRAD_N = 1 << 22
+# Most bytes of fp32 weight the torch form of the backward pass decodes at once (a chunk of 16-row tiles).
 BACKWARD_CHUNK_BYTES = 64 * 2**20
 
 
@@ -183,9 +185,10 @@ def _kernel_input(x2: torch.Tensor, K: int, fmt: str, fwht_block: int, range_che
 class _PackedLinearFn(torch.autograd.Function):
     """``x -> x W^T`` through the fused kernel, differentiable in x (as ``F.linear`` with
     the reference's frozen committed weight is, ``layers.py:34-35``).  Backward:
-    ``grad_x = grad_y W``, with W decoded on the device (fb_dequant, fp32) in chunks of row
-    tiles (``_grad_x``) and, for a rotated weight W' = W H, rotated back:
-    ``grad_x = (grad_y W') H``."""
+    ``grad_x = grad_y W`` and, for a rotated weight W' = W H, rotated back:
+    ``grad_x = (grad_y W') H``, in one native call (fb_grad_x).  Where the gradient itself is
+    to be differentiated, and for more rows of W than fb_grad_x takes, the same from torch
+    operations on W decoded in chunks of row tiles (``_grad_x``)."""
 
     @staticmethod
     def forward(ctx, x2, wdev, N, K, fmt, fwht_block, range_check, f16_exact, fp4_mfma=False,
@@ -195,13 +198,24 @@ class _PackedLinearFn(torch.autograd.Function):
         y = torch.empty(x2.shape[0], N, dtype=ydt, device=x2.device)
         _gemv_chunks(wdev, N, packed_k(K), fmt, fwht_block, xk, y, fp4_mfma, ws_cache)
         ctx.save_for_backward(wdev)
-        ctx.cfg = (N, K, fmt, fwht_block, x2.dtype)
+        ctx.cfg = (N, K, fmt, fwht_block, x2.dtype, f16_exact)
         return y
 
     @staticmethod
     def backward(ctx, gy):
         (wdev,) = ctx.saved_tensors
-        N, K, fmt, fwht_block, xdt = ctx.cfg
+        N, K, fmt, fwht_block, xdt, f16_exact = ctx.cfg
+        if not torch.is_grad_enabled() and N <= MAX_GRAD_N and gy.dtype in C.DTYPE_CODE:
+            kp = packed_k(K)
+            gx = torch.empty(gy.shape[0], kp, device=gy.device,
+                             dtype=xdt if xdt in C.DTYPE_CODE else torch.float32)
+            if gx.numel():
+                C.grad_x(wdev, gy.contiguous(), gx,
+                         C.make_shape(N, kp, gy.shape[0], C.FMT_BY_NAME[fmt], fwht_block,
+                                      C.DT_F16, C.DTYPE_CODE[gy.dtype]), f16_exact)
+            if kp != K:
+                gx = gx[:, :K].contiguous()
+            return gx.to(xdt), None, None, None, None, None, None, None, None, None
         gx = _grad_x(wdev, N, packed_k(K), fmt, fwht_block, gy)
         if fwht_block:
             gx = _fwht_last_dim(gx, fwht_block)

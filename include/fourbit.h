@@ -249,6 +249,25 @@ int fb_gemv_mx_presplit(const void* wdev, const void* xs, void* y, const fb_shap
 /* Workspace bytes of fb_gemv_mx_presplit (0: none used, or a shape it does not take). */
 size_t fb_mx_presplit_workspace_bytes(const fb_shape_t* s);
 
+/* The activation gradient: gx[B,K] = (gy[B,N] . W[N,K]) H, W the exact decode (fb_dequant's) and
+ * H the layer's blockwise rotation (none for fwht_block 0).  Replaces the backward of
+ * F.linear in the reference's forward (layers.py:33-38), where W is frozen.  s as fb_gemm's,
+ * with y_dtype gy's dtype (F16, BF16 or F32); gx_dtype is gx's.  The products are exact and
+ * summed in fp32, whatever gy's dtype: gy and W are multiplied as exact sums of 16-bit terms.
+ * f16_exact (E2M1 only): nonzero when every weight is exact in fp16 (all E8M0 bytes in
+ * 104..140), which lets an fp16 gy run as one term; GF4 weights are fp16 values.
+ * ws: device workspace, 256-byte aligned, of at least fb_grad_x_workspace_bytes(s, f16_exact)
+ * bytes (the transposed 16-bit weight, at most 256 MiB of it at once unless 512 of its K-columns
+ * take more, gy's terms, the sums of contraction parts, and for a rotated layer the fp32
+ * gradient).  Its contents need no initialisation; calls that share it must not overlap.
+ * N <= 2^22, B <= 2^24 (FB_ERR_SHAPE). */
+int fb_grad_x(const void* wdev, const void* gy, void* gx, const fb_shape_t* s, int32_t gx_dtype,
+              int32_t f16_exact, void* ws, size_t ws_bytes, void* stream);
+
+/* Workspace bytes of fb_grad_x for this shape on the current device (0: a shape it does not
+ * take). */
+size_t fb_grad_x_workspace_bytes(const fb_shape_t* s, int32_t f16_exact);
+
 /* GF4 packer on the GPU: the same arithmetic as fb_quantize_gf4 (keep == NULL) and
  * fb_quantize_gf4_masked, one wavefront per (row, 128-group), fp64; the outputs are
  * bit-identical to the host packers.  w fp32 [N,K], keep uint8 [N,K] or NULL, codes uint8

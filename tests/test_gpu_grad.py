@@ -1,0 +1,125 @@
+"""fb_grad_x (the activation gradient) against grad_y times the exact decode in fp64: edges of
+its tiles and chunks (rows of gy, of W and of K around them), every way it holds gy and W in 16
+bits, K ranges and contraction parts, the rotation, and infinities."""
+import pytest
+import torch
+
+from if_i_could_turn_back_time_amd import PackedWeight, QuantLinear, _capi as C
+from if_i_could_turn_back_time_amd import linear as LN
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+ULP = {torch.float32: 2.0 ** -24, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+
+
+def _weight(fmt, N, K, g, block=0):
+    return PackedWeight.quantize(torch.randn(N, K, generator=g) * 0.02, fmt, fwht_block=block,
+                                 device=DEV)
+
+
+def _run(pw, gy, gx_dtype, f16_exact=True):
+    M, N = gy.shape
+    shape = C.make_shape(N, pw.K, M, pw.fmt, pw.fwht_block, C.DT_F16, C.DTYPE_CODE[gy.dtype])
+    gx = torch.full((M, pw.K), float("nan"), dtype=gx_dtype, device=DEV)
+    return C.grad_x(pw.wdev, gy, gx, shape, f16_exact)
+
+
+@pytest.mark.parametrize("fmt,gdt,exact16", [
+    ("gf4", torch.float16, True), ("gf4", torch.bfloat16, True), ("gf4", torch.float32, True),
+    ("e2m1", torch.bfloat16, True), ("e2m1", torch.float16, True),
+    ("e2m1", torch.float16, False), ("e2m1", torch.float32, True)])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 128), (17, 16, 512), (31, 127, 640), (32, 128, 1152),
+                                   (65, 264, 384), (129, 1000, 2176), (300, 2051, 4224),
+                                   (513, 515, 896), (64, 8200, 128)])
+def test_grad_vs_exact_product(fmt, gdt, exact16, M, N, K):
+    print("grad", fmt, gdt, exact16, M, N, K, flush=True)
+    g = torch.Generator().manual_seed(M + N + K)
+    pw = _weight(fmt, N, K, g)
+    # magnitudes from 1e-7 (fp16: subnormal) to 1
+    gy = torch.randn(M, N, generator=g) * 10.0 ** torch.randint(-7, 1, (M, N), generator=g)
+    buf = torch.full((M * N + 4096,), float("nan"), dtype=gdt, device=DEV)
+    gd = buf[2048:2048 + M * N].view(M, N)
+    gd.copy_(gy)
+    w = pw.dequant_host().double().to(DEV)
+    ref = gd.double() @ w
+    # every product is exact; at most 6 N of them are summed in fp32
+    bound = 6 * N * 2.0 ** -24 * (gd.double().abs() @ w.abs()) + 1e-40
+    for xdt in (torch.float32, gdt):
+        gx = _run(pw, gd, xdt, exact16)
+        err = (gx.double() - ref).abs()
+        assert bool((err <= bound + ULP[xdt] * (ref.abs() + bound) + 2.0 ** -25 *
+                     (xdt == torch.float16)).all()), (xdt, float((err - bound).max()))
+        assert torch.equal(gx, _run(pw, gd, xdt, exact16))
+
+
+@pytest.mark.parametrize("M,N,K,block", [(5, 40, 256, 256), (33, 130, 4096, 4096),
+                                         (20, 64, 11008, 256), (18, 48, 6144, 2048),
+                                         (17, 32, 384, 128), (17, 32, 256, 2)])
+def test_grad_rotated(M, N, K, block):
+    g = torch.Generator().manual_seed(block)
+    pw = _weight("gf4", N, K, g, block)
+    for gdt in (torch.float16, torch.float32):
+        gy = torch.randn(M, N, generator=g).to(gdt).to(DEV)
+        ref = LN._fwht_last_dim(gy.double().float() @ pw.dequant_host().to(DEV), block).double()
+        gx = _run(pw, gy, torch.float32)
+        # fp32 sums of N products, then log2(block) additions, on values whose block has this norm
+        norm = (gy.double().abs() @ pw.dequant_host().double().abs().to(DEV)).norm(dim=1).max()
+        assert float((gx.double() - ref).abs().max()) <= (2 * N + 24) * 2.0 ** -24 * float(norm)
+
+
+def test_grad_in_k_ranges(monkeypatch):
+    """A weight larger than the operand buffer runs a range of K at a time (here one span of
+    4,200,000 / 8 rows: a span's operands alone pass the limit)."""
+    N, K = 40000, 1536
+    g = torch.Generator().manual_seed(5)
+    codes = torch.randint(0, 256, (N, K // 2), generator=g, dtype=torch.uint8)
+    meta = torch.randint(118, 124, (N, K // 32), generator=g, dtype=torch.uint8)
+    pw = PackedWeight("e2m1", N, K, codes, meta, 0, DEV)
+    gy = torch.randn(19, N, generator=g).bfloat16().to(DEV)
+    shape = C.make_shape(N, K, 19, C.FMT_E2M1, 0, C.DT_BF16, C.DT_BF16)
+    import ctypes
+    assert C.lib().fb_grad_x_workspace_bytes(ctypes.byref(shape), 1) < 2 * N * K * 2
+    w = pw.dequant_device().double()
+    ref = gy.double() @ w
+    gx = _run(pw, gy, torch.float32)
+    assert bool(((gx.double() - ref).abs() <= N * 2.0 ** -24 * (gy.double().abs() @ w.abs())).all())
+
+
+@pytest.mark.parametrize("fmt", ["gf4", "e2m1"])
+@pytest.mark.parametrize("gdt", [torch.float16, torch.bfloat16, torch.float32])
+def test_grad_infinities_as_in_fp32(fmt, gdt):
+    """Non-finite gradients give what an fp32 product gives: +-inf by the weight's sign, NaN
+    where the weight is 0, and leave the other rows alone."""
+    g = torch.Generator().manual_seed(9)
+    pw = _weight(fmt, 48, 256, g)
+    gy = torch.randn(20, 48, generator=g)
+    gy[2, 7], gy[5, 0], gy[9, 47] = float("inf"), float("-inf"), float("nan")
+    if gdt == torch.float32:
+        gy[11, 3] = 3.4e38
+    gy = gy.to(gdt).to(DEV)
+    ref = gy.float() @ pw.dequant_host().to(DEV)
+    gx = _run(pw, gy, torch.float32)
+    assert torch.equal(torch.isnan(gx), torch.isnan(ref))
+    assert torch.equal(gx[[2, 5]], ref[[2, 5]]) or torch.equal(
+        torch.nan_to_num(gx[[2, 5]]), torch.nan_to_num(ref[[2, 5]]))
+    fin = torch.isfinite(ref)
+    assert torch.equal(torch.isfinite(gx), fin)
+    assert torch.allclose(gx[fin], ref[fin], rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("kw", [dict(fmt="gf4"), dict(fmt="gf4", hadamard=256),
+                                dict(fmt="e2m1"), dict(fmt="e2m1", fp4_mfma=True)])
+def test_layer_gradient_and_its_gradient(kw):
+    """The layer's backward (native) equals its differentiable form (torch operations), for an
+    expanded grad_y too, and can itself be differentiated."""
+    torch.manual_seed(4)
+    q = QuantLinear(torch.nn.Linear(768 if "hadamard" in kw else 700, 130), **kw).to(DEV)
+    x = torch.randn(37, q.in_features, device=DEV, requires_grad=True)
+    for gy in (torch.randn(37, 130, device=DEV), torch.ones(1, 1, device=DEV).expand(37, 130)):
+        y = q(x)
+        (a,) = torch.autograd.grad(y, x, gy, retain_graph=True)
+        g2 = gy.clone().requires_grad_(True)
+        (b,) = torch.autograd.grad(y, x, g2, create_graph=True)
+        assert a.is_contiguous() and torch.allclose(a, b, rtol=1e-5, atol=1e-5)
+        (c,) = torch.autograd.grad(b.sum(), g2)
+        assert c.shape == gy.shape and bool(torch.isfinite(c).all())
