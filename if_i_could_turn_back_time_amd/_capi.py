@@ -42,6 +42,7 @@ EXPORTED = (
     "fb_jenks2_ssd_host", "fb_jenks2_ssd_workspace", "fb_jenks2_ssd_gpu",
     "fb_jenks2_ssd_filters_host", "fb_jenks2_ssd_filters_gpu",
     "fb_gemm", "fb_gemm_workspace_bytes", "fb_grad_x", "fb_grad_x_workspace_bytes",
+    "fb_to_device_gpu",
 )
 
 
@@ -77,6 +78,7 @@ def lib() -> ctypes.CDLL:
         "fb_quantize_e2m1": (ctypes.c_int, [vp, i32, i32, vp, vp, i32]),
         "fb_fwht_rows_f32": (ctypes.c_int, [vp, i32, i32, i32, i32]),
         "fb_to_device": (ctypes.c_int, [vp, vp, vp, sp]),
+        "fb_to_device_gpu": (ctypes.c_int, [vp, vp, vp, sp, vp]),
         "fb_from_device": (ctypes.c_int, [vp, vp, vp, sp]),
         "fb_dequant_host": (ctypes.c_int, [vp, vp, vp, sp]),
         "fb_gemv": (ctypes.c_int, [vp, vp, vp, sp, vp, sz, vp]),
@@ -212,6 +214,23 @@ def to_device_layout(codes: torch.Tensor, meta: torch.Tensor, shape: FbShape) ->
     meta = meta.detach().contiguous()
     out = torch.empty(device_bytes(shape), dtype=torch.uint8)
     check(lib().fb_to_device(_ptr(codes), _ptr(meta), _ptr(out), ctypes.byref(shape)))
+    return out
+
+
+def to_device_layout_gpu(codes: torch.Tensor, meta: torch.Tensor, shape: FbShape) -> torch.Tensor:
+    """to_device_layout of device tensors, on the GPU (fb_to_device_gpu): the same bytes."""
+    if not (codes.is_cuda and codes.device == meta.device):
+        raise RuntimeError("fb_to_device_gpu needs tensors on one ROCm GPU")
+    if codes.dtype != torch.uint8 or not (codes.is_contiguous() and meta.is_contiguous()):
+        raise ValueError("codes must be uint8, codes and meta contiguous")
+    G = shape.K // 128
+    want = shape.N * G * (32 if shape.fmt == FMT_GF4 else 4)
+    if codes.numel() != shape.N * shape.K // 2 or meta.numel() * meta.element_size() != want:
+        raise ValueError("codes / meta do not match the shape")
+    out = torch.empty(device_bytes(shape), dtype=torch.uint8, device=codes.device)
+    with torch.cuda.device(codes.device):
+        check(lib().fb_to_device_gpu(_ptr(codes), _ptr(meta), _ptr(out), ctypes.byref(shape),
+                                     _stream(codes.device)))
     return out
 
 

@@ -34,6 +34,13 @@
 #include <stdint.h>
 #include <string.h>
 
+// the table solve also runs on the GPU (the device form of fb_to_device)
+#ifdef __HIPCC__
+#define FB_HOST_DEVICE __host__ __device__
+#else
+#define FB_HOST_DEVICE
+#endif
+
 namespace fb {
 
 constexpr int kItemCodes = 128;   // K-elements per item
@@ -51,10 +58,10 @@ inline uint8_t perm8(const uint8_t* t, uint8_t sel) {
   return t[sel];
 }
 
-inline uint8_t rep(uint8_t b) { return (b & 0x80) ? 0xFF : 0x00; }
+FB_HOST_DEVICE inline uint8_t rep(uint8_t b) { return (b & 0x80) ? 0xFF : 0x00; }
 
 // Solves A', B' for one 16-entry byte plane T (see the header comment).
-inline void gf4_xor_tables(const uint8_t T[16], uint8_t A[8], uint8_t B[8]) {
+FB_HOST_DEVICE inline void gf4_xor_tables(const uint8_t T[16], uint8_t A[8], uint8_t B[8]) {
   A[4] = T[4];
   A[5] = T[5] ^ 0xFF;
   A[6] = T[6] ^ 0xFF;

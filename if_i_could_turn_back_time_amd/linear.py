@@ -279,7 +279,9 @@ class PackedWeight:
     """Packed 4-bit weight: canonical host buffers + the device stream, and a GEMV."""
 
     def __init__(self, fmt: str, N: int, K: int, codes: torch.Tensor, meta: torch.Tensor,
-                 fwht_block: int = 0, device=None):
+                 fwht_block: int = 0, device=None, *, wdev: torch.Tensor | None = None):
+        """``wdev``: the device stream of ``codes`` and ``meta`` where it has been built
+        already (by fb_to_device_gpu)."""
         self.fmt = C.FMT_BY_NAME[fmt]
         self.fmt_name = fmt
         self.N, self.K, self.fwht_block = N, K, fwht_block
@@ -287,7 +289,7 @@ class PackedWeight:
         self.f16_exact = self.fmt != C.FMT_E2M1 or e2m1_scales_fit_f16(meta)
         self._ws = {}
         shape = C.make_shape(N, K, 1, self.fmt, fwht_block)
-        self.wdev = C.to_device_layout(codes, meta, shape)
+        self.wdev = C.to_device_layout(codes, meta, shape) if wdev is None else wdev
         if device is not None:
             self.wdev = self.wdev.to(device)
 
@@ -298,28 +300,34 @@ class PackedWeight:
         """Packs fp32 ``w [N,K]``.  ``keep`` (GF4 only, no rotation): entries where it is
         0 decode to exactly 0.  ``packer='gpu'`` packs on the GPU (``device``, or cuda:0)
         with the same bytes as the host packer."""
-        w = w.detach().float().cpu().contiguous()
+        if packer not in ("host", "gpu"):
+            raise ValueError(f"packer must be 'host' or 'gpu', got {packer!r}")
+        # the GPU packers take w where it is; the rotation and the host packers run on the CPU
+        w = w.detach().float()
+        if packer == "host" or fwht_block:
+            w = w.cpu()
+        w = w.contiguous()
         N, K = w.shape
         if keep is not None and (fmt != "gf4" or fwht_block):
             raise ValueError("keep masks apply to unrotated GF4 packing only")
-        if packer not in ("host", "gpu"):
-            raise ValueError(f"packer must be 'host' or 'gpu', got {packer!r}")
+        if fmt not in C.FMT_BY_NAME:
+            raise ValueError(f"unknown fmt {fmt!r}")
         if fwht_block:
             w = C.fwht_rows(w, fwht_block, nthreads)
-        if fmt == "gf4" and packer == "gpu":
+        if packer == "gpu":
             dev = device if device is not None and torch.device(device).type == "cuda" else "cuda:0"
-            codes, meta = C.quantize_gf4_gpu(w.to(dev), None if keep is None else keep.to(dev))
-            codes, meta = codes.cpu(), meta.cpu()
-        elif fmt == "gf4":
+            if fmt == "gf4":
+                codes, meta = C.quantize_gf4_gpu(w.to(dev), None if keep is None else keep.to(dev))
+            else:
+                codes, meta = C.quantize_e2m1_gpu(w.to(dev))
+            shape = C.make_shape(N, K, 1, C.FMT_BY_NAME[fmt], fwht_block)
+            wdev = C.to_device_layout_gpu(codes, meta, shape)
+            return cls(fmt, N, K, codes.cpu(), meta.cpu(), fwht_block, device,
+                       wdev=wdev if device is not None else wdev.cpu())
+        if fmt == "gf4":
             codes, meta = C.quantize_gf4(w, nthreads, keep)
-        elif fmt == "e2m1" and packer == "gpu":
-            dev = device if device is not None and torch.device(device).type == "cuda" else "cuda:0"
-            codes, meta = C.quantize_e2m1_gpu(w.to(dev))
-            codes, meta = codes.cpu(), meta.cpu()
-        elif fmt == "e2m1":
-            codes, meta = C.quantize_e2m1(w, nthreads)
         else:
-            raise ValueError(f"unknown fmt {fmt!r}")
+            codes, meta = C.quantize_e2m1(w, nthreads)
         return cls(fmt, N, K, codes, meta, fwht_block, device)
 
     @classmethod

@@ -280,6 +280,12 @@ size_t fb_grad_x_workspace_bytes(const fb_shape_t* s, int32_t f16_exact);
 int fb_quantize_gf4_gpu(const float* w, const uint8_t* keep, int32_t N, int32_t K,
                         uint8_t* codes, uint16_t* codebook, void* stream);
 
+/* fb_to_device on the GPU: codes (16-byte aligned), meta (codebooks or scales, 4-byte aligned)
+ * and wdev (fb_device_bytes(s) bytes, 16-byte aligned) are device pointers; the same bytes.
+ * Asynchronous on the stream. */
+int fb_to_device_gpu(const uint8_t* codes, const void* meta, void* wdev, const fb_shape_t* s,
+                     void* stream);
+
 /* E2M1 packer on the GPU: the same rule and bytes as fb_quantize_e2m1, 32 lanes per
  * 32-group.  w fp32 [N,K], codes uint8 [N,K/2] and scales uint8 [N,K/32] are device
  * pointers; asynchronous on the stream; non-finite weights are not detected here. */
