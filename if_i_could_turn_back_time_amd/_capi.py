@@ -42,7 +42,7 @@ EXPORTED = (
     "fb_jenks2_ssd_host", "fb_jenks2_ssd_workspace", "fb_jenks2_ssd_gpu",
     "fb_jenks2_ssd_filters_host", "fb_jenks2_ssd_filters_gpu",
     "fb_gemm", "fb_gemm_workspace_bytes", "fb_grad_x", "fb_grad_x_workspace_bytes",
-    "fb_to_device_gpu",
+    "fb_to_device_gpu", "fb_cast_rows",
 )
 
 
@@ -86,6 +86,7 @@ def lib() -> ctypes.CDLL:
         "fb_gemm_workspace_bytes": (sz, [sp]),
         "fb_grad_x": (ctypes.c_int, [vp, vp, vp, sp, i32, i32, vp, sz, vp]),
         "fb_grad_x_workspace_bytes": (sz, [sp, i32]),
+        "fb_cast_rows": (ctypes.c_int, [vp, i32, i32, i32, vp, i32, i32, vp]),
         "fb_dequant": (ctypes.c_int, [vp, vp, i32, sp, vp]),
         "fb_quantize_gf4_gpu": (ctypes.c_int, [vp, vp, i32, i32, vp, vp, vp]),
         "fb_quantize_e2m1_gpu": (ctypes.c_int, [vp, i32, i32, vp, vp, vp]),
@@ -116,6 +117,25 @@ def lib() -> ctypes.CDLL:
         raise RuntimeError(f"libfourbit ABI {L.fb_abi_version()} != expected {ABI_VERSION}")
     _lib = L
     return L
+
+
+_native = None
+
+
+def native():
+    """The extension module ``_fourbit_torch`` (fourbit_torch.cpp), built beside the library:
+    the forward and the activation gradient as one native call each.  Raises if it has not
+    been built."""
+    global _native
+    if _native is None:
+        lib()
+        try:
+            from . import _fourbit_torch
+        except ImportError as e:
+            raise RuntimeError("_fourbit_torch is missing or does not load: build it with "
+                               "`python -m if_i_could_turn_back_time_amd.build_lib`") from e
+        _native = _fourbit_torch
+    return _native
 
 
 def strerror(code: int) -> str:

@@ -23,6 +23,7 @@ INCLUDE = ROOT / "include"
 BUILD = ROOT / "_build"
 LIB = PKG / "libfourbit.so"
 TRACE_LIB = PKG / "libfourbit_trace.so"
+TORCH_EXT = PKG / "_fourbit_torch.so"
 C_TESTS = ROOT / "tests" / "c"
 ARCH = "gfx950"
 
@@ -46,6 +47,26 @@ def _hipcc() -> str:
         if cand and os.path.exists(cand):
             return cand
     raise RuntimeError("hipcc not found (ROCm is required to build libfourbit.so)")
+
+
+def _torch_extension_cmds(obj: Path, out: Path) -> tuple[list[str], list[str]]:
+    """The compile and link lines of ``_fourbit_torch``: fourbit_torch.cpp against torch's and
+    ROCm's headers, linked to libfourbit.so beside it."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    hip = Path(_hipcc()).resolve().parents[1]
+    inc = [f"-I{p}" for p in cpp_extension.include_paths()]
+    inc += [f"-I{sysconfig.get_paths()['include']}", f"-I{hip / 'include'}", f"-I{INCLUDE}"]
+    comp = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden",
+            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *inc,
+            "-c", str(CSRC / "fourbit_torch.cpp"), "-o", str(obj)]
+    link = ["g++", "-shared", str(obj), "-o", str(out), f"-L{cpp_extension.library_paths()[0]}",
+            "-ltorch_cpu", "-ltorch", "-ltorch_python", "-lc10", "-lc10_hip", f"-L{PKG}",
+            "-l:libfourbit.so", "-Wl,-rpath,$ORIGIN"]
+    return comp, link
 
 
 def _run(cmd: list[str]) -> None:
@@ -92,6 +113,9 @@ def build(verbose: bool = False) -> Path:
         [_hipcc(), *HIP_FLAGS, "-mllvm", "-amdgpu-sched-strategy=max-ilp", "-DFB_PHASE_TRACE",
          *inc, "-c", str(CSRC / "fourbit_gemv_ilp.hip"), "-o", str(trace_ilp_o)],
     ]
+    ext_tmp = TORCH_EXT.with_suffix(".so.tmp")
+    ext_comp, ext_link = _torch_extension_cmds(BUILD / "fourbit_torch.o", ext_tmp)
+    steps.append(ext_comp)
     for cmd in steps:
         if verbose:
             print(" ".join(cmd), flush=True)
@@ -107,6 +131,11 @@ def build(verbose: bool = False) -> Path:
             print(" ".join(link), flush=True)
         _run(link)
         os.replace(tmp, lib)
+    # torch's way in: one native call per forward (needs the library just linked)
+    if verbose:
+        print(" ".join(ext_link), flush=True)
+    _run(ext_link)
+    os.replace(ext_tmp, TORCH_EXT)
     # the GPU test suite's native (no Python) caller of the C ABI, linked to the library
     # through a path relative to itself, so that it runs wherever the tree is copied
     caller = [_hipcc(), *HIP_FLAGS, f"-I{INCLUDE}", str(C_TESTS / "abi_gpu.cpp"), "-o",

@@ -311,6 +311,32 @@ __global__ __launch_bounds__(256) void gemm_sum(const float* __restrict__ part, 
   }
 }
 
+// x [M, K] of one dtype -> [M, ld] of another (round to nearest even), zeros past K: the
+// conversion and the padding to whole groups in one pass.  8 outputs per thread.
+__global__ __launch_bounds__(256) void cast_rows_kernel(const void* __restrict__ x, int xdt,
+                                                        int64_t M, int K,
+                                                        uint16_t* __restrict__ out, int odt,
+                                                        int ld) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
+  if (i >= M * ld) return;
+  const int64_t m = i / ld;
+  const int k = (int)(i - m * ld);
+  const int64_t at = m * K + k;
+  unsigned h[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    float v = 0.f;
+    if (k + e < K)
+      v = xdt == FB_DT_F32   ? static_cast<const float*>(x)[at + e]
+          : xdt == FB_DT_F16 ? (float)static_cast<const _Float16*>(x)[at + e]
+                             : (float)static_cast<const __bf16*>(x)[at + e];
+    h[e] = odt == FB_DT_F16 ? __builtin_bit_cast(unsigned short, (_Float16)v)
+                            : __builtin_bit_cast(unsigned short, (__bf16)v);
+  }
+  *reinterpret_cast<u32x4*>(out + i) = u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16),
+                                             h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
+}
+
 // ---------------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------------
@@ -445,6 +471,24 @@ int fb_gpu::sum_parts(const float* part, int P, int64_t n, void* y, int ydt, int
 }
 
 extern "C" {
+
+int fb_cast_rows(const void* x, int32_t x_dtype, int32_t M, int32_t K, void* out,
+                 int32_t out_dtype, int32_t ld, void* stream) {
+  if (!x || !out) return FB_ERR_NULL;
+  if (M < 1 || K < 1 || ld < K || ld % 128) return FB_ERR_SHAPE;
+  if ((x_dtype != FB_DT_F16 && x_dtype != FB_DT_BF16 && x_dtype != FB_DT_F32) ||
+      (out_dtype != FB_DT_F16 && out_dtype != FB_DT_BF16))
+    return FB_ERR_DTYPE;
+  if ((reinterpret_cast<uintptr_t>(out) & 15u) ||
+      (reinterpret_cast<uintptr_t>(x) & (x_dtype == FB_DT_F32 ? 3u : 1u)))
+    return FB_ERR_ALIGN;
+  const int64_t blocks = ((int64_t)M * ld / 8 + 255) / 256;
+  if (blocks > INT32_MAX) return FB_ERR_SHAPE;
+  hipLaunchKernelGGL(cast_rows_kernel, dim3((unsigned)blocks), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), x, x_dtype, (int64_t)M, K,
+                     static_cast<uint16_t*>(out), out_dtype, ld);
+  return hipGetLastError() == hipSuccess ? FB_OK : FB_ERR_HIP;
+}
 
 size_t fb_gemm_workspace_bytes(const fb_shape_t* s) {
   if (!s || gemm_check(s) != FB_OK) return 0;

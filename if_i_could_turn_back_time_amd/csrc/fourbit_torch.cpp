@@ -1,0 +1,160 @@
+// The packed linear layer's call path from torch: one native call per forward (and per activation
+// gradient) instead of a dozen Python, ctypes and dispatcher steps.  It checks, converts and
+// allocates exactly as linear.py's packed_linear does and launches the same kernels; what it
+// does not recognise (another dtype, a refused shape, a wrapped tensor, an active dispatch
+// mode) it leaves to packed_linear by returning None.  A decode call of a 4096^2 layer takes
+// 5 us on the GPU and took 22 us of host time through Python.
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <optional>
+#include <stdexcept>
+
+#include "fourbit.h"
+
+namespace py = pybind11;
+
+namespace {
+
+constexpr int64_t kMaxGemvBatch = 16;
+constexpr int64_t kMaxGemmK = 1 << 22;  // fb_gemm's limits
+constexpr int64_t kMaxGemmRows = 1 << 24;
+
+void check(int code) {
+  if (code != FB_OK) throw std::runtime_error(fb_strerror(code));
+}
+
+int dtype_code(at::ScalarType t) {
+  return t == at::kHalf ? FB_DT_F16 : t == at::kBFloat16 ? FB_DT_BF16 : t == at::kFloat ? FB_DT_F32 : -1;
+}
+
+// A plain dense GPU tensor whose memory this code may read: no functorch wrapper, fake or
+// functional tensor, and nobody watching the operators.
+bool plain(const at::Tensor& t) {
+  const auto ks = t.key_set();
+  return t.is_cuda() && t.layout() == at::kStrided && t.has_storage() &&
+         !ks.has(c10::DispatchKey::Python) && !ks.has(c10::DispatchKey::Functionalize) &&
+         !ks.has(c10::DispatchKey::FuncTorchBatched) &&
+         !ks.has(c10::DispatchKey::FuncTorchGradWrapper) && !t.is_neg() && !t.is_conj();
+}
+
+bool watched() {
+  return c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+         c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer) ||
+         c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
+
+void* stream_of(const at::Tensor& t) {
+  return c10::hip::getCurrentHIPStream(t.device().index()).stream();
+}
+
+at::Tensor scratch(size_t bytes, const at::Tensor& like) {
+  return at::empty({(int64_t)bytes}, like.options().dtype(at::kByte));
+}
+
+void* ptr_or_null(const at::Tensor& t, size_t bytes) { return bytes ? t.data_ptr() : nullptr; }
+
+// F.linear(x, W, bias) for a packed W, no gradients; None where packed_linear has to decide.
+std::optional<at::Tensor> linear_forward(const at::Tensor& x, const at::Tensor& wdev, int64_t N,
+                                         int64_t K, int64_t fmt, int64_t fwht_block, bool f16_exact,
+                                         bool fp4_mfma, const std::optional<at::Tensor>& bias) {
+  if (watched() || !plain(x) || !plain(wdev) || x.device() != wdev.device() || x.dim() < 1 ||
+      x.size(-1) != K || K < 1 || x.numel() == 0)
+    return std::nullopt;
+  if (bias && (!plain(*bias) || bias->device() != x.device())) return std::nullopt;
+  const int xdt = dtype_code(x.scalar_type());
+  if (xdt < 0) return std::nullopt;
+  const bool e2m1 = fmt == FB_FMT_E2M1;
+  if (fp4_mfma && (!e2m1 || fwht_block)) return std::nullopt;
+  int kdt = xdt;  // the kernels' activation dtype
+  if (!e2m1 || fwht_block)
+    kdt = FB_DT_F16;
+  else if (fp4_mfma || xdt == FB_DT_F32)
+    kdt = FB_DT_BF16;
+  if (e2m1 && kdt == FB_DT_F16 && !f16_exact) return std::nullopt;
+  const int64_t kp = (K + 127) / 128 * 128, M = x.numel() / K;
+  if (M > kMaxGemmRows || (M > kMaxGemvBatch && kp > kMaxGemmK)) return std::nullopt;
+
+  fb_shape_t s{};
+  s.N = (int32_t)N;
+  s.K = (int32_t)kp;
+  s.B = (int32_t)M;
+  s.group = e2m1 ? 32 : 128;
+  s.fmt = (int32_t)fmt;
+  s.fwht_block = (int32_t)fwht_block;
+  s.x_dtype = kdt;
+  s.y_dtype = xdt;
+  if ((size_t)wdev.numel() < fb_device_bytes(&s) || !fb_device_bytes(&s)) return std::nullopt;
+
+  c10::DeviceGuard guard(x.device());
+  void* const stream = stream_of(x);
+  const at::Tensor xc = x.is_contiguous() ? x : x.contiguous();
+  at::Tensor xk = xc;
+  if (kdt != xdt || kp != K) {
+    xk = at::empty({M, kp}, x.options().dtype(kdt == FB_DT_F16 ? at::kHalf : at::kBFloat16));
+    check(fb_cast_rows(xc.data_ptr(), xdt, (int32_t)M, (int32_t)K, xk.data_ptr(), kdt,
+                       (int32_t)kp, stream));
+  }
+  if (reinterpret_cast<uintptr_t>(xk.data_ptr()) & 15u) return std::nullopt;
+  auto sizes = x.sizes().vec();
+  sizes.back() = N;
+  at::Tensor y = at::empty(sizes, x.options());
+  if (M > kMaxGemvBatch) {
+    const size_t need = fb_gemm_workspace_bytes(&s);
+    const at::Tensor ws = need ? scratch(need, x) : at::Tensor();
+    check(fb_gemm(wdev.data_ptr(), xk.data_ptr(), y.data_ptr(), &s, ptr_or_null(ws, need), need,
+                  stream));
+  } else if (fp4_mfma) {
+    const size_t need = fb_mx_workspace_bytes(&s);
+    if (!need) return std::nullopt;
+    const at::Tensor ws = scratch(need, x);
+    check(fb_gemv_mx(wdev.data_ptr(), xk.data_ptr(), y.data_ptr(), &s, ws.data_ptr(), need,
+                     stream));
+  } else {
+    const size_t need = fb_workspace_bytes(&s);
+    const at::Tensor ws = need ? scratch(need, x) : at::Tensor();
+    check(fb_gemv(wdev.data_ptr(), xk.data_ptr(), y.data_ptr(), &s, ptr_or_null(ws, need), need,
+                  stream));
+  }
+  if (bias) y.add_(bias->scalar_type() == y.scalar_type() ? *bias : bias->to(y.scalar_type()));
+  return y;
+}
+
+// gx[M, K] = (gy . W) H for gy [M, N], in xdtype; None where the caller has to decide.
+std::optional<at::Tensor> linear_grad_x(const at::Tensor& gy, const at::Tensor& wdev, int64_t N,
+                                        int64_t K, int64_t fmt, int64_t fwht_block, bool f16_exact,
+                                        at::ScalarType xt) {
+  const int gdt = dtype_code(gy.scalar_type()), xdt = dtype_code(xt);
+  const int64_t kp = (K + 127) / 128 * 128;
+  if (watched() || !plain(gy) || !plain(wdev) || gy.device() != wdev.device() || gy.dim() != 2 ||
+      gy.size(1) != N || gdt < 0 || xdt < 0 || gy.numel() == 0 || gy.size(0) > kMaxGemmRows)
+    return std::nullopt;
+  fb_shape_t s{};
+  s.N = (int32_t)N;
+  s.K = (int32_t)kp;
+  s.B = (int32_t)gy.size(0);
+  s.group = fmt == FB_FMT_E2M1 ? 32 : 128;
+  s.fmt = (int32_t)fmt;
+  s.fwht_block = (int32_t)fwht_block;
+  s.x_dtype = FB_DT_F16;
+  s.y_dtype = gdt;
+  const size_t need = fb_grad_x_workspace_bytes(&s, f16_exact);
+  if (!need || (size_t)wdev.numel() < fb_device_bytes(&s)) return std::nullopt;
+  c10::DeviceGuard guard(gy.device());
+  const at::Tensor g = gy.contiguous();
+  at::Tensor gx = at::empty({gy.size(0), kp}, gy.options().dtype(xt));
+  const at::Tensor ws = scratch(need, gy);
+  check(fb_grad_x(wdev.data_ptr(), g.data_ptr(), gx.data_ptr(), &s, xdt, f16_exact, ws.data_ptr(),
+                  need, stream_of(gy)));
+  return kp == K ? gx : gx.narrow(1, 0, K).contiguous();
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_fourbit_torch, m) {
+  m.def("linear_forward", &linear_forward);
+  m.def("linear_grad_x", &linear_grad_x);
+}

@@ -191,35 +191,60 @@ class _PackedLinearFn(torch.autograd.Function):
     operations on W decoded in chunks of row tiles (``_grad_x``)."""
 
     @staticmethod
-    def forward(ctx, x2, wdev, N, K, fmt, fwht_block, range_check, f16_exact, fp4_mfma=False,
-                ws_cache=None):
-        xk = _kernel_input(x2, K, fmt, fwht_block, range_check, f16_exact, fp4_mfma)
-        ydt = x2.dtype if x2.dtype in C.DTYPE_CODE else torch.float32
-        y = torch.empty(x2.shape[0], N, dtype=ydt, device=x2.device)
-        _gemv_chunks(wdev, N, packed_k(K), fmt, fwht_block, xk, y, fp4_mfma, ws_cache)
+    def forward(ctx, x2, bias, wdev, N, K, fmt, fwht_block, range_check, f16_exact,
+                fp4_mfma=False, ws_cache=None):
+        y = None
+        if not range_check:
+            y = _native_forward(x2, wdev, N, K, fmt, fwht_block, f16_exact, fp4_mfma, bias)
+        if y is None:
+            y = _forward(x2, wdev, N, K, fmt, fwht_block, range_check, f16_exact, fp4_mfma,
+                         ws_cache)
+            if bias is not None:
+                y.add_(bias.to(y.dtype))
         ctx.save_for_backward(wdev)
-        ctx.cfg = (N, K, fmt, fwht_block, x2.dtype, f16_exact)
+        ctx.cfg = (N, K, fmt, fwht_block, x2.dtype, f16_exact,
+                   None if bias is None else bias.dtype)
         return y
 
     @staticmethod
     def backward(ctx, gy):
         (wdev,) = ctx.saved_tensors
-        N, K, fmt, fwht_block, xdt, f16_exact = ctx.cfg
-        if not torch.is_grad_enabled() and N <= MAX_GRAD_N and gy.dtype in C.DTYPE_CODE:
-            kp = packed_k(K)
-            gx = torch.empty(gy.shape[0], kp, device=gy.device,
-                             dtype=xdt if xdt in C.DTYPE_CODE else torch.float32)
-            if gx.numel():
-                C.grad_x(wdev, gy.contiguous(), gx,
-                         C.make_shape(N, kp, gy.shape[0], C.FMT_BY_NAME[fmt], fwht_block,
-                                      C.DT_F16, C.DTYPE_CODE[gy.dtype]), f16_exact)
-            if kp != K:
-                gx = gx[:, :K].contiguous()
-            return gx.to(xdt), None, None, None, None, None, None, None, None, None
-        gx = _grad_x(wdev, N, packed_k(K), fmt, fwht_block, gy)
-        if fwht_block:
-            gx = _fwht_last_dim(gx, fwht_block)
-        return gx[:, :K].to(xdt), None, None, None, None, None, None, None, None, None
+        N, K, fmt, fwht_block, xdt, f16_exact, bdt = ctx.cfg
+        gb = gy.sum(0).to(bdt) if ctx.needs_input_grad[1] else None
+        gx = None
+        if ctx.needs_input_grad[0]:
+            if not torch.is_grad_enabled() and N <= MAX_GRAD_N and type(gy) is torch.Tensor:
+                gx = C.native().linear_grad_x(gy, wdev, N, K, C.FMT_BY_NAME[fmt], fwht_block,
+                                              f16_exact,
+                                              xdt if xdt in C.DTYPE_CODE else torch.float32)
+            if gx is None:
+                gx = _grad_x(wdev, N, packed_k(K), fmt, fwht_block, gy)
+                if fwht_block:
+                    gx = _fwht_last_dim(gx, fwht_block)
+                gx = gx[:, :K]
+            gx = gx.to(xdt)
+        return gx, gb, None, None, None, None, None, None, None, None, None
+
+
+def _forward(x2, wdev, N, K, fmt, fwht_block, range_check, f16_exact, fp4_mfma, ws_cache):
+    """y = x2 W^T through torch and ctypes calls, for what the native call does not take."""
+    xk = _kernel_input(x2, K, fmt, fwht_block, range_check, f16_exact, fp4_mfma)
+    ydt = x2.dtype if x2.dtype in C.DTYPE_CODE else torch.float32
+    y = torch.empty(x2.shape[0], N, dtype=ydt, device=x2.device)
+    _gemv_chunks(wdev, N, packed_k(K), fmt, fwht_block, xk, y, fp4_mfma, ws_cache)
+    return y
+
+
+_PLAIN = (torch.Tensor, nn.Parameter)
+
+
+def _native_forward(x, wdev, N, K, fmt, fwht_block, f16_exact, fp4_mfma, bias):
+    """The whole forward in one native call (fourbit_torch.cpp), or None where x, the weight or
+    the bias is not a plain GPU tensor it takes."""
+    if type(x) not in _PLAIN or (bias is not None and type(bias) not in _PLAIN):
+        return None
+    return C.native().linear_forward(x, wdev, N, K, C.FMT_BY_NAME[fmt], fwht_block, f16_exact,
+                                     fp4_mfma, bias)
 
 
 def packed_linear(wdev: torch.Tensor, N: int, K: int, fmt: str, fwht_block: int,
@@ -241,6 +266,12 @@ def packed_linear(wdev: torch.Tensor, N: int, K: int, fmt: str, fwht_block: int,
     split into two MX-E4M3 terms, which hold a bf16 value exactly unless its 32-value block
     spans more than E4M3's exponent range (fp16 and fp32 x are rounded to bf16 first).  No
     CPU path: x must be on the GPU."""
+    grad = torch.is_grad_enabled()
+    bias_grad = grad and bias is not None and bias.requires_grad
+    if not (range_check or bias_grad or (grad and x.requires_grad)):
+        y = _native_forward(x, wdev, N, K, fmt, fwht_block, f16_exact, fp4_mfma, bias)
+        if y is not None:
+            return y
     if x.dim() == 0 or x.shape[-1] != K:
         raise RuntimeError(f"packed linear: input of shape {tuple(x.shape)} does not end in "
                            f"in_features={K}")
@@ -251,28 +282,18 @@ def packed_linear(wdev: torch.Tensor, N: int, K: int, fmt: str, fwht_block: int,
         raise ValueError("the native FP4 path (fp4_mfma) takes unrotated E2M1 weights")
     lead = x.shape[:-1]
     x2 = x.reshape(-1, K)
-    if torch.is_grad_enabled() and x.requires_grad:
-        y = _PackedLinearFn.apply(x2, wdev, N, K, fmt, fwht_block, range_check, f16_exact,
+    if grad and x.requires_grad:
+        y = _PackedLinearFn.apply(x2, bias, wdev, N, K, fmt, fwht_block, range_check, f16_exact,
                                   fp4_mfma, ws_cache)
-        if bias is not None:
-            y = y + bias.to(y.dtype)
         return y.reshape(*lead, N)
     with torch.no_grad():
-        y = _PackedLinearFn.forward(_NoCtx(), x2, wdev, N, K, fmt, fwht_block, range_check,
-                                    f16_exact, fp4_mfma, ws_cache)
+        y = _forward(x2, wdev, N, K, fmt, fwht_block, range_check, f16_exact, fp4_mfma, ws_cache)
     if bias is not None:
-        if torch.is_grad_enabled() and bias.requires_grad:
+        if bias_grad:
             y = y + bias.to(y.dtype)
         else:
             y.add_(bias.to(y.dtype))  # y is this call's own buffer
     return y.reshape(*lead, N)
-
-
-class _NoCtx:
-    """Stand-in for the autograd context when no graph is built."""
-
-    def save_for_backward(self, *a):
-        pass
 
 
 class PackedWeight:

@@ -185,6 +185,12 @@ int fb_gemm(const void* wdev, const void* x, void* y, const fb_shape_t* s, void*
  * not take). */
 size_t fb_gemm_workspace_bytes(const fb_shape_t* s);
 
+/* Activations into the kernels' form: x [M, K] (F16, BF16 or F32) as out [M, ld] of F16 or BF16,
+ * rounded to nearest even, zeros from K to ld (a multiple of 128, >= K).  Device pointers, out
+ * 16-byte aligned; asynchronous on the stream. */
+int fb_cast_rows(const void* x, int32_t x_dtype, int32_t M, int32_t K, void* out,
+                 int32_t out_dtype, int32_t ld, void* stream);
+
 /* fb_gemv that allocates nothing and takes no workspace.  No counterpart in the reference:
  * it is for callers that cannot allocate device memory around a call (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  The once-per-call
