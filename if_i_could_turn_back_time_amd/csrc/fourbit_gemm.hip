@@ -2,7 +2,8 @@
 // W^T, one launch over all of x, where 16-row GEMV calls would read and decode the whole
 // weight once per 16 rows.
 //
-// Workgroup tile: (64 RT rows of W) x (16 CT rows of x), 4 waves, one per SIMD; each wave owns
+// Workgroup tile: (64 RT rows of W) x (16 CT rows of x), 4 waves, one per SIMD, two workgroups
+// per CU; each wave owns
 // RT 16-row weight tiles and all CT column tiles, RT * CT * 4 fp32 accumulators per lane.
 //  - W goes from the device stream straight into MFMA A operands, as in the GEMV: lane L's 16
 //    bytes of a block are row L % 16, item L / 16, so no weight passes through LDS.  Every
@@ -12,17 +13,17 @@
 //    write LDS directly (no VGPRs, no ds_write); the 16-byte units of an x row are permuted by
 //    unit ^ (row % 16) on the load's source side, which leaves the MFMA B reads (16 rows, 256
 //    bytes apart) without a bank conflict.
-//  - Nibbles and x are requested kBufs - 1 chunks ahead (3 where four chunks fit the LDS that
-//    the occupancy allows, else 1), with one barrier per chunk.
+//  - Nibbles and x are requested kBufs - 1 (1 or 3) chunks ahead, with one barrier per chunk.
 //  - Each k-step's decode (21 VALU instructions per GF4 row tile, 8 codes per lane) is written
 //    between the MFMAs of the step before it, a half decode per column tile, and the column
-//    tiles are separate scheduling regions: with one or two waves per SIMD the decode only
-//    hides behind the MFMAs if the instruction stream alternates them.
+//    tiles are separate scheduling regions, so that the instruction stream alternates the two
+//    (left to itself the compiler groups them, and a wave then waits for its own MFMAs).
 // What bounds it: E2M1 runs at the matrix cores' power-limited rate (8192 -> 28672, M = 2048:
-// 737 us, 1305 TFLOP/s; the library's bf16 GEMM of 8192^3 reaches 1418 on the same card);
-// GF4 issues as many cycles of decode and MFMA instructions as its MFMAs take (1006 us, 956
-// TFLOP/s; 16-row GEMV calls: 4840 us).  Small M is bound by latency and the x fill of each
-// CU; the K range is then cut into P parts whose fp32 sums gemm_sum adds in part order.
+// 635 us, 1515 TFLOP/s; the library's bf16 GEMM of 8192^3 reaches 1418 on the same card; one
+// workgroup of wider staging per CU: 737 us); GF4 issues nearly as many cycles of decode and MFMA
+// instructions as its MFMAs take (964 us, 998 TFLOP/s; 16-row GEMV calls: 4840 us; one workgroup
+// per CU: 1006).  Small M is bound by latency and the x fill of each CU; the K range is then
+// cut into P parts whose fp32 sums gemm_sum adds in part order.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -65,14 +66,15 @@ struct GemmTile {
   static constexpr int kRows = RT * 16 * kGemmWaves;  // rows of W
   static constexpr int kCols = CT * 16;               // rows of x
   static constexpr int kBuf = kCols * kRowBytes;      // one staged chunk
-  // CT <= 4: four chunks in at most 64 KiB, so two workgroups share a CU; CT = 8: four chunks
-  // in 128 KiB, one workgroup; CT = 6: two or four would both leave one workgroup per CU
-  static constexpr int kBufs = kBuf * 4 <= 128 * 1024 ? 4 : 2;
-  static constexpr int kOcc = kBuf * kBufs <= 80 * 1024 ? 2 : 1;
+  // Two workgroups share a CU (two waves per SIMD: one's decode issues while the other's
+  // MFMAs run), so two chunks of the wide tiles are staged at a time; four of the small ones,
+  // whose chunks are too short to cover a request's latency.
+  static constexpr int kBufs = kBuf * 4 <= 64 * 1024 && RT * CT <= 12 ? 4 : 2;
+  static_assert(kBuf * kBufs <= 80 * 1024, "two workgroups per CU");
 };
 
 template <int FMT, int XDT, int RT, int CT>
-__global__ __launch_bounds__(kGemmWaves * 64, (GemmTile<RT, CT>::kOcc)) void gemm_kernel(GemmArgs a) {
+__global__ __launch_bounds__(kGemmWaves * 64, 2) void gemm_kernel(GemmArgs a) {
   using T = GemmTile<RT, CT>;
   constexpr int BB = FMT == FB_FMT_GF4 ? fb::kGf4BlockBytes : fb::kE2m1BlockBytes;
   constexpr int NB = T::kBufs, D = NB - 1;
@@ -341,22 +343,26 @@ __global__ __launch_bounds__(256) void cast_rows_kernel(const void* __restrict__
 // host side
 // ---------------------------------------------------------------------------------
 // Tile shapes the plan chooses from, with the time in us that a span (512 K-values) of one
-// tile takes on a CU when one workgroup runs there (one) and when two do (two, both done;
-// 0: LDS holds one workgroup).  Fitted to 2,300 timings of every shape and part count over
-// M = 17..1024 on 4096^2, 8192^2, 4096 -> 11008, 11008 -> 4096 and 8192 -> 28672; the plan it
-// picks is within 2% (geometric mean; 17% at worst) of the best one timed.  A table rather
-// than a formula because the costs follow no simple one: small tiles are bound by latency
-// and the x fill, large GF4 tiles by instruction issue, large E2M1 tiles by the MFMAs.
+// tile takes on a CU when one workgroup runs there and when two do (both done).  Fitted to
+// 6,000 timings of every shape and part count over M = 17..2048 on 4096^2, 8192^2, 4096 ->
+// 11008, 11008 -> 4096 and 8192 -> 28672; the plan it picks is within 1.1% (geometric mean; 12%
+// at worst) of the best one timed.  A table rather than a formula because the costs follow no
+// simple one: small tiles are bound by latency and the x fill, GF4's wide ones by instruction
+// issue (RT = 4 does not fit two workgroups' registers there), E2M1's by the MFMAs.
 struct GemmShape {
   int rt, ct;
-  float one[2], two[2];  // [GF4, E2M1]
+  float one, two;
 };
-constexpr GemmShape kGemmShapes[] = {
-    {4, 8, {7.12f, 5.37f}, {0, 0}},         {4, 4, {5.10f, 2.76f}, {8.24f, 4.55f}},
-    {3, 6, {4.82f, 3.23f}, {0, 0}},         {2, 6, {3.47f, 2.33f}, {0, 0}},
-    {2, 4, {2.65f, 1.51f}, {4.48f, 2.84f}}, {2, 3, {2.34f, 1.26f}, {3.79f, 2.23f}},
-    {2, 2, {1.92f, 1.07f}, {3.21f, 1.73f}},
-};
+constexpr GemmShape kGf4Shapes[] = {{3, 8, 5.65f, 9.84f}, {3, 6, 4.52f, 8.04f},
+                                    {2, 8, 4.08f, 7.35f}, {2, 6, 3.26f, 5.82f},
+                                    {2, 4, 2.69f, 4.82f}, {2, 3, 2.36f, 3.93f},
+                                    {2, 2, 1.94f, 3.34f}};
+constexpr GemmShape kE2m1Shapes[] = {{4, 8, 5.32f, 8.83f}, {4, 6, 3.89f, 6.70f},
+                                     {4, 4, 2.74f, 4.85f}, {3, 6, 3.04f, 5.44f},
+                                     {4, 3, 2.23f, 4.12f}, {2, 4, 1.55f, 3.15f},
+                                     {2, 3, 1.28f, 2.39f}, {2, 2, 1.08f, 1.86f}};
+// the same fits' cost of a part-sum launch and of its traffic per million fp32 sums
+constexpr float kSumCost[] = {2.32f, 2.68f}, kSumPerMillion[] = {1.27f, 1.25f};
 constexpr int kMaxParts = 8;
 constexpr int64_t kMaxPartBytes = 256ll << 20;
 
@@ -364,26 +370,22 @@ struct GemmPlan {
   int rt = 0, ct = 0, P = 1;
 };
 
-GemmPlan gemm_plan(const fb_shape_t* s, int cus) {
+template <size_t NS>
+GemmPlan gemm_plan(const fb_shape_t* s, int cus, const GemmShape (&shapes)[NS], double sum_cost,
+                   double sum_per_million) {
   const int GS = (s->K / 128 + 3) / 4;
-  const int f = s->fmt == FB_FMT_GF4 ? 0 : 1;
-  const double mn = 1e-6 * s->B * (double)s->N;
-  // the same fit's cost of a part-sum launch, and of its traffic per million fp32 sums
-  const double sum0 = f ? 2.23 : 1.79, sum1 = f ? 1.70 : 1.83;
   GemmPlan best;
   double bt = 0;
-  for (const GemmShape& c : kGemmShapes) {
+  for (const GemmShape& c : shapes) {
     const int64_t T = (int64_t)((s->N + c.rt * 64 - 1) / (c.rt * 64)) *
                       ((s->B + c.ct * 16 - 1) / (c.ct * 16));
-    const int occ = c.two[f] > 0 ? 2 : 1;
     for (int P = 1; P <= kMaxParts && P <= GS; ++P) {
       const int S = (GS + P - 1) / P;
       if (S * (P - 1) >= GS) continue;  // an empty part
       if (P > 1 && 4 * (int64_t)P * s->B * s->N > kMaxPartBytes) break;
-      const int64_t slots = (int64_t)cus * occ, full = T * P / slots, rem = T * P % slots;
-      double t = S * (full * (occ == 2 ? c.two[f] : c.one[f]) +
-                      (rem == 0 ? 0.0 : rem <= cus ? c.one[f] : c.two[f]));
-      if (P > 1) t += sum0 + sum1 * mn * P;
+      const int64_t slots = 2 * (int64_t)cus, full = T * P / slots, rem = T * P % slots;
+      double t = S * (full * c.two + (rem == 0 ? 0.0 : rem <= cus ? c.one : c.two));
+      if (P > 1) t += sum_cost + sum_per_million * 1e-6 * s->B * (double)s->N * P;
       if (!best.rt || t < bt) {
         bt = t;
         best.rt = c.rt;
@@ -393,6 +395,11 @@ GemmPlan gemm_plan(const fb_shape_t* s, int cus) {
     }
   }
   return best;
+}
+
+GemmPlan gemm_plan(const fb_shape_t* s, int cus) {
+  return s->fmt == FB_FMT_GF4 ? gemm_plan(s, cus, kGf4Shapes, kSumCost[0], kSumPerMillion[0])
+                              : gemm_plan(s, cus, kE2m1Shapes, kSumCost[1], kSumPerMillion[1]);
 }
 
 template <int FMT, int XDT, int RT, int CT>
@@ -410,11 +417,19 @@ int launch_gemm(GemmArgs a, int P, hipStream_t hs) {
 
 template <int FMT, int XDT>
 int launch_gemm_tile(const GemmArgs& a, const GemmPlan& pl, hipStream_t hs) {
-  switch (pl.rt * 100 + pl.ct) {
-    case 408: return launch_gemm<FMT, XDT, 4, 8>(a, pl.P, hs);
-    case 404: return launch_gemm<FMT, XDT, 4, 4>(a, pl.P, hs);
+  const int shape = pl.rt * 100 + pl.ct;
+  if constexpr (FMT == FB_FMT_GF4) {
+    if (shape == 308) return launch_gemm<FMT, XDT, 3, 8>(a, pl.P, hs);
+    if (shape == 208) return launch_gemm<FMT, XDT, 2, 8>(a, pl.P, hs);
+    if (shape == 206) return launch_gemm<FMT, XDT, 2, 6>(a, pl.P, hs);
+  } else {
+    if (shape == 408) return launch_gemm<FMT, XDT, 4, 8>(a, pl.P, hs);
+    if (shape == 406) return launch_gemm<FMT, XDT, 4, 6>(a, pl.P, hs);
+    if (shape == 404) return launch_gemm<FMT, XDT, 4, 4>(a, pl.P, hs);
+    if (shape == 403) return launch_gemm<FMT, XDT, 4, 3>(a, pl.P, hs);
+  }
+  switch (shape) {
     case 306: return launch_gemm<FMT, XDT, 3, 6>(a, pl.P, hs);
-    case 206: return launch_gemm<FMT, XDT, 2, 6>(a, pl.P, hs);
     case 204: return launch_gemm<FMT, XDT, 2, 4>(a, pl.P, hs);
     case 203: return launch_gemm<FMT, XDT, 2, 3>(a, pl.P, hs);
     default: return launch_gemm<FMT, XDT, 2, 2>(a, pl.P, hs);
