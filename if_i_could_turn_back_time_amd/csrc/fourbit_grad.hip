@@ -12,8 +12,8 @@
 //     precision of an fp32 GEMM of the exact weight.
 // The matrix cores do 16-bit products 16 times as fast as fp32 ones, so even fp32 gy against
 // GF4 (6 term pairs) is faster than an fp32 GEMM.  Measured (us; the fp32 decode and library
-// GEMM of before): GF4 4096^2, M = 256, fp16 gy: 28 (about 190); GF4 8192^2, M = 1024: 161 fp16,
-// 358 bf16, 852 fp32.  At M <= 64 it is bound by pass 1 (10 us + 0.35 us per million weights and
+// GEMM of before): GF4 4096^2, M = 256, fp16 gy: 29 (about 190); GF4 8192^2, M = 1024: 163 fp16,
+// 329 bf16, 819 fp32.  At M <= 64 it is bound by pass 1 (10 us + 0.35 us per million weights and
 // plane: the 16-bit stores), beyond by the MFMAs (1,080 TFLOP/s at M = 1024).
 #include <hip/hip_runtime.h>
 
@@ -183,12 +183,12 @@ struct GradTile {
   static constexpr int kRows = RT * 16 * kGradWaves;
   static constexpr int kCols = CT * 16;
   static constexpr int kBuf = kCols * kRowBytes;
-  static constexpr int kBufs = kBuf * 4 <= 128 * 1024 ? 4 : 2;
-  static constexpr int kOcc = kBuf * kBufs <= 80 * 1024 ? 2 : 1;
+  static constexpr int kBufs = kBuf * 4 <= 64 * 1024 ? 4 : 2;
+  static_assert(kBuf * kBufs <= 80 * 1024, "two workgroups per CU");
 };
 
 template <int XDT, int RT, int CT>
-__global__ __launch_bounds__(kGradWaves * 64, (GradTile<RT, CT>::kOcc)) void grad_gemm_kernel(
+__global__ __launch_bounds__(kGradWaves * 64, 2) void grad_gemm_kernel(
     GradArgs g) {
   using T = GradTile<RT, CT>;
   constexpr int NB = T::kBufs, D = NB - 1;
@@ -402,16 +402,16 @@ constexpr int kMaxParts = 8;
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 
 // Tile shapes with the time in us that a chunk (128 contraction values) of one tile takes on a
-// CU when one workgroup runs there and when two do (0: LDS holds one).  Fitted to 1,500 timings
-// of every shape and part count over M = 17..1024, 1 to 6 term pairs and 5 layers of 1024 ->
-// 2048 to 8192^2; the plan it picks is within 2.3% (geometric mean; 20% at worst) of the best.
+// CU when one workgroup runs there and when two do.  Fitted to 2,900 timings of these and of six
+// other shapes at every part count, over M = 17..1024, 1 to 6 term pairs and 5 layers of 1024 ->
+// 2048 to 8192^2; the plan it picks is within 2.9% (geometric mean; 19% at worst) of the best.
 struct GradShape {
   int rt, ct;
   float one, two;
 };
 constexpr GradShape kGradShapes[] = {
-    {4, 8, 1.83f, 0}, {4, 4, 1.17f, 2.01f}, {2, 4, 0.66f, 1.19f}, {2, 2, 0.50f, 0.915f}};
-constexpr float kSumCost = 4.6f, kSumPerMillion = 1.33f;  // the part sum's, the same fit
+    {3, 8, 1.41f, 2.39f}, {2, 8, 1.05f, 1.84f}, {2, 4, 0.66f, 1.21f}, {2, 2, 0.50f, 0.92f}};
+constexpr float kSumCost = 4.6f, kSumPerMillion = 1.17f;  // the part sum's, the same fit
 
 struct GradPlan {
   int mode = 0;      // grad_decode_kernel's MODE
@@ -422,7 +422,7 @@ struct GradPlan {
   int want = 0;      // terms of gy to make: bit 0 t0, 1 finite t0, 2 t1, 3 t2
   int QN = 0, GS = 0, ldb = 0;
   int spans = 0;     // spans of K decoded at once
-  int rt = 4, ct = 8, P = 1;
+  int rt = 0, ct = 0, P = 1;
   size_t a_bytes = 0, b_bytes = 0, part_bytes = 0, rot_bytes = 0;
   size_t total() const { return a_bytes + b_bytes + part_bytes + rot_bytes; }
 };
@@ -435,14 +435,12 @@ void grad_tiles(GradPlan& pl, int M, int K, int cus) {
     const int kw = std::min(K, pl.spans * 512);
     const int64_t T = (int64_t)((kw + c.rt * 64 - 1) / (c.rt * 64)) *
                       ((M + c.ct * 16 - 1) / (c.ct * 16));
-    const int occ = c.two > 0 ? 2 : 1;
     for (int P = 1; P <= kMaxParts && P <= total; ++P) {
       const int S = (total + P - 1) / P;
       if (S * (P - 1) >= total) continue;
       if (P > 1 && 4 * (int64_t)P * M * K > kMaxPartBytes) break;
-      const int64_t slots = (int64_t)cus * occ, full = T * P / slots, rem = T * P % slots;
-      double t = S * (full * (occ == 2 ? c.two : c.one) +
-                      (rem == 0 ? 0.0 : rem <= cus ? c.one : c.two));
+      const int64_t slots = 2 * (int64_t)cus, full = T * P / slots, rem = T * P % slots;
+      double t = S * (full * c.two + (rem == 0 ? 0.0 : rem <= cus ? c.one : c.two));
       if (P > 1) t += kSumCost + kSumPerMillion * 1e-6 * M * (double)K * P;
       if (!have || t < bt) {
         have = true;
@@ -517,8 +515,8 @@ int launch_grad(GradArgs g, int P, int kw, hipStream_t hs) {
 template <int XDT>
 int launch_grad_tile(const GradArgs& g, const GradPlan& pl, int kw, hipStream_t hs) {
   switch (pl.rt * 100 + pl.ct) {
-    case 408: return launch_grad<XDT, 4, 8>(g, pl.P, kw, hs);
-    case 404: return launch_grad<XDT, 4, 4>(g, pl.P, kw, hs);
+    case 308: return launch_grad<XDT, 3, 8>(g, pl.P, kw, hs);
+    case 208: return launch_grad<XDT, 2, 8>(g, pl.P, kw, hs);
     case 204: return launch_grad<XDT, 2, 4>(g, pl.P, kw, hs);
     default: return launch_grad<XDT, 2, 2>(g, pl.P, kw, hs);
   }
