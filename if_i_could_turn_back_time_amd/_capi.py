@@ -82,7 +82,7 @@ def lib() -> ctypes.CDLL:
         "fb_from_device": (ctypes.c_int, [vp, vp, vp, sp]),
         "fb_dequant_host": (ctypes.c_int, [vp, vp, vp, sp]),
         "fb_gemv": (ctypes.c_int, [vp, vp, vp, sp, vp, sz, vp]),
-        "fb_gemm": (ctypes.c_int, [vp, vp, vp, sp, vp, sz, vp]),
+        "fb_gemm": (ctypes.c_int, [vp, vp, vp, sp, vp, i32, vp, sz, vp]),
         "fb_gemm_workspace_bytes": (sz, [sp]),
         "fb_grad_x": (ctypes.c_int, [vp, vp, vp, sp, i32, i32, vp, sz, vp]),
         "fb_grad_x_workspace_bytes": (sz, [sp, i32]),
@@ -337,15 +337,21 @@ def _check_gemv_operands(name, wdev, x, y, shape):
         raise ValueError("weight stream is smaller than fb_device_bytes(shape)")
 
 
-def gemm(wdev: torch.Tensor, x: torch.Tensor, y: torch.Tensor, shape: FbShape) -> torch.Tensor:
-    """y[B,N] = x'[B,K] . W^T on the GPU for any number of rows (asynchronous on the current
+def gemm(wdev: torch.Tensor, x: torch.Tensor, y: torch.Tensor, shape: FbShape,
+         bias: torch.Tensor | None = None) -> torch.Tensor:
+    """y[B,N] = x'[B,K] . W^T (+ bias [N]) on the GPU for any number of rows (asynchronous on the current
     stream).  The workspace is the allocator's, for this call only: rotated x and part sums
     of a long prompt are too large to keep per layer."""
     _check_gemv_operands("fb_gemm", wdev, x, y, shape)
+    if bias is not None and (bias.device != x.device or not bias.is_contiguous()
+                             or bias.dtype not in DTYPE_CODE or tuple(bias.shape) != (shape.N,)):
+        raise ValueError("bias must be a contiguous float [N] tensor on x's device")
     need = lib().fb_gemm_workspace_bytes(ctypes.byref(shape))
     with torch.cuda.device(x.device):
         ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
         check(lib().fb_gemm(_ptr(wdev), _ptr(x), _ptr(y), ctypes.byref(shape),
+                            _ptr(bias) if bias is not None else None,
+                            DTYPE_CODE[bias.dtype] if bias is not None else 0,
                             _ptr(ws) if need else None, need, _stream(x.device)))
     return y
 

@@ -35,6 +35,12 @@ __device__ __forceinline__ void store_y(void* y, int64_t idx, float v, int ydt) 
   }
 }
 
+__device__ __forceinline__ float load_as_float(const void* p, int64_t idx, int dt) {
+  return dt == FB_DT_F32   ? static_cast<const float*>(p)[idx]
+         : dt == FB_DT_F16 ? (float)static_cast<const _Float16*>(p)[idx]
+                           : (float)static_cast<const __bf16*>(p)[idx];
+}
+
 // Four outputs at idx, which 16-byte alignment of y and idx % 4 == 0 make one store.
 __device__ __forceinline__ void store4(void* y, int64_t idx, const f32x4& v, int ydt) {
   if (ydt == FB_DT_F32) {

@@ -40,7 +40,8 @@ __attribute__((visibility("hidden"))) int cu_count();
 __attribute__((visibility("hidden"))) int rotate_rows(const void* x, void* xo, int rows, int K,
                                                       int block, hipStream_t hs);
 __attribute__((visibility("hidden"))) int sum_parts(const float* part, int P, int64_t n, void* y,
-                                                    int ydt, int vec, hipStream_t hs);
+                                                    int ydt, int vec, const void* bias, int bdt,
+                                                    int N, hipStream_t hs);
 }  // namespace fb_gpu
 
 namespace {
@@ -53,11 +54,12 @@ struct GemmArgs {
   const void* x;
   void* y;
   float* part;  // P > 1: the parts' fp32 sums [P, M, N]; else null
+  const void* bias;  // [N] of dtype bdt, or null; added in fp32 before y's one rounding
   int M, N, K;
   int GS;       // spans per row
   int tiles_n, tiles_m;
   int spp;      // spans per K-part
-  int ydt;
+  int ydt, bdt;
   int vec;      // y (and part) rows take 4-value stores: N % 4 == 0, 16-byte aligned y
 };
 
@@ -264,6 +266,17 @@ __global__ __launch_bounds__(kGemmWaves * 64, 2) void gemm_kernel(GemmArgs a) {
   }
 
   // lane: x row 16 ct + lane % 16, weight rows 4 (lane / 16) .. + 3 of each row tile
+  if (a.bias && !a.part) {
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      f32x4 b;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        b[e] = load_as_float(a.bias, min((t0 + r) * 16 + (lane >> 4) * 4 + e, a.N - 1), a.bdt);
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) acc[r][ct] += b;
+    }
+  }
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
     const int m = ct * 16 + (lane & 15);
@@ -293,9 +306,11 @@ __global__ __launch_bounds__(kGemmWaves * 64, 2) void gemm_kernel(GemmArgs a) {
   }
 }
 
-// y = the P parts' sums added in part order (deterministic), four outputs per thread.
+// y = the P parts' sums added in part order (deterministic) plus the bias of column i % N, four
+// outputs per thread.
 __global__ __launch_bounds__(256) void gemm_sum(const float* __restrict__ part, int P, int64_t n,
-                                                void* __restrict__ y, int ydt, int vec) {
+                                                void* __restrict__ y, int ydt, int vec,
+                                                const void* __restrict__ bias, int bdt, int N) {
   const int64_t i0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i0 >= n) return;
   if (vec) {
@@ -303,11 +318,17 @@ __global__ __launch_bounds__(256) void gemm_sum(const float* __restrict__ part, 
 #pragma unroll 4
     for (int p = 1; p < P; ++p)
       a += __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(part + (int64_t)p * n + i0));
+    if (bias) {  // vec: N % 4 == 0, so the four columns are consecutive
+      const int c = (int)(i0 % N);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a[e] += load_as_float(bias, c + e, bdt);
+    }
     store4(y, i0, a, ydt);
   } else {
     for (int64_t i = i0; i < min(n, i0 + 4); ++i) {
       float a = part[i];
       for (int p = 1; p < P; ++p) a += part[(int64_t)p * n + i];
+      if (bias) a += load_as_float(bias, i % N, bdt);
       store_y(y, i, a, ydt);
     }
   }
@@ -328,10 +349,7 @@ __global__ __launch_bounds__(256) void cast_rows_kernel(const void* __restrict__
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     float v = 0.f;
-    if (k + e < K)
-      v = xdt == FB_DT_F32   ? static_cast<const float*>(x)[at + e]
-          : xdt == FB_DT_F16 ? (float)static_cast<const _Float16*>(x)[at + e]
-                             : (float)static_cast<const __bf16*>(x)[at + e];
+    if (k + e < K) v = load_as_float(x, at + e, xdt);
     h[e] = odt == FB_DT_F16 ? __builtin_bit_cast(unsigned short, (_Float16)v)
                             : __builtin_bit_cast(unsigned short, (__bf16)v);
   }
@@ -438,7 +456,7 @@ int launch_gemm_tile(const GemmArgs& a, const GemmPlan& pl, hipStream_t hs) {
 
 // x (rotated already where the layer is) times W^T with the parts' sums in ws (pl.P > 1).
 int gemm_run(const void* wdev, const void* x, void* y, const fb_shape_t* s, const GemmPlan& pl,
-             void* ws, hipStream_t hs) {
+             const void* bias, int bdt, void* ws, hipStream_t hs) {
   GemmArgs a{};
   a.w = static_cast<const uint8_t*>(wdev);
   a.x = x;
@@ -449,6 +467,8 @@ int gemm_run(const void* wdev, const void* x, void* y, const fb_shape_t* s, cons
   a.K = s->K;
   a.GS = (s->K / 128 + 3) / 4;
   a.ydt = s->y_dtype;
+  a.bias = bias;
+  a.bdt = bdt;
   a.vec = (s->N & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0;
   int st;
   if (s->fmt == FB_FMT_GF4)
@@ -458,7 +478,8 @@ int gemm_run(const void* wdev, const void* x, void* y, const fb_shape_t* s, cons
   else
     st = launch_gemm_tile<FB_FMT_E2M1, FB_DT_F16>(a, pl, hs);
   if (st != FB_OK || pl.P == 1) return st;
-  return fb_gpu::sum_parts(a.part, pl.P, (int64_t)s->B * s->N, y, s->y_dtype, a.vec, hs);
+  return fb_gpu::sum_parts(a.part, pl.P, (int64_t)s->B * s->N, y, s->y_dtype, a.vec, bias, bdt,
+                           s->N, hs);
 }
 
 size_t rot_bytes(const fb_shape_t* s) {
@@ -476,12 +497,13 @@ int gemm_check(const fb_shape_t* s) {
 
 }  // namespace
 
-// y[i] = part 0's + part 1's + ... sum i, for n sums (vec: n % 4 == 0 and y 16-byte aligned)
+// y[i] = part 0's + part 1's + ... sum i, plus bias[i % N] where there is one, for n sums (vec:
+// n % 4 == 0, N % 4 == 0 with a bias, and y 16-byte aligned)
 int fb_gpu::sum_parts(const float* part, int P, int64_t n, void* y, int ydt, int vec,
-                      hipStream_t hs) {
+                      const void* bias, int bdt, int N, hipStream_t hs) {
   if ((n + 1023) / 1024 > INT32_MAX) return FB_ERR_SHAPE;
   hipLaunchKernelGGL(gemm_sum, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, hs, part, P, n,
-                     y, ydt, vec);
+                     y, ydt, vec, bias, bdt, N);
   return hipGetLastError() == hipSuccess ? FB_OK : FB_ERR_HIP;
 }
 
@@ -511,11 +533,17 @@ size_t fb_gemm_workspace_bytes(const fb_shape_t* s) {
   return rot_bytes(s) + (pl.P > 1 ? ((size_t)pl.P * s->B * s->N * 4 + 255) & ~size_t(255) : 0);
 }
 
-int fb_gemm(const void* wdev, const void* x, void* y, const fb_shape_t* s, void* ws,
-            size_t ws_bytes, void* stream) {
+int fb_gemm(const void* wdev, const void* x, void* y, const fb_shape_t* s, const void* bias,
+            int32_t bias_dtype, void* ws, size_t ws_bytes, void* stream) {
   if (!s || !wdev || !x || !y) return FB_ERR_NULL;
   const int st = gemm_check(s);
   if (st != FB_OK) return st;
+  if (bias) {
+    if (bias_dtype != FB_DT_F16 && bias_dtype != FB_DT_BF16 && bias_dtype != FB_DT_F32)
+      return FB_ERR_DTYPE;
+    if (reinterpret_cast<uintptr_t>(bias) & (bias_dtype == FB_DT_F32 ? 3u : 1u))
+      return FB_ERR_ALIGN;
+  }
   if ((reinterpret_cast<uintptr_t>(wdev) & 15u) || (reinterpret_cast<uintptr_t>(x) & 15u) ||
       (reinterpret_cast<uintptr_t>(y) & 3u))
     return FB_ERR_ALIGN;
@@ -531,7 +559,7 @@ int fb_gemm(const void* wdev, const void* x, void* y, const fb_shape_t* s, void*
     if (rc != FB_OK) return rc;
     x = ws;
   }
-  return gemm_run(wdev, x, y, s, pl, static_cast<uint8_t*>(ws) + rot, hs);
+  return gemm_run(wdev, x, y, s, pl, bias, bias_dtype, static_cast<uint8_t*>(ws) + rot, hs);
 }
 
 }  // extern "C"

@@ -29,7 +29,8 @@
 namespace fb_gpu {
 __attribute__((visibility("hidden"))) int cu_count();
 __attribute__((visibility("hidden"))) int sum_parts(const float* part, int P, int64_t n, void* y,
-                                                    int ydt, int vec, hipStream_t hs);
+                                                    int ydt, int vec, const void* bias, int bdt,
+                                                    int N, hipStream_t hs);
 }  // namespace fb_gpu
 
 namespace {
@@ -593,7 +594,8 @@ int grad_run(const GradPlan& pl, const fb_shape_t* s, const void* wdev, const vo
     if (st != FB_OK) return st;
   }
   if (pl.P > 1) {
-    const int st = fb_gpu::sum_parts(part, pl.P, (int64_t)s->B * s->K, g.gx, g.dt, g.vec, hs);
+    const int st = fb_gpu::sum_parts(part, pl.P, (int64_t)s->B * s->K, g.gx, g.dt, g.vec,
+                                     nullptr, 0, s->K, hs);
     if (st != FB_OK) return st;
   }
   if (s->fwht_block) {

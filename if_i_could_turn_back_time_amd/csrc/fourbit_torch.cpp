@@ -105,8 +105,14 @@ std::optional<at::Tensor> linear_forward(const at::Tensor& x, const at::Tensor& 
   if (M > kMaxGemvBatch) {
     const size_t need = fb_gemm_workspace_bytes(&s);
     const at::Tensor ws = need ? scratch(need, x) : at::Tensor();
-    check(fb_gemm(wdev.data_ptr(), xk.data_ptr(), y.data_ptr(), &s, ptr_or_null(ws, need), need,
+    // the GEMM adds the bias itself where it is a plain vector
+    const bool fused = bias && bias->dim() == 1 && bias->size(0) == N && bias->is_contiguous() &&
+                       dtype_code(bias->scalar_type()) >= 0;
+    check(fb_gemm(wdev.data_ptr(), xk.data_ptr(), y.data_ptr(), &s,
+                  fused ? bias->data_ptr() : nullptr,
+                  fused ? dtype_code(bias->scalar_type()) : 0, ptr_or_null(ws, need), need,
                   stream));
+    if (fused) return y;
   } else if (fp4_mfma) {
     const size_t need = fb_mx_workspace_bytes(&s);
     if (!need) return std::nullopt;

@@ -174,12 +174,14 @@ int fb_gemv(const void* wdev, const void* x, void* y, const fb_shape_t* s, void*
  * layout and rotation as fb_gemv's; replaces the same reference interface
  * (QuantLinear.forward, layers.py:33-38) where its input has many rows.  fb_gemv is the faster
  * one for B <= 16.  K <= 2^22, B <= 2^24 (FB_ERR_SHAPE).
+ * bias: [N] of bias_dtype (F16, BF16 or F32) on the device, or NULL; added to the fp32 sums
+ * before y's one rounding.
  * ws: device workspace, 256-byte aligned, of at least fb_gemm_workspace_bytes(s) bytes (the
  * rotated x, and the fp32 sums of K-parts for shapes that leave CUs idle otherwise; required
  * where that is not 0: FB_ERR_NULL / FB_ERR_ALIGN / FB_ERR_WORKSPACE).  Its contents need no
  * initialisation; calls that share it must not overlap. */
-int fb_gemm(const void* wdev, const void* x, void* y, const fb_shape_t* s, void* ws,
-            size_t ws_bytes, void* stream);
+int fb_gemm(const void* wdev, const void* x, void* y, const fb_shape_t* s, const void* bias,
+            int32_t bias_dtype, void* ws, size_t ws_bytes, void* stream);
 
 /* Workspace bytes of fb_gemm for this shape on the current device (0: none, or a shape it does
  * not take). */

@@ -85,8 +85,8 @@ def test_gemm_refusals():
     buf = (ctypes.c_uint8 * 512)()
     p = (ctypes.addressof(buf) + 255) // 256 * 256
 
-    def rc(shape, w=p, x=p, y=p, ws=None, nb=0):
-        return L.fb_gemm(w, x, y, ctypes.byref(shape), ws, nb, None)
+    def rc(shape, w=p, x=p, y=p, ws=None, nb=0, bias=None, bdt=0):
+        return L.fb_gemm(w, x, y, ctypes.byref(shape), bias, bdt, ws, nb, None)
 
     big = C.make_shape(64, (1 << 22) + 128, 32)
     assert rc(big) == -2 and L.fb_gemm_workspace_bytes(ctypes.byref(big)) == 0
@@ -99,3 +99,24 @@ def test_gemm_refusals():
     assert rc(ok, w=None) == -1 and rc(ok, x=p + 2) == -7 and rc(ok, y=p + 2) == -7
     assert rc(C.make_shape(64, 4096, 32, C.FMT_E2M1, 4096, C.DT_BF16)) == -5
     assert rc(C.make_shape(64, 100, 32)) == -2
+    plain = C.make_shape(64, 512, 2048)
+    assert rc(plain, bias=p, bdt=3) == -5 and rc(plain, bias=p + 2, bdt=2) == -7
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bdt", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(33, 70, 512), (40, 132, 8192), (520, 1000, 640)])
+def test_gemm_bias(bdt, M, N, K):
+    """The bias joins the fp32 sums, in the tile's epilogue or in the K-parts' sum."""
+    g = torch.Generator().manual_seed(N)
+    pw = PackedWeight.quantize(torch.randn(N, K, generator=g) * 0.02, "gf4", device=DEV)
+    x = torch.randn(M, K, generator=g).half().to(DEV)
+    bias = torch.randn(N, generator=g).to(bdt).to(DEV)
+    for ydt, ulp in ((torch.float32, 2.0 ** -24), (torch.float16, 2.0 ** -11)):
+        shape = C.make_shape(N, K, M, C.FMT_GF4, 0, C.DT_F16, C.DTYPE_CODE[ydt])
+        y = torch.full((M, N), float("nan"), dtype=ydt, device=DEV)
+        C.gemm(pw.wdev, x, y, shape, bias)
+        w = pw.dequant_host().double().to(DEV)
+        ref = x.double() @ w.T + bias.double()
+        bound = (K + 1) * 2.0 ** -24 * (x.double().abs() @ w.abs().T + bias.double().abs())
+        assert bool(((y.double() - ref).abs() <= bound + ulp * (ref.abs() + bound)).all())
