@@ -550,13 +550,13 @@ def jenks2_host(w: torch.Tensor):
 
 def jenks2_gpu(w: torch.Tensor):
     """fb_jenks2_gpu over the flattened fp32 values of a device tensor: (keep bool [n] on
-    the device, split, gvf).  Raises on non-finite values (one torch reduction first)."""
+    the device, split, gvf).  Raises on non-finite values: they make the GVF NaN (the sum of
+    squares and the square of the sum are then both infinite, or NaN), and finite fp32 values
+    cannot, their fp64 sums staying in range."""
     if not w.is_cuda:
         raise RuntimeError("fb_jenks2_gpu needs a device tensor (ROCm GPU)")
     w = w.detach().reshape(-1).to(torch.float32).contiguous()
     n = w.numel()
-    if not bool(torch.isfinite(w).all()):
-        raise RuntimeError(strerror(ERR_VALUE))
     with torch.cuda.device(w.device):
         need = ctypes.c_size_t(0)
         check(lib().fb_jenks2_workspace(n, ctypes.byref(need)))
@@ -568,8 +568,10 @@ def jenks2_gpu(w: torch.Tensor):
         check(lib().fb_jenks2_gpu(_ptr(w), n, _ptr(keep), split_p, split_p + 8,
                                   ws.data_ptr() + off, need.value, _stream(w.device)))
         host = out.cpu()
-    split = int(host[:1].view(torch.int64).item())
-    return keep.bool(), split, float(host[1].item())
+    gvf = float(host[1].item())
+    if gvf != gvf:
+        raise RuntimeError(strerror(ERR_VALUE))
+    return keep.view(torch.bool), int(host[:1].view(torch.int64).item()), gvf
 
 
 JENKS2_FILTER_MAX = 1024  # FB_JENKS2_FILTER_MAX

@@ -31,10 +31,18 @@ namespace {
 constexpr int kBlk = 256;  // elements per block (sequential local sums)
 constexpr int kSup = 256;  // blocks per superblock
 
+// Which of the values equal to the one at the split are kept: those at index >= first.
+struct J2Ties {
+  float t;        // the value at the split's sorted position
+  int before;     // values equal to t at sorted positions before the split
+  int first;
+};
+constexpr int kTieSeg = 16384;  // values one workgroup counts
+
 struct J2Layout {
   int64_t n, nblk, nsup;
   size_t sort_bytes;
-  size_t off_keys_in, off_keys_out, off_vals_in, off_vals_out, off_sort;
+  size_t off_keys, off_sort, off_ties, off_cnt;
   size_t off_t1, off_t2, off_bx1, off_bx2, off_u1, off_u2, off_sx1, off_sx2;
   size_t off_bmin, off_bidx, off_smin, off_sidx, off_ssd0, total;
 };
@@ -46,9 +54,9 @@ int j2_layout(int64_t n, J2Layout& L) {
   L.nblk = (n + kBlk - 1) / kBlk;
   L.nsup = (L.nblk + kSup - 1) / kSup;
   size_t sort_bytes = 0;
-  if (hipcub::DeviceRadixSort::SortPairs(nullptr, sort_bytes, (const float*)nullptr,
-                                         (float*)nullptr, (const int*)nullptr, (int*)nullptr,
-                                         (int)n, 0, 32, (hipStream_t)0) != hipSuccess)
+  if (hipcub::DeviceRadixSort::SortKeys(nullptr, sort_bytes, (const float*)nullptr,
+                                        (float*)nullptr, (int)n, 0, 32,
+                                        (hipStream_t)0) != hipSuccess)
     return FB_ERR_HIP;
   L.sort_bytes = sort_bytes;
   size_t o = 0;
@@ -57,11 +65,10 @@ int j2_layout(int64_t n, J2Layout& L) {
     o = align256(o + bytes);
     return at;
   };
-  L.off_keys_in = take(4 * (size_t)n);
-  L.off_keys_out = take(4 * (size_t)n);
-  L.off_vals_in = take(4 * (size_t)n);
-  L.off_vals_out = take(4 * (size_t)n);
+  L.off_keys = take(4 * (size_t)n);
   L.off_sort = take(sort_bytes);
+  L.off_ties = take(sizeof(J2Ties));
+  L.off_cnt = take(4 * (size_t)((n + kTieSeg - 1) / kTieSeg));
   L.off_t1 = take(8 * (size_t)L.nblk);
   L.off_t2 = take(8 * (size_t)L.nblk);
   L.off_bx1 = take(8 * (size_t)L.nblk);
@@ -77,18 +84,6 @@ int j2_layout(int64_t n, J2Layout& L) {
   L.off_ssd0 = take(8);
   L.total = o;
   return FB_OK;
-}
-
-// keys: the values with -0.0 made +0.0 (so the radix order treats them as equal and the
-// sort keeps their index order); payload: the index.
-__global__ void j2_prep(const float* __restrict__ w, float* __restrict__ keys,
-                        int* __restrict__ vals, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) {
-    const float v = w[i];
-    keys[i] = v == 0.0f ? 0.0f : v;
-    vals[i] = i;
-  }
 }
 
 template <typename T>
@@ -149,42 +144,42 @@ __global__ void j2_block_totals(const T* __restrict__ s, int n, int nblk,
   t2[b] = a2;
 }
 
-// Exclusive block prefixes within each superblock and the superblock totals: one thread per
-// superblock, reading and writing 4 blocks' values at a time.
-__global__ void j2_super(const double* __restrict__ t1, const double* __restrict__ t2, int nblk,
-                         int nsup, double* __restrict__ bx1, double* __restrict__ bx2,
-                         double* __restrict__ u1, double* __restrict__ u2) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= nsup) return;
-  const int b0 = s * kSup, b1 = min(nblk, b0 + kSup);
-  double a1 = 0.0, a2 = 0.0;
-  int b = b0;
-  for (; b + 4 <= b1; b += 4) {
-    double v1[4], v2[4], o1[4], o2[4];
-    *reinterpret_cast<double2*>(v1) = reinterpret_cast<const double2*>(t1 + b)[0];
-    *reinterpret_cast<double2*>(v1 + 2) = reinterpret_cast<const double2*>(t1 + b)[1];
-    *reinterpret_cast<double2*>(v2) = reinterpret_cast<const double2*>(t2 + b)[0];
-    *reinterpret_cast<double2*>(v2 + 2) = reinterpret_cast<const double2*>(t2 + b)[1];
+// Exclusive block prefixes within each superblock and the superblock totals: one wave per
+// superblock.  Lane 0 sums d's block totals and lane 1 q's, in order, from LDS (one thread per
+// superblock reading them from memory took 29 us for 256 superblocks: every addition waited
+// for a load).
+__global__ __launch_bounds__(64) void j2_super(const double* __restrict__ t1,
+                                               const double* __restrict__ t2, int nblk,
+                                               double* __restrict__ bx1, double* __restrict__ bx2,
+                                               double* __restrict__ u1, double* __restrict__ u2) {
+  __shared__ double l[2][kSup + 2];  // + 2: the two lanes in different banks
+  const int s = blockIdx.x;
+  const int b0 = s * kSup, m = min(nblk - b0, kSup);
+  for (int i = threadIdx.x; i < kSup; i += 64) {
+    l[0][i] = i < m ? t1[b0 + i] : 0.0;
+    l[1][i] = i < m ? t2[b0 + i] : 0.0;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    double* const v = l[threadIdx.x];
+    double a = 0.0;
+    for (int i = 0; i < kSup; i += 16) {  // totals past m are 0 and leave a as it is
+      double x[16];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      o1[e] = a1;
-      o2[e] = a2;
-      a1 = a1 + v1[e];
-      a2 = a2 + v2[e];
+      for (int e = 0; e < 16; ++e) x[e] = v[i + e];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        v[i + e] = a;
+        a = i + e < m ? a + x[e] : a;
+      }
     }
-    reinterpret_cast<double2*>(bx1 + b)[0] = *reinterpret_cast<double2*>(o1);
-    reinterpret_cast<double2*>(bx1 + b)[1] = *reinterpret_cast<double2*>(o1 + 2);
-    reinterpret_cast<double2*>(bx2 + b)[0] = *reinterpret_cast<double2*>(o2);
-    reinterpret_cast<double2*>(bx2 + b)[1] = *reinterpret_cast<double2*>(o2 + 2);
+    (threadIdx.x ? u2 : u1)[s] = a;
   }
-  for (; b < b1; ++b) {
-    bx1[b] = a1;
-    bx2[b] = a2;
-    a1 = a1 + t1[b];
-    a2 = a2 + t2[b];
+  __syncthreads();
+  for (int i = threadIdx.x; i < m; i += 64) {
+    bx1[b0 + i] = l[0][i];
+    bx2[b0 + i] = l[1][i];
   }
-  u1[s] = a1;
-  u2[s] = a2;
 }
 
 // Exclusive superblock prefixes; sx[nsup] is the total.  The workgroup stages the superblock
@@ -332,21 +327,94 @@ __global__ __launch_bounds__(kFinalThreads) void j2_final(const double* __restri
   }
 }
 
-// keep[i] = 1 when w[i] sits at a sorted position >= split.  With t the value at position
-// split: every value above t is kept and every value below is not; values equal to t sit in
-// index order (the sort is stable), so of those the ones at index >= order[split] are kept.
-// A streaming pass over w, not a scatter through the permutation.  (-0.0 == +0.0 as floats,
-// as in the sort's keys.)
-__global__ void j2_mask(const float* __restrict__ w, const float* __restrict__ skeys,
-                        const int* __restrict__ order, int n, const int64_t* __restrict__ split,
-                        uint8_t* __restrict__ keep) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+// keep[i] = 1 when w[i] sits at a position >= split of the stable ascending sort.  With t the
+// value at that position: every value above t is kept and every value below is not; values
+// equal to t (-0.0 == +0.0) sit in index order, so of those all but the first `before` are.  So
+// the sort needs no indices: keys alone, and where the split falls inside a run of equal values
+// (rare) a count finds the index of the first one kept.
+__global__ void j2_ties(const float* __restrict__ skeys, const int64_t* __restrict__ split,
+                        J2Ties* __restrict__ out) {
   const int64_t sp = *split;
   const float t = skeys[sp];
-  const int it = order[sp];
-  const float v = w[i];
-  keep[i] = (v > t || (v == t && i >= it)) ? 1 : 0;
+  int64_t lo = sp;
+  if (sp > 0 && !(skeys[sp - 1] < t)) {  // first position not below t
+    lo = 0;
+    int64_t hi = sp - 1;
+    while (lo < hi) {
+      const int64_t mid = (lo + hi) >> 1;
+      if (skeys[mid] < t)
+        lo = mid + 1;
+      else
+        hi = mid;
+    }
+  }
+  out->t = t;
+  out->before = (int)(sp - lo);
+  out->first = 0;
+}
+
+// How many values of each segment equal t (only where the split is inside a run of them).
+__global__ __launch_bounds__(256) void j2_tie_count(const float* __restrict__ w, int n,
+                                                    const J2Ties* __restrict__ ties,
+                                                    int* __restrict__ cnt) {
+  if (ties->before == 0) return;
+  __shared__ int part[4];
+  const float t = ties->t;
+  const int64_t i0 = (int64_t)blockIdx.x * kTieSeg;
+  const int64_t i1 = i0 + kTieSeg < n ? i0 + kTieSeg : n;
+  int c = 0;
+  for (int64_t i = i0 + threadIdx.x; i < i1; i += 256) c += w[i] == t ? 1 : 0;
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) c += __shfl_xor(c, m, 64);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = c;
+  __syncthreads();
+  if (threadIdx.x == 0) cnt[blockIdx.x] = part[0] + part[1] + part[2] + part[3];
+}
+
+// The index of the value equal to t that has `before` others ahead of it: one wave walks the
+// segments' counts, then the segment.
+__global__ __launch_bounds__(64) void j2_tie_find(const float* __restrict__ w, int n, int nseg,
+                                                  const int* __restrict__ cnt,
+                                                  J2Ties* __restrict__ ties) {
+  int left = ties->before;
+  if (left == 0) return;
+  const float t = ties->t;
+  int seg = 0;
+  for (; seg < nseg - 1; ++seg) {
+    const int c = cnt[seg];
+    if (left < c) break;
+    left -= c;
+  }
+  const int64_t i0 = (int64_t)seg * kTieSeg;
+  const int64_t i1 = i0 + kTieSeg < n ? i0 + kTieSeg : n;
+  for (int64_t i = i0; i < i1; i += 64) {
+    const int64_t at = i + threadIdx.x;
+    const uint64_t b = __ballot(at < i1 && w[at] == t);
+    const int c = __popcll(b);
+    if (left < c) {
+      const uint64_t below = threadIdx.x == 0 ? 0ull : (~0ull >> (64 - threadIdx.x));
+      if ((b >> threadIdx.x & 1) && __popcll(b & below) == left) ties->first = (int)at;
+      return;
+    }
+    left -= c;
+  }
+}
+
+// The streaming pass over w that writes the mask, 4 values a thread where w and keep allow it.
+__global__ void j2_mask(const float* __restrict__ w, int n, const J2Ties* __restrict__ ties,
+                        uint8_t* __restrict__ keep, int vec) {
+  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+  if (i >= n) return;
+  const float t = ties->t;
+  const int it = ties->first;
+  auto kept = [&](float v, int64_t at) -> unsigned { return v > t || (v == t && at >= it); };
+  if (vec && i + 4 <= n) {
+    const float4 v = *reinterpret_cast<const float4*>(w + i);
+    *reinterpret_cast<unsigned*>(keep + i) = kept(v.x, i) | (kept(v.y, i + 1) << 8) |
+                                             (kept(v.z, i + 2) << 16) | (kept(v.w, i + 3) << 24);
+  } else {
+    for (int64_t j = i; j < n && j < i + 4; ++j) keep[j] = (uint8_t)kept(w[j], j);
+  }
 }
 
 int grid_of(int64_t items, int threads) { return (int)((items + threads - 1) / threads); }
@@ -666,9 +734,8 @@ int ssd_gpu(const T* srt, int64_t n, T* out, void* ws, hipStream_t hs) {
   const int ni = (int)n, nblk = (int)L.nblk, nsup = (int)L.nsup;
   hipLaunchKernelGGL(j2_block_totals<T>, dim3(grid_of(nblk, 64)), dim3(64), 0, hs, srt, ni, nblk,
                      at(L.off_t1), at(L.off_t2));
-  hipLaunchKernelGGL(j2_super, dim3(grid_of(nsup, 64)), dim3(64), 0, hs, at(L.off_t1),
-                     at(L.off_t2), nblk, nsup, at(L.off_bx1), at(L.off_bx2), at(L.off_u1),
-                     at(L.off_u2));
+  hipLaunchKernelGGL(j2_super, dim3(nsup), dim3(64), 0, hs, at(L.off_t1), at(L.off_t2), nblk,
+                     at(L.off_bx1), at(L.off_bx2), at(L.off_u1), at(L.off_u2));
   hipLaunchKernelGGL(j2_top, dim3(1), dim3(kTopThreads), 0, hs, at(L.off_u1), at(L.off_u2), nsup,
                      at(L.off_sx1), at(L.off_sx2));
   hipLaunchKernelGGL(j2_ssd<T>, dim3(grid_of(nblk, 64)), dim3(64), 0, hs, srt, ni, nblk, nsup,
@@ -803,10 +870,9 @@ int fb_jenks2_gpu(const float* w, int64_t n, uint8_t* keep, int64_t* split, doub
   hipStream_t hs = static_cast<hipStream_t>(stream);
   uint8_t* base = static_cast<uint8_t*>(ws);
   auto at = [&](size_t off) { return static_cast<void*>(base + off); };
-  float* keys_in = static_cast<float*>(at(L.off_keys_in));
-  float* keys_out = static_cast<float*>(at(L.off_keys_out));
-  int* vals_in = static_cast<int*>(at(L.off_vals_in));
-  int* vals_out = static_cast<int*>(at(L.off_vals_out));
+  float* keys = static_cast<float*>(at(L.off_keys));
+  J2Ties* ties = static_cast<J2Ties*>(at(L.off_ties));
+  int* cnt = static_cast<int*>(at(L.off_cnt));
   double *t1 = static_cast<double*>(at(L.off_t1)), *t2 = static_cast<double*>(at(L.off_t2));
   double *bx1 = static_cast<double*>(at(L.off_bx1)), *bx2 = static_cast<double*>(at(L.off_bx2));
   double *u1 = static_cast<double*>(at(L.off_u1)), *u2 = static_cast<double*>(at(L.off_u2));
@@ -817,24 +883,26 @@ int fb_jenks2_gpu(const float* w, int64_t n, uint8_t* keep, int64_t* split, doub
   int* sidx = static_cast<int*>(at(L.off_sidx));
   double* ssd0 = static_cast<double*>(at(L.off_ssd0));
   const int ni = (int)n, nblk = (int)L.nblk, nsup = (int)L.nsup;
-  hipLaunchKernelGGL(j2_prep, dim3(grid_of(n, 256)), dim3(256), 0, hs, w, keys_in, vals_in, ni);
   size_t sb = L.sort_bytes;
-  if (hipcub::DeviceRadixSort::SortPairs(at(L.off_sort), sb, keys_in, keys_out, vals_in, vals_out,
-                                         ni, 0, 32, hs) != hipSuccess)
+  if (hipcub::DeviceRadixSort::SortKeys(at(L.off_sort), sb, w, keys, ni, 0, 32, hs) != hipSuccess)
     return FB_ERR_HIP;
-  hipLaunchKernelGGL(j2_block_totals<float>, dim3(grid_of(nblk, 64)), dim3(64), 0, hs, keys_out, ni,
+  hipLaunchKernelGGL(j2_block_totals<float>, dim3(grid_of(nblk, 64)), dim3(64), 0, hs, keys, ni,
                      nblk, t1, t2);
-  hipLaunchKernelGGL(j2_super, dim3(grid_of(nsup, 64)), dim3(64), 0, hs, t1, t2, nblk, nsup, bx1,
-                     bx2, u1, u2);
+  hipLaunchKernelGGL(j2_super, dim3(nsup), dim3(64), 0, hs, t1, t2, nblk, bx1, bx2, u1, u2);
   hipLaunchKernelGGL(j2_top, dim3(1), dim3(kTopThreads), 0, hs, u1, u2, nsup, sx1, sx2);
-  hipLaunchKernelGGL(j2_ssd<float>, dim3(grid_of(nblk, 64)), dim3(64), 0, hs, keys_out, ni, nblk,
+  hipLaunchKernelGGL(j2_ssd<float>, dim3(grid_of(nblk, 64)), dim3(64), 0, hs, keys, ni, nblk,
                      nsup, bx1, bx2, sx1, sx2, bmin, bidx, ssd0, (float*)nullptr);
   hipLaunchKernelGGL(j2_min_super, dim3(nsup), dim3(64), 0, hs, bmin, bidx, nblk, nsup, smin,
                      sidx);
   hipLaunchKernelGGL(j2_final, dim3(1), dim3(kFinalThreads), 0, hs, smin, sidx, nsup, ssd0, split,
                      gvf);
-  hipLaunchKernelGGL(j2_mask, dim3(grid_of(n, 256)), dim3(256), 0, hs, w, keys_out, vals_out, ni,
-                     split, keep);
+  hipLaunchKernelGGL(j2_ties, dim3(1), dim3(1), 0, hs, keys, split, ties);
+  const int nseg = grid_of(n, kTieSeg);
+  hipLaunchKernelGGL(j2_tie_count, dim3(nseg), dim3(256), 0, hs, w, ni, ties, cnt);
+  hipLaunchKernelGGL(j2_tie_find, dim3(1), dim3(64), 0, hs, w, ni, nseg, cnt, ties);
+  const int vec = (reinterpret_cast<uintptr_t>(w) & 15u) == 0 &&
+                  (reinterpret_cast<uintptr_t>(keep) & 3u) == 0;
+  hipLaunchKernelGGL(j2_mask, dim3(grid_of(n, 1024)), dim3(256), 0, hs, w, ni, ties, keep, vec);
   return hipGetLastError() == hipSuccess ? FB_OK : FB_ERR_HIP;
 }
 
