@@ -334,6 +334,16 @@ __global__ __launch_bounds__(256) void gemm_sum(const float* __restrict__ part, 
   }
 }
 
+// y[m, n] += bias[n] for the GEMV's 1 to 16 rows, rounded as torch's y.add_(bias.to(y.dtype)):
+// the bias to y's dtype, then the sum.
+template <typename T>
+__global__ __launch_bounds__(256) void add_bias_kernel(T* __restrict__ y, int64_t n, int N,
+                                                       const void* __restrict__ bias, int bdt) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  y[i] = (T)((float)y[i] + (float)(T)load_as_float(bias, i % N, bdt));
+}
+
 // x [M, K] of one dtype -> [M, ld] of another (round to nearest even), zeros past K: the
 // conversion and the padding to whole groups in one pass.  8 outputs per thread.
 __global__ __launch_bounds__(256) void cast_rows_kernel(const void* __restrict__ x, int xdt,
@@ -508,6 +518,33 @@ int fb_gpu::sum_parts(const float* part, int P, int64_t n, void* y, int ydt, int
 }
 
 extern "C" {
+
+int fb_add_bias(void* y, int32_t y_dtype, int32_t M, int32_t N, const void* bias,
+                int32_t bias_dtype, void* stream) {
+  if (!y || !bias) return FB_ERR_NULL;
+  if (M < 1 || N < 1) return FB_ERR_SHAPE;
+  if (bias_dtype != FB_DT_F16 && bias_dtype != FB_DT_BF16 && bias_dtype != FB_DT_F32)
+    return FB_ERR_DTYPE;
+  if ((reinterpret_cast<uintptr_t>(bias) & (bias_dtype == FB_DT_F32 ? 3u : 1u)) ||
+      (reinterpret_cast<uintptr_t>(y) & (y_dtype == FB_DT_F32 ? 3u : 1u)))
+    return FB_ERR_ALIGN;
+  const int64_t n = (int64_t)M * N;
+  if ((n + 255) / 256 > INT32_MAX) return FB_ERR_SHAPE;
+  const dim3 grid((unsigned)((n + 255) / 256)), block(256);
+  hipStream_t hs = static_cast<hipStream_t>(stream);
+  if (y_dtype == FB_DT_F32)
+    hipLaunchKernelGGL(add_bias_kernel<float>, grid, block, 0, hs, static_cast<float*>(y), n, N,
+                       bias, bias_dtype);
+  else if (y_dtype == FB_DT_F16)
+    hipLaunchKernelGGL(add_bias_kernel<_Float16>, grid, block, 0, hs, static_cast<_Float16*>(y), n,
+                       N, bias, bias_dtype);
+  else if (y_dtype == FB_DT_BF16)
+    hipLaunchKernelGGL(add_bias_kernel<__bf16>, grid, block, 0, hs, static_cast<__bf16*>(y), n, N,
+                       bias, bias_dtype);
+  else
+    return FB_ERR_DTYPE;
+  return hipGetLastError() == hipSuccess ? FB_OK : FB_ERR_HIP;
+}
 
 int fb_cast_rows(const void* x, int32_t x_dtype, int32_t M, int32_t K, void* out,
                  int32_t out_dtype, int32_t ld, void* stream) {

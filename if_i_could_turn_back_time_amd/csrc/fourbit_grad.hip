@@ -393,6 +393,29 @@ __global__ __launch_bounds__(256) void grad_rotate_kernel(const float* __restric
     if (256 * e + t < kw) store_y(out, row * K + k0 + 256 * e + t, x[e] * sc, dt);
 }
 
+// gb[n] = sum over m of gy[m, n], fp32 sums in a fixed order: a workgroup's 16 waves take every
+// 16th row of 64 columns, then one wave adds the 16 sums in order.  gy was just read or is about
+// to be, so it comes from the caches; bound by the latency of M / 16 dependent rows.
+__global__ __launch_bounds__(1024) void grad_bias_kernel(const void* __restrict__ gy, int M, int N,
+                                                         int dt, void* __restrict__ gb, int odt) {
+  __shared__ float l[16][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int n = blockIdx.x * 64 + lane;
+  float a = 0.f;
+  if (n < N) {
+#pragma unroll 8
+    for (int m = wave; m < M; m += 16) a += load_as_float(gy, (int64_t)m * N + n, dt);
+  }
+  l[wave][lane] = a;
+  __syncthreads();
+  if (wave == 0 && n < N) {
+    float s = l[0][lane];
+#pragma unroll
+    for (int w = 1; w < 16; ++w) s += l[w][lane];
+    store_y(gb, n, s, odt);
+  }
+}
+
 // ---------------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------------
@@ -612,6 +635,20 @@ int grad_run(const GradPlan& pl, const fb_shape_t* s, const void* wdev, const vo
 }  // namespace
 
 extern "C" {
+
+int fb_grad_bias(const void* gy, int32_t gy_dtype, int32_t M, int32_t N, void* gb,
+                 int32_t gb_dtype, void* stream) {
+  if (!gy || !gb) return FB_ERR_NULL;
+  if (M < 1 || N < 1) return FB_ERR_SHAPE;
+  for (int32_t d : {gy_dtype, gb_dtype})
+    if (d != FB_DT_F16 && d != FB_DT_BF16 && d != FB_DT_F32) return FB_ERR_DTYPE;
+  if ((reinterpret_cast<uintptr_t>(gy) & (gy_dtype == FB_DT_F32 ? 3u : 1u)) ||
+      (reinterpret_cast<uintptr_t>(gb) & (gb_dtype == FB_DT_F32 ? 3u : 1u)))
+    return FB_ERR_ALIGN;
+  hipLaunchKernelGGL(grad_bias_kernel, dim3((N + 63) / 64), dim3(1024), 0,
+                     static_cast<hipStream_t>(stream), gy, M, N, gy_dtype, gb, gb_dtype);
+  return hipGetLastError() == hipSuccess ? FB_OK : FB_ERR_HIP;
+}
 
 size_t fb_grad_x_workspace_bytes(const fb_shape_t* s, int32_t f16_exact) {
   GradPlan pl;

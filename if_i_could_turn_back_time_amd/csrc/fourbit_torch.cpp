@@ -99,20 +99,20 @@ std::optional<at::Tensor> linear_forward(const at::Tensor& x, const at::Tensor& 
                        (int32_t)kp, stream));
   }
   if (reinterpret_cast<uintptr_t>(xk.data_ptr()) & 15u) return std::nullopt;
+  // a bias that is a plain vector is added by the GEMM, or by one small kernel
+  const bool vector_bias = bias && bias->dim() == 1 && bias->size(0) == N &&
+                           bias->is_contiguous() && dtype_code(bias->scalar_type()) >= 0;
+  const int bdt = vector_bias ? dtype_code(bias->scalar_type()) : 0;
   auto sizes = x.sizes().vec();
   sizes.back() = N;
   at::Tensor y = at::empty(sizes, x.options());
   if (M > kMaxGemvBatch) {
     const size_t need = fb_gemm_workspace_bytes(&s);
     const at::Tensor ws = need ? scratch(need, x) : at::Tensor();
-    // the GEMM adds the bias itself where it is a plain vector
-    const bool fused = bias && bias->dim() == 1 && bias->size(0) == N && bias->is_contiguous() &&
-                       dtype_code(bias->scalar_type()) >= 0;
     check(fb_gemm(wdev.data_ptr(), xk.data_ptr(), y.data_ptr(), &s,
-                  fused ? bias->data_ptr() : nullptr,
-                  fused ? dtype_code(bias->scalar_type()) : 0, ptr_or_null(ws, need), need,
+                  vector_bias ? bias->data_ptr() : nullptr, bdt, ptr_or_null(ws, need), need,
                   stream));
-    if (fused) return y;
+    if (vector_bias) return y;
   } else if (fp4_mfma) {
     const size_t need = fb_mx_workspace_bytes(&s);
     if (!need) return std::nullopt;
@@ -125,7 +125,10 @@ std::optional<at::Tensor> linear_forward(const at::Tensor& x, const at::Tensor& 
     check(fb_gemv(wdev.data_ptr(), xk.data_ptr(), y.data_ptr(), &s, ptr_or_null(ws, need), need,
                   stream));
   }
-  if (bias) y.add_(bias->scalar_type() == y.scalar_type() ? *bias : bias->to(y.scalar_type()));
+  if (vector_bias)
+    check(fb_add_bias(y.data_ptr(), xdt, (int32_t)M, (int32_t)N, bias->data_ptr(), bdt, stream));
+  else if (bias)
+    y.add_(bias->scalar_type() == y.scalar_type() ? *bias : bias->to(y.scalar_type()));
   return y;
 }
 
@@ -158,9 +161,24 @@ std::optional<at::Tensor> linear_grad_x(const at::Tensor& gy, const at::Tensor& 
   return kp == K ? gx : gx.narrow(1, 0, K).contiguous();
 }
 
+// The bias gradient: gy's column sums in bdtype; None where the caller has to decide.
+std::optional<at::Tensor> linear_grad_bias(const at::Tensor& gy, at::ScalarType bt) {
+  const int gdt = dtype_code(gy.scalar_type()), bdt = dtype_code(bt);
+  if (watched() || !plain(gy) || gy.dim() != 2 || gdt < 0 || bdt < 0 || gy.numel() == 0 ||
+      gy.size(0) > INT32_MAX || gy.size(1) > INT32_MAX)
+    return std::nullopt;
+  c10::DeviceGuard guard(gy.device());
+  const at::Tensor g = gy.contiguous();
+  at::Tensor gb = at::empty({gy.size(1)}, gy.options().dtype(bt));
+  check(fb_grad_bias(g.data_ptr(), gdt, (int32_t)gy.size(0), (int32_t)gy.size(1), gb.data_ptr(),
+                     bdt, stream_of(gy)));
+  return gb;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_fourbit_torch, m) {
   m.def("linear_forward", &linear_forward);
   m.def("linear_grad_x", &linear_grad_x);
+  m.def("linear_grad_bias", &linear_grad_bias);
 }

@@ -210,10 +210,15 @@ class _PackedLinearFn(torch.autograd.Function):
     def backward(ctx, gy):
         (wdev,) = ctx.saved_tensors
         N, K, fmt, fwht_block, xdt, f16_exact, bdt = ctx.cfg
-        gb = gy.sum(0).to(bdt) if ctx.needs_input_grad[1] else None
-        gx = None
+        native = not torch.is_grad_enabled() and type(gy) is torch.Tensor
+        gb = gx = None
+        if ctx.needs_input_grad[1]:
+            if native:
+                gb = C.native().linear_grad_bias(gy, bdt)
+            if gb is None:
+                gb = gy.sum(0).to(bdt)
         if ctx.needs_input_grad[0]:
-            if not torch.is_grad_enabled() and N <= MAX_GRAD_N and type(gy) is torch.Tensor:
+            if native and N <= MAX_GRAD_N:
                 gx = C.native().linear_grad_x(gy, wdev, N, K, C.FMT_BY_NAME[fmt], fwht_block,
                                               f16_exact,
                                               xdt if xdt in C.DTYPE_CODE else torch.float32)

@@ -187,6 +187,11 @@ int fb_gemm(const void* wdev, const void* x, void* y, const fb_shape_t* s, const
  * not take). */
 size_t fb_gemm_workspace_bytes(const fb_shape_t* s);
 
+/* y [M, N] += bias [N], in place, the bias rounded to y's dtype first (fb_gemv's rows; fb_gemm
+ * takes the bias itself).  Device pointers; asynchronous on the stream. */
+int fb_add_bias(void* y, int32_t y_dtype, int32_t M, int32_t N, const void* bias,
+                int32_t bias_dtype, void* stream);
+
 /* Activations into the kernels' form: x [M, K] (F16, BF16 or F32) as out [M, ld] of F16 or BF16,
  * rounded to nearest even, zeros from K to ld (a multiple of 128, >= K).  Device pointers, out
  * 16-byte aligned; asynchronous on the stream. */
@@ -271,6 +276,11 @@ size_t fb_mx_presplit_workspace_bytes(const fb_shape_t* s);
  * N <= 2^22, B <= 2^24 (FB_ERR_SHAPE). */
 int fb_grad_x(const void* wdev, const void* gy, void* gx, const fb_shape_t* s, int32_t gx_dtype,
               int32_t f16_exact, void* ws, size_t ws_bytes, void* stream);
+
+/* The bias gradient gb[N] (of gb_dtype) = the column sums of gy [M, N] (gy_dtype), summed in fp32
+ * in a fixed order.  Device pointers; asynchronous on the stream. */
+int fb_grad_bias(const void* gy, int32_t gy_dtype, int32_t M, int32_t N, void* gb,
+                 int32_t gb_dtype, void* stream);
 
 /* Workspace bytes of fb_grad_x for this shape on the current device (0: a shape it does not
  * take). */

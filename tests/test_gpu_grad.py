@@ -123,3 +123,31 @@ def test_layer_gradient_and_its_gradient(kw):
         assert a.is_contiguous() and torch.allclose(a, b, rtol=1e-5, atol=1e-5)
         (c,) = torch.autograd.grad(b.sum(), g2)
         assert c.shape == gy.shape and bool(torch.isfinite(c).all())
+
+
+@pytest.mark.parametrize("gdt", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N", [(1, 1), (15, 63), (16, 64), (17, 65), (333, 1000), (2100, 130)])
+def test_grad_bias(gdt, M, N):
+    """Column sums in fp32 (at most M / 16 + 16 roundings each), and the layer's bias gradient."""
+    g = torch.Generator().manual_seed(M)
+    gy = torch.randn(M, N, generator=g).to(gdt).to(DEV)
+    gb = C.native().linear_grad_bias(gy, torch.float32)
+    ref = gy.double().sum(0)
+    bound = (M / 16 + 17) * 2.0 ** -24 * gy.double().abs().sum(0)
+    assert bool(((gb.double() - ref).abs() <= bound + 1e-40).all())
+    q = QuantLinear(torch.nn.Linear(128, N), fmt="gf4").to(DEV)
+    x = torch.randn(M, 128, device=DEV, dtype=gdt, requires_grad=True)
+    gx, gq = torch.autograd.grad(q(x), (x, q.bias), gy)
+    assert gq.dtype == q.bias.dtype and torch.equal(gq, gb)
+
+
+@pytest.mark.parametrize("ydt", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N", [(1, 300), (3, 77), (16, 4096)])
+def test_gemv_bias_is_the_in_place_add(ydt, M, N):
+    """The native path's bias of 1 to 16 rows rounds as y.add_(bias.to(y.dtype))."""
+    q = QuantLinear(torch.nn.Linear(256, N), fmt="gf4").to(DEV)
+    x = torch.randn(M, 256, device=DEV, dtype=ydt)
+    with torch.no_grad():
+        y = q(x)
+        b, q.bias = q.bias, None
+        assert torch.equal(y, q(x).add_(b.to(ydt)))
