@@ -80,6 +80,10 @@ __global__ __launch_bounds__(kGemmWaves * 64, 2) void gemm_kernel(GemmArgs a) {
   using T = GemmTile<RT, CT>;
   constexpr int BB = FMT == FB_FMT_GF4 ? fb::kGf4BlockBytes : fb::kE2m1BlockBytes;
   constexpr int NB = T::kBufs, D = NB - 1;
+  // The barrier in the middle of the chunk before, where a chunk is long enough for the shorter
+  // time that leaves its requests: 1 to 6% over 13 shapes with CT = 3 and 4 (8192 -> 28672, M = 64,
+  // GF4: 55.1 -> 52.2 us), 0 to 3% slower with CT = 2.
+  constexpr bool kEarly = NB == 4 && CT >= 3;
   constexpr int XD = T::kBuf / (kGemmWaves * 1024);  // 1 KiB x requests of one wave per chunk
   __shared__ __align__(1024) uint8_t xb0[T::kBuf], xb1[T::kBuf];
   __shared__ __align__(1024) uint8_t xb2[NB == 4 ? T::kBuf : 16], xb3[NB == 4 ? T::kBuf : 16];
@@ -195,21 +199,26 @@ __global__ __launch_bounds__(kGemmWaves * 64, 2) void gemm_kernel(GemmArgs a) {
     }
   };
   u32x4 A[2][RT];  // this k-step's operands and the next one's
-  // One chunk: 4 k-steps of RT x CT MFMAs.  B operands are read two column tiles ahead.
-  auto compute = [&](const uint8_t* buf, const u32x4 (&nb)[RT], const u32x4 (&nbn)[RT], int c) {
-    u32x4 B[3];
-    auto readb = [&](int i) {
-      return *reinterpret_cast<const u32x4*>(buf + (rbase ^ ((i / CT) * 16)) +
-                                             (i % CT) * 16 * kRowBytes);
-    };
-    B[0] = readb(0);
-    B[1] = readb(1);
+  // k-steps [s0, s1) of a chunk: RT x CT MFMAs each, B operands read kAhead column tiles ahead
+  // (with four chunks staged, from the next chunk too).
+  constexpr int kAhead = kEarly ? 3 : 2, kRing = kAhead + 1;
+  u32x4 B[kRing];
+  auto readb = [&](const uint8_t* buf, int i) {
+    return *reinterpret_cast<const u32x4*>(buf + (rbase ^ ((i / CT) * 16)) +
+                                           (i % CT) * 16 * kRowBytes);
+  };
+  auto compute = [&](const uint8_t* buf, const uint8_t* bufn, const u32x4 (&nb)[RT],
+                     const u32x4 (&nbn)[RT], int c, int s0, int s1) {
+    const int ring0 = kEarly ? c * 4 * CT : 0;  // 16 CT is a multiple of the early ring's 4
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
+    for (int s = s0; s < s1; ++s) {
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) {
-        const int i = s * CT + ct;
-        if (i + 2 < 4 * CT) B[(i + 2) % 3] = readb(i + 2);
+        const int i = s * CT + ct, ia = i + kAhead;
+        if (ia < 4 * CT)
+          B[(ring0 + ia) % kRing] = readb(buf, ia);
+        else if (kEarly)
+          B[(ring0 + ia) % kRing] = readb(bufn, ia - 4 * CT);
         // this step's share of the next k-step's 2 RT half decodes
 #pragma unroll
         for (int q = ct * 2 * RT / CT; q < (ct + 1) * 2 * RT / CT; ++q) {
@@ -222,7 +231,8 @@ __global__ __launch_bounds__(kGemmWaves * 64, 2) void gemm_kernel(GemmArgs a) {
             decode_half(A[0][r], nbn[r], tbn[r], 0, 0, h);
         }
 #pragma unroll
-        for (int r = 0; r < RT; ++r) acc[r][ct] = mfma<XDT>(A[s & 1][r], B[i % 3], acc[r][ct]);
+        for (int r = 0; r < RT; ++r)
+          acc[r][ct] = mfma<XDT>(A[s & 1][r], B[(ring0 + i) % kRing], acc[r][ct]);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -241,21 +251,41 @@ __global__ __launch_bounds__(kGemmWaves * 64, 2) void gemm_kernel(GemmArgs a) {
       decode_half(A[0][r], nib[0][r], tb[r], 0, 0, 0);
       decode_half(A[0][r], nib[0][r], tb[r], 0, 0, 1);
     }
+    if constexpr (kEarly) {  // the first chunk: D - 1 chunks' requests are younger
+      wait_barrier<(D - 1) * (XD + RT)>();
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) B[i] = readb(bufs[0], i);
+    }
     for (int sp = sp0; sp < sp1; ++sp) {
       const int spn = min(sp + 1, sp1 - 1);
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        // The x of chunk c was requested D chunks ago; each of the D - 1 chunks since then
-        // requested XD pieces of x and RT nibble chunks (and sometimes tables), so at most that
-        // many younger requests in flight means it has arrived.  Past the barrier every
-        // wave's part of it has, and every wave has read the chunk before.
-        wait_barrier<(D - 1) * (XD + RT)>();
         const int cn = (c + D) & 3;
         const int spx = c + D >= 4 ? spn : sp;
+        // Every chunk requests XD pieces of x and RT nibble chunks (and sometimes tables), so at
+        // most k chunks' worth of requests in flight means that all older ones have arrived.
+        // Past the barrier every wave's part of them has.
+        if constexpr (kEarly) {
+          // In the middle of chunk c: the next one must be there (the one after it is still on
+          // its way), and every wave is done with the one before, whose place the request
+          // takes.  So B operands can be read ahead across the chunk's end.
+          compute(bufs[c], bufs[(c + 1) & 3], nib[c], nib[(c + 1) & 3], c, 0, 2);
+          wait_barrier<XD + RT>();
+        } else {
+          // chunk c is there (D - 1 younger ones may not be), and every wave is done with the
+          // one before
+          wait_barrier<(D - 1) * (XD + RT)>();
+        }
         load_nib(spx, cn, nib[cn % NB]);
         if (cn == 0) load_tab(spx, tbn);
         stage(spx, cn, bufs[cn]);
-        compute(bufs[c], nib[c % NB], nib[(c + 1) % NB], c);
+        if constexpr (kEarly) {
+          compute(bufs[c], bufs[(c + 1) & 3], nib[c], nib[(c + 1) & 3], c, 2, 4);
+        } else {
+#pragma unroll
+          for (int i = 0; i < kAhead; ++i) B[i] = readb(bufs[c], i);
+          compute(bufs[c], nullptr, nib[c % NB], nib[(c + 1) % NB], c, 0, 4);
+        }
       }
 #pragma unroll
       for (int r = 0; r < RT; ++r) {
