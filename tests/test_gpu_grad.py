@@ -128,12 +128,12 @@ def test_layer_gradient_and_its_gradient(kw):
 @pytest.mark.parametrize("gdt", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,N", [(1, 1), (15, 63), (16, 64), (17, 65), (333, 1000), (2100, 130)])
 def test_grad_bias(gdt, M, N):
-    """Column sums in fp32 (at most M / 16 + 16 roundings each), and the layer's bias gradient."""
+    """Column sums in fp32 (at most M / 64 + 64 roundings each), and the layer's bias gradient."""
     g = torch.Generator().manual_seed(M)
     gy = torch.randn(M, N, generator=g).to(gdt).to(DEV)
     gb = C.native().linear_grad_bias(gy, torch.float32)
     ref = gy.double().sum(0)
-    bound = (M / 16 + 17) * 2.0 ** -24 * gy.double().abs().sum(0)
+    bound = (M / 64 + 65) * 2.0 ** -24 * gy.double().abs().sum(0)
     assert bool(((gb.double() - ref).abs() <= bound + 1e-40).all())
     q = QuantLinear(torch.nn.Linear(128, N), fmt="gf4").to(DEV)
     x = torch.randn(M, 128, device=DEV, dtype=gdt, requires_grad=True)
