@@ -597,9 +597,17 @@ class QuantLinear(nn.Linear):
         if self.fp4_mfma and (self.fmt != "e2m1" or self.fwht_block):
             self.fp4_mfma = False  # the native FP4 path takes unrotated E2M1 weights only
         shape = self._shape()
-        self.wdev = C.to_device_layout(self.codes.cpu(), self.meta.cpu(), shape).to(
-            self.codes.device)
-        self._f16_exact = self.fmt != "e2m1" or e2m1_scales_fit_f16(self.meta.cpu())
+        # on the GPU where the buffers are (4096x11008 GF4: 15 us instead of a copy to the host,
+        # 16 threads' permutation and a copy back, 10 ms)
+        if (self.codes.is_cuda and self.meta.device == self.codes.device
+                and self.codes.dtype == torch.uint8
+                and self.meta.dtype in (torch.uint8, torch.int16)
+                and self.codes.is_contiguous() and self.meta.is_contiguous()):
+            self.wdev = C.to_device_layout_gpu(self.codes, self.meta, shape)
+        else:
+            self.wdev = C.to_device_layout(self.codes.cpu(), self.meta.cpu(), shape).to(
+                self.codes.device)
+        self._f16_exact = self.fmt != "e2m1" or e2m1_scales_fit_f16(self.meta)
 
     # -- reference API ------------------------------------------------------------
     def dequantized_weight(self) -> torch.Tensor:

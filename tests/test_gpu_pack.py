@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from if_i_could_turn_back_time_amd import PackedWeight, _capi as C
+from if_i_could_turn_back_time_amd import PackedWeight, QuantLinear, _capi as C
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -55,3 +55,15 @@ def test_quantize_on_gpu_or_cpu_weights(fmt, device):
         pw = PackedWeight.quantize(src, fmt, device=device, packer="gpu")
         for a, b in ((pw.codes, host.codes), (pw.meta, host.meta), (pw.wdev, host.wdev)):
             assert a.device == b.device and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("kw", [dict(fmt="gf4"), dict(fmt="e2m1"), dict(fmt="gf4", hadamard=128)])
+def test_checkpoint_loads_to_the_same_stream_on_gpu_and_cpu(kw):
+    torch.manual_seed(3)
+    lin = torch.nn.Linear(384 if "hadamard" in kw else 300, 70)
+    src = QuantLinear(lin, **kw)
+    for dev in ("cpu", DEV):
+        q = QuantLinear(lin, pack=False).to(dev)
+        q.load_state_dict(src.state_dict())
+        assert q.wdev.device.type == torch.device(dev).type
+        assert torch.equal(q.wdev.cpu(), src.wdev) and q._f16_exact == src._f16_exact
