@@ -421,6 +421,7 @@ __global__ __launch_bounds__(1024) void grad_bias_kernel(const void* __restrict_
 // host side
 // ---------------------------------------------------------------------------------
 constexpr int64_t kMaxOperandBytes = 256ll << 20;  // transposed weight held at once
+constexpr int kMaxRowsW = 1 << 18;  // one span of these is 256 MiB of 16-bit operands per plane
 constexpr int64_t kMaxPartBytes = 256ll << 20;
 constexpr int kMaxParts = 8;
 
@@ -478,11 +479,11 @@ void grad_tiles(GradPlan& pl, int M, int K, int cus) {
   }
 }
 
-// s->y_dtype is gy's dtype.  Contraction rows of N values are addressed with 32-bit offsets.
+// s->y_dtype is gy's dtype.
 int grad_plan(const fb_shape_t* s, const void* gy, int f16_exact, GradPlan& pl) {
   const int st = fb_validate(s);
   if (st != FB_OK) return st;
-  if (s->N > (1 << 22) || s->B > (1 << 24)) return FB_ERR_SHAPE;
+  if (s->N > kMaxRowsW || s->B > (1 << 24)) return FB_ERR_SHAPE;
   const bool gf4 = s->fmt == FB_FMT_GF4;
   const int dt = s->y_dtype;
   if (dt == FB_DT_F16 && (gf4 || f16_exact)) {

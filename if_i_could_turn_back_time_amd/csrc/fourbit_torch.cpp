@@ -10,6 +10,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/utils/pybind.h>
 
+#include <algorithm>
 #include <optional>
 #include <stdexcept>
 
@@ -22,6 +23,9 @@ namespace {
 constexpr int64_t kMaxGemvBatch = 16;
 constexpr int64_t kMaxGemmK = 1 << 22;  // fb_gemm's limits
 constexpr int64_t kMaxGemmRows = 1 << 24;
+// Rows of grad_y at once: bounds fb_grad_x's 16-bit terms of them, and each pass's decode of W
+// is under 1% of its products.
+constexpr int64_t kGradRows = 8192;
 
 void check(int code) {
   if (code != FB_OK) throw std::runtime_error(fb_strerror(code));
@@ -139,25 +143,30 @@ std::optional<at::Tensor> linear_grad_x(const at::Tensor& gy, const at::Tensor& 
   const int gdt = dtype_code(gy.scalar_type()), xdt = dtype_code(xt);
   const int64_t kp = (K + 127) / 128 * 128;
   if (watched() || !plain(gy) || !plain(wdev) || gy.device() != wdev.device() || gy.dim() != 2 ||
-      gy.size(1) != N || gdt < 0 || xdt < 0 || gy.numel() == 0 || gy.size(0) > kMaxGemmRows)
+      gy.size(1) != N || gdt < 0 || xdt < 0 || gy.numel() == 0)
     return std::nullopt;
   fb_shape_t s{};
   s.N = (int32_t)N;
   s.K = (int32_t)kp;
-  s.B = (int32_t)gy.size(0);
+  s.B = (int32_t)std::min(gy.size(0), kGradRows);
   s.group = fmt == FB_FMT_E2M1 ? 32 : 128;
   s.fmt = (int32_t)fmt;
   s.fwht_block = (int32_t)fwht_block;
   s.x_dtype = FB_DT_F16;
   s.y_dtype = gdt;
-  const size_t need = fb_grad_x_workspace_bytes(&s, f16_exact);
-  if (!need || (size_t)wdev.numel() < fb_device_bytes(&s)) return std::nullopt;
+  if (!fb_grad_x_workspace_bytes(&s, f16_exact) || (size_t)wdev.numel() < fb_device_bytes(&s))
+    return std::nullopt;
   c10::DeviceGuard guard(gy.device());
   const at::Tensor g = gy.contiguous();
   at::Tensor gx = at::empty({gy.size(0), kp}, gy.options().dtype(xt));
-  const at::Tensor ws = scratch(need, gy);
-  check(fb_grad_x(wdev.data_ptr(), g.data_ptr(), gx.data_ptr(), &s, xdt, f16_exact, ws.data_ptr(),
-                  need, stream_of(gy)));
+  for (int64_t r = 0; r < gy.size(0); r += kGradRows) {
+    s.B = (int32_t)std::min(gy.size(0) - r, kGradRows);
+    const size_t need = fb_grad_x_workspace_bytes(&s, f16_exact);
+    const at::Tensor ws = scratch(need, gy);
+    check(fb_grad_x(wdev.data_ptr(), static_cast<const char*>(g.data_ptr()) + r * N * g.element_size(),
+                    static_cast<char*>(gx.data_ptr()) + r * kp * gx.element_size(), &s, xdt,
+                    f16_exact, ws.data_ptr(), need, stream_of(gy)));
+  }
   return kp == K ? gx : gx.narrow(1, 0, K).contiguous();
 }
 

@@ -122,8 +122,9 @@ def _gemv_chunks(wdev, N, kp, fmt, fwht_block, xk, y, fp4_mfma=False, ws_cache=N
             C.gemv(wdev, xk[b0:b1], y[b0:b1], shape, ws)
 
 
-# fb_grad_x addresses a row of grad_y with 32-bit offsets.
-MAX_GRAD_N = 1 << 22
+# fb_grad_x holds the 16-bit operands of at least 512 weight columns at once: 256 MiB at this
+# many rows.
+MAX_GRAD_N = 1 << 18
 # Most bytes of fp32 weight the torch form of the backward pass decodes at once (a chunk of 16-row tiles).
 BACKWARD_CHUNK_BYTES = 64 * 2**20
 

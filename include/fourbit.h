@@ -273,7 +273,7 @@ size_t fb_mx_presplit_workspace_bytes(const fb_shape_t* s);
  * bytes (the transposed 16-bit weight, at most 256 MiB of it at once unless 512 of its K-columns
  * take more, gy's terms, the sums of contraction parts, and for a rotated layer the fp32
  * gradient).  Its contents need no initialisation; calls that share it must not overlap.
- * N <= 2^22, B <= 2^24 (FB_ERR_SHAPE). */
+ * N <= 2^18, B <= 2^24 (FB_ERR_SHAPE). */
 int fb_grad_x(const void* wdev, const void* gy, void* gx, const fb_shape_t* s, int32_t gx_dtype,
               int32_t f16_exact, void* ws, size_t ws_bytes, void* stream);
 
