@@ -10,9 +10,9 @@
 //    weight is decoded once per workgroup.
 //  - x goes through LDS in chunks of 128 K-values: the 32 values of each of a span's four
 //    128-value items that the four k-steps of one 16-byte nibble chunk multiply.  The loads
-//    write LDS directly (no VGPRs, no ds_write); the 16-byte units of an x row are permuted by
-//    unit ^ (row % 16) on the load's source side, which leaves the MFMA B reads (16 rows, 256
-//    bytes apart) without a bank conflict.
+//    write LDS directly (no VGPRs, no ds_write); the 16-byte units of an x row are permuted on
+//    the load's source side (unit_mask), which leaves the MFMA B reads (16 rows, 256 bytes
+//    apart) without a bank conflict.
 //  - Nibbles and x are requested kBufs - 1 (1 or 3) chunks ahead, with one barrier per chunk.
 //  - Each k-step's decode (21 VALU instructions per GF4 row tile, 8 codes per lane) is written
 //    between the MFMAs of the step before it, a half decode per column tile, and the column
@@ -48,6 +48,13 @@ namespace {
 
 constexpr int kGemmWaves = 4;
 constexpr int kRowBytes = 256;  // one x row of a chunk: 128 K-values, 32 of each item of a span
+
+// What the 16-byte units of an x row n (mod 16) in LDS are permuted by (unit u sits at place u ^
+// unit_mask(n)).  A 16-byte LDS read serves 16 lanes at a time over all 64 banks: lanes 0-3,
+// 12-15, 20-23 and 24-27 together, and so on.  In the B read lane L takes row L % 16, unit
+// 4 (L / 16) + s, so such a set holds 16 different rows, of two neighbouring items, and n itself
+// as the mask would put half of them on the same places (4 of 12 cycles per read, counted).
+__device__ __forceinline__ int unit_mask(int n) { return n ^ ((((n >> 2) ^ (n >> 3)) & 1) << 2); }
 
 struct GemmArgs {
   const uint8_t* w;
@@ -133,7 +140,7 @@ __global__ __launch_bounds__(kGemmWaves * 64, 2) void gemm_kernel(GemmArgs a) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int row = (wave * XD + j) * 4 + (lane >> 4);
-    const int u = (lane & 15) ^ (row & 15);
+    const int u = (lane & 15) ^ unit_mask(row & 15);
     xoff[j] = (unsigned)row * (unsigned)a.K * 2u + (u >> 2) * 256 + (u & 3) * 16;
     xk[j] = (u >> 2) * 128;
   }
@@ -179,7 +186,8 @@ __global__ __launch_bounds__(kGemmWaves * 64, 2) void gemm_kernel(GemmArgs a) {
     for (int c = 0; c < CT; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // B operand of column tile ct, k-step s: x row lane % 16, unit 4 (lane / 16) + s
-  const unsigned rbase = (lane & 15) * kRowBytes + ((((lane >> 4) * 4) ^ (lane & 15)) << 4);
+  const unsigned rbase =
+      (lane & 15) * kRowBytes + ((((lane >> 4) * 4) ^ unit_mask(lane & 15)) << 4);
 
   // Half h of the A operand of k-step s of chunk c (words 2h, 2h + 1 of 4), from nibbles nb
   // and tables tt.
