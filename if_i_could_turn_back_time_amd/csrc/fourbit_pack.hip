@@ -33,9 +33,9 @@
 // exact).  So it rounds as the division does.  x = s^2 is 0 or at least 2^-298 (s is a
 // multiple of the smallest fp32), so nothing underflows.
 //
-// Bound by the VALU (fp64 adds, compares and selects: about 95 instructions per i, 14,300 per group in all).  4096^2
-// (131,072 groups): 17.9 ms with the class loop outermost (SSD with a division
-// in it, back pointers kept), 4.0 ms now, the VALU busy 97% of the time.
+// Bound by the VALU (fp64 adds, minima and readlanes: about 95 instructions per i, 14,300 per
+// group in all).  4096^2 (131,072 groups): 17.9 ms with the class loop outermost (SSD with a
+// division in it, back pointers kept), 4.0 ms now, the VALU busy 97% of the time.
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 

@@ -258,20 +258,21 @@ def packed_linear(wdev: torch.Tensor, N: int, K: int, fmt: str, fwht_block: int,
                   range_check: bool = False, f16_exact: bool = True,
                   fp4_mfma: bool = False, ws_cache: dict | None = None) -> torch.Tensor:
     """``F.linear(x, W, bias)`` for a packed 4-bit ``W [N, K]`` (device stream ``wdev``
-    of a ``packed_k(K)``-wide weight), through fb_gemv in chunks of 16 rows of x.
+    of a ``packed_k(K)``-wide weight): fb_gemv for up to 16 rows of x, fb_gemm for more.
 
     x may have any leading shape and dtype: it is cast to fp16 (GF4, or any rotation) or
     kept in fp16/bf16 (E2M1; fp32 becomes bf16) and zero-padded to ``packed_k(K)``; y
     has x's dtype (fp32 for other dtypes).  Differentiable in x (and bias): the weight is
     frozen, as the reference's committed weight is.  ``range_check`` (see
     ``_kernel_input``) raises instead of letting fp16 staging overflow, at the cost of a
-    host sync; ``ws_cache`` keeps the call's fb_gemv workspace for the next calls (a dict
-    the caller owns, e.g. one per module); ``f16_exact``
-    (E2M1 only) says whether the weight's scales decode exactly to fp16.  ``fp4_mfma``
-    (unrotated E2M1 only) runs the matrix cores' native FP4 path (fb_gemv_mx): x as bf16,
-    split into two MX-E4M3 terms, which hold a bf16 value exactly unless its 32-value block
-    spans more than E4M3's exponent range (fp16 and fp32 x are rounded to bf16 first).  No
-    CPU path: x must be on the GPU."""
+    host sync; ``ws_cache`` keeps the Python path's fb_gemv workspace for the next calls (a dict
+    the caller owns, e.g. one per module; the native call takes its own from the allocator);
+    ``f16_exact`` (E2M1 only) says whether the weight's scales decode exactly to fp16.  ``fp4_mfma``
+    (unrotated E2M1 only) runs the matrix cores' native FP4 path (fb_gemv_mx) for up to 16 rows
+    (more run fb_gemm on the bf16 x and the exact weight): x as bf16, split into two MX-E4M3
+    terms, which hold a bf16 value exactly unless its 32-value block spans more than E4M3's
+    exponent range (fp16 and fp32 x are rounded to bf16 first).  No CPU path: x must be on the
+    GPU."""
     grad = torch.is_grad_enabled()
     bias_grad = grad and bias is not None and bias.requires_grad
     if not (range_check or bias_grad or (grad and x.requires_grad)):
@@ -293,7 +294,12 @@ def packed_linear(wdev: torch.Tensor, N: int, K: int, fmt: str, fwht_block: int,
                                   fp4_mfma, ws_cache)
         return y.reshape(*lead, N)
     with torch.no_grad():
-        y = _forward(x2, wdev, N, K, fmt, fwht_block, range_check, f16_exact, fp4_mfma, ws_cache)
+        y = None
+        if not range_check:
+            y = _native_forward(x2, wdev, N, K, fmt, fwht_block, f16_exact, fp4_mfma, None)
+        if y is None:
+            y = _forward(x2, wdev, N, K, fmt, fwht_block, range_check, f16_exact, fp4_mfma,
+                         ws_cache)
     if bias is not None:
         if bias_grad:
             y = y + bias.to(y.dtype)
@@ -469,7 +475,7 @@ class QuantLinear(nn.Linear):
         # captured).  Off by default, so the forward never syncs and can be captured in a
         # HIP graph; an overflow then shows as non-finite outputs.
         self.range_check = False
-        # fb_gemv / fb_gemv_mx workspaces of this module, per (device, stream)
+        # the Python path's fb_gemv / fb_gemv_mx workspaces of this module, per (device, stream)
         self._ws_cache = {}
         self._f16_exact = True
         self.register_load_state_dict_post_hook(QuantLinear._rebuild_after_load)
@@ -641,10 +647,11 @@ class QuantLinear(nn.Linear):
 
 def fp4_mfma_shared(layers, x: torch.Tensor):
     """Runs several E2M1 ``QuantLinear`` layers that take the same input x (the q/k/v or
-    gate/up projections of one activation) on the native FP4 path with one split of x per
-    16 rows (fb_mx_split, then fb_gemv_mx_presplit per layer): ``(y_0, y_1, ...)``, each
-    what ``layer(x)`` gives with ``fp4_mfma=True``.  When autograd needs x's gradient each
-    layer runs on its own (the split is not differentiable; every layer's backward is).
+    gate/up projections of one activation) on the native FP4 path with one split of x
+    (fb_mx_split, then fb_gemv_mx_presplit per layer): ``(y_0, y_1, ...)``, each what
+    ``layer(x)`` gives with ``fp4_mfma=True``.  Each layer runs on its own for more than 16 rows
+    (fb_gemm takes x unsplit) and when autograd needs x's gradient (the split is not
+    differentiable; every layer's backward is).
     No counterpart in the reference, whose layers each run their own ``F.linear``."""
     layers = list(layers)
     if not layers:
@@ -661,8 +668,10 @@ def fp4_mfma_shared(layers, x: torch.Tensor):
     if not x.is_cuda:
         raise RuntimeError("the packed 4-bit linear runs the HIP kernel: move the modules and "
                            "input to a ROCm GPU")
-    if torch.is_grad_enabled() and (x.requires_grad or any(
-            q.bias is not None and q.bias.requires_grad for q in layers)):
+    # more rows than a GEMV takes run the GEMM, which needs no split of x
+    if x.numel() // K > MAX_GEMV_BATCH and packed_k(K) <= MAX_GEMM_K or (
+            torch.is_grad_enabled() and (x.requires_grad or any(
+                q.bias is not None and q.bias.requires_grad for q in layers))):
         return tuple(packed_linear(q.wdev, q.out_features, K, "e2m1", 0, x, q.bias,
                                    range_check=q.range_check, f16_exact=q._f16_exact,
                                    fp4_mfma=True, ws_cache=q._ws_cache) for q in layers)
@@ -673,10 +682,6 @@ def fp4_mfma_shared(layers, x: torch.Tensor):
     ydt = x2.dtype if x2.dtype in C.DTYPE_CODE else torch.float32
     ys = [torch.empty(x2.shape[0], q.out_features, dtype=ydt, device=x.device) for q in layers]
     with torch.no_grad():
-        if xk.shape[0] > MAX_GEMV_BATCH and kp <= MAX_GEMM_K:  # as _gemv_chunks does: no split
-            for q, y in zip(layers, ys):
-                _gemv_chunks(q.wdev, q.out_features, kp, "e2m1", 0, xk, y)
-            xk = xk[:0]
         for b0 in range(0, xk.shape[0], MAX_GEMV_BATCH):
             b1 = min(b0 + MAX_GEMV_BATCH, xk.shape[0])
             sh0 = C.make_shape(layers[0].out_features, kp, b1 - b0, C.FMT_E2M1, 0, C.DT_BF16,
