@@ -129,22 +129,44 @@ MAX_GRAD_N = 1 << 18
 BACKWARD_CHUNK_BYTES = 64 * 2**20
 
 
+class _DecodedProduct(torch.autograd.Function):
+    """``g @ W`` for a chunk of row tiles, W decoded (fb_dequant, fp32) for this product only.
+    Its backward decodes W again: autograd would keep a W for every chunk, or, with one buffer
+    for all of them, the last chunk's W for each."""
+
+    @staticmethod
+    def forward(ctx, g, wdev, shape):
+        ctx.save_for_backward(wdev)
+        ctx.shape = shape
+        return g @ C.dequant_device(wdev, shape, torch.float32)
+
+    @staticmethod
+    def backward(ctx, v):
+        (wdev,) = ctx.saved_tensors
+        return v @ C.dequant_device(wdev, ctx.shape, torch.float32).t(), None, None
+
+
 def _grad_x(wdev, N, kp, fmt, fwht_block, gy: torch.Tensor) -> torch.Tensor:
     """``grad_y [M, N] @ W [N, kp]`` in fp32 with W decoded on the device (fb_dequant,
     exact) a chunk of row tiles at a time: at most ``BACKWARD_CHUNK_BYTES`` of decoded
-    weight exist at once, whatever the layer's size.  Chunks are added in row order."""
+    weight exist at once, whatever the layer's size.  Chunks are added in row order.
+    Differentiable in grad_y."""
     f = C.FMT_BY_NAME[fmt]
     rows = max(16, BACKWARD_CHUNK_BYTES // (kp * 4) // 16 * 16)
     gyf = gy.float()
     gx = torch.zeros(gy.shape[0], kp, dtype=torch.float32, device=gy.device)
+    differentiable = torch.is_grad_enabled() and gy.requires_grad
     buf = None
     for r0 in range(0, N, rows):
         r1 = min(N, r0 + rows)
         shape = C.make_shape(r1 - r0, kp, 1, f, fwht_block)
+        w = wdev[C.tile_offset(shape, r0):]
+        if differentiable:
+            gx = gx + _DecodedProduct.apply(gyf[:, r0:r1], w, shape)
+            continue
         if buf is None or buf.shape[0] != r1 - r0:
             buf = torch.empty(r1 - r0, kp, dtype=torch.float32, device=gy.device)
-        W = C.dequant_device(wdev[C.tile_offset(shape, r0):], shape, torch.float32, out=buf)
-        gx.addmm_(gyf[:, r0:r1], W)
+        gx.addmm_(gyf[:, r0:r1], C.dequant_device(w, shape, torch.float32, out=buf))
     return gx
 
 
