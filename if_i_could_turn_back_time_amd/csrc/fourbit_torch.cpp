@@ -68,7 +68,9 @@ std::optional<at::Tensor> linear_forward(const at::Tensor& x, const at::Tensor& 
   if (watched() || !plain(x) || !plain(wdev) || x.device() != wdev.device() || x.dim() < 1 ||
       x.size(-1) != K || K < 1 || x.numel() == 0)
     return std::nullopt;
-  if (bias && (!plain(*bias) || bias->device() != x.device())) return std::nullopt;
+  // a bias of more dimensions broadcasts against the [M, N] product, not against y's shape
+  if (bias && (!plain(*bias) || bias->device() != x.device() || bias->dim() > 1))
+    return std::nullopt;
   const int xdt = dtype_code(x.scalar_type());
   if (xdt < 0) return std::nullopt;
   const bool e2m1 = fmt == FB_FMT_E2M1;

@@ -266,6 +266,13 @@ def _forward(x2, wdev, N, K, fmt, fwht_block, range_check, f16_exact, fp4_mfma, 
 _PLAIN = (torch.Tensor, nn.Parameter)
 
 
+def _vector_bias(bias, N: int) -> bool:
+    """Whether bias is an ordinary [N] vector, which the kernels add and _PackedLinearFn
+    differentiates.  Any other one (a row per row of x, a single value) broadcasts against the
+    [M, N] product as a torch operation."""
+    return type(bias) in _PLAIN and bias.dim() == 1 and bias.shape[0] == N
+
+
 def _native_forward(x, wdev, N, K, fmt, fwht_block, f16_exact, fp4_mfma, bias):
     """The whole forward in one native call (fourbit_torch.cpp), or None where x, the weight or
     the bias is not a plain GPU tensor it takes."""
@@ -312,8 +319,11 @@ def packed_linear(wdev: torch.Tensor, N: int, K: int, fmt: str, fwht_block: int,
     lead = x.shape[:-1]
     x2 = x.reshape(-1, K)
     if grad and x.requires_grad:
-        y = _PackedLinearFn.apply(x2, bias, wdev, N, K, fmt, fwht_block, range_check, f16_exact,
-                                  fp4_mfma, ws_cache)
+        inside = _vector_bias(bias, N)
+        y = _PackedLinearFn.apply(x2, bias if inside else None, wdev, N, K, fmt, fwht_block,
+                                  range_check, f16_exact, fp4_mfma, ws_cache)
+        if bias is not None and not inside:
+            y = y + bias.to(y.dtype)
         return y.reshape(*lead, N)
     with torch.no_grad():
         y = None

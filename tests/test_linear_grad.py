@@ -1,5 +1,7 @@
-"""The packed linear layer under autograd: second derivatives over several decoded chunks."""
+"""The packed linear layer under autograd: second derivatives over several decoded chunks, and
+the bias in every shape and every kind of derivative."""
 import ctypes
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -18,6 +20,32 @@ def _dequant_cpu(wdev, shape, out_dtype=torch.float32, out=None):
         return w
     ctypes.memmove(out.data_ptr(), w.data_ptr(), w.numel() * 4)
     return out
+
+
+@pytest.fixture(params=["cpu", pytest.param(DEV, marks=pytest.mark.gpu)])
+def dev(request, monkeypatch):
+    """The GPU, or the CPU with the kernels' calls replaced by products with the decoded weight
+    (what packed_linear and its autograd functions do around them stays)."""
+    if request.param == "cpu":
+        def forward(x2, wdev, N, K, fmt, fwht_block, *rest):
+            shape = C.make_shape(N, LN.packed_k(K), 1, C.FMT_BY_NAME[fmt], fwht_block)
+            return x2 @ _dequant_cpu(wdev, shape)[:, :K].t().to(x2.dtype)
+
+        def declines(*args):
+            return None
+
+        monkeypatch.setattr(torch.Tensor, "is_cuda", property(lambda t: True))
+        monkeypatch.setattr(LN, "_forward", forward)
+        monkeypatch.setattr(C, "dequant_device", _dequant_cpu)
+        monkeypatch.setattr(C, "_native", SimpleNamespace(
+            linear_forward=declines, linear_grad_x=declines, linear_grad_bias=declines))
+    return request.param
+
+
+def _layer(dev, K=256, N=40, **kw):
+    w = torch.randn(N, K) * 0.05
+    pw = PackedWeight.quantize(w, **{"fmt": "gf4", **kw})
+    return pw.wdev.to(dev), pw.dequant_host().to(dev)
 
 
 @pytest.mark.parametrize("fmt", ["gf4", "e2m1"])
@@ -56,3 +84,46 @@ def test_layer_gradient_of_the_gradient_over_chunks(kw, monkeypatch):
     vr = LN._fwht_last_dim(v, q.fwht_block) if q.fwht_block else v
     bound = (768 + 16) * 2.0 ** -24 * float((vr.abs() @ w.abs().t()).max())
     assert torch.allclose(c, vr @ w.t(), rtol=0, atol=2 * bound)
+
+
+@pytest.mark.parametrize("shape", [(40,), (1,), (), (1, 40), (6, 40), (6, 1), (2, 3, 40)])
+@pytest.mark.parametrize("lead", [(6,), (2, 3), (1,), ()])
+def test_bias_of_any_shape(dev, shape, lead):
+    """A bias broadcasts against the [M, N] product, whatever x's leading shape, and gets a
+    gradient of its own shape; what y + bias refuses is refused."""
+    K, N, M = 256, 40, int(torch.Size(lead).numel())
+    wdev, w = _layer(dev)
+    x, bias = torch.randn(*lead, K, device=dev), torch.randn(shape, device=dev)
+    gy = torch.randn(M, N, device=dev)
+
+    def reference(x, b):
+        return (x.half().float().reshape(M, K) @ w.t() + b).reshape(*lead, N)
+
+    for xg in (False, True):
+        for bg in (False, True):
+            out = []
+            for f in (reference, lambda x, b: LN.packed_linear(wdev, N, K, "gf4", 0, x, b)):
+                xi, bi = x.clone().requires_grad_(xg), bias.clone().requires_grad_(bg)
+                try:
+                    y = f(xi, bi)
+                except RuntimeError:
+                    out.append(None)
+                    continue
+                ins = [t for t in (xi, bi) if t.requires_grad]
+                grads = torch.autograd.grad(y, ins, gy.reshape(y.shape)) if ins else ()
+                out.append((y.detach(), *grads))
+            ref, got = out
+            if ref is None:
+                assert got is None
+                continue
+            for a, b in zip(ref, got, strict=True):
+                assert a.shape == b.shape and torch.allclose(a, b, rtol=1e-3, atol=1e-3)
+    with torch.no_grad():
+        try:
+            ref = reference(x, bias)
+        except RuntimeError:
+            with pytest.raises(RuntimeError):
+                LN.packed_linear(wdev, N, K, "gf4", 0, x, bias)
+        else:
+            got = LN.packed_linear(wdev, N, K, "gf4", 0, x, bias)
+            assert got.shape == ref.shape and torch.allclose(got, ref, rtol=1e-3, atol=1e-3)
