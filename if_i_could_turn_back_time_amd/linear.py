@@ -206,9 +206,9 @@ def _kernel_input(x2: torch.Tensor, K: int, fmt: str, fwht_block: int, range_che
 
 
 class _PackedLinearFn(torch.autograd.Function):
-    """``x -> x W^T`` through the fused kernel, differentiable in x (as ``F.linear`` with
-    the reference's frozen committed weight is, ``layers.py:34-35``).  Backward:
-    ``grad_x = grad_y W`` and, for a rotated weight W' = W H, rotated back:
+    """``x -> x W^T (+ bias)`` through the fused kernel, differentiable in x (as ``F.linear`` with
+    the reference's frozen committed weight is, ``layers.py:34-35``); the bias is a constant
+    here.  Backward: ``grad_x = grad_y W`` and, for a rotated weight W' = W H, rotated back:
     ``grad_x = (grad_y W') H``, in one native call (fb_grad_x).  Where the gradient itself is
     to be differentiated, and for more rows of W than fb_grad_x takes, the same from torch
     operations on W decoded in chunks of row tiles (``_grad_x``)."""
@@ -225,33 +225,46 @@ class _PackedLinearFn(torch.autograd.Function):
             if bias is not None:
                 y.add_(bias.to(y.dtype))
         ctx.save_for_backward(wdev)
-        ctx.cfg = (N, K, fmt, fwht_block, x2.dtype, f16_exact,
-                   None if bias is None else bias.dtype)
+        ctx.cfg = (N, K, fmt, fwht_block, x2.dtype, f16_exact)
         return y
 
     @staticmethod
     def backward(ctx, gy):
         (wdev,) = ctx.saved_tensors
-        N, K, fmt, fwht_block, xdt, f16_exact, bdt = ctx.cfg
-        native = not torch.is_grad_enabled() and type(gy) is torch.Tensor
-        gb = gx = None
-        if ctx.needs_input_grad[1]:
-            if native:
-                gb = C.native().linear_grad_bias(gy, bdt)
-            if gb is None:
-                gb = gy.sum(0).to(bdt)
-        if ctx.needs_input_grad[0]:
-            if native and N <= MAX_GRAD_N:
-                gx = C.native().linear_grad_x(gy, wdev, N, K, C.FMT_BY_NAME[fmt], fwht_block,
-                                              f16_exact,
-                                              xdt if xdt in C.DTYPE_CODE else torch.float32)
-            if gx is None:
-                gx = _grad_x(wdev, N, packed_k(K), fmt, fwht_block, gy)
-                if fwht_block:
-                    gx = _fwht_last_dim(gx, fwht_block)
-                gx = gx[:, :K]
-            gx = gx.to(xdt)
-        return gx, gb, None, None, None, None, None, None, None, None, None
+        N, K, fmt, fwht_block, xdt, f16_exact = ctx.cfg
+        gx = None
+        if _native_gradient(gy) and N <= MAX_GRAD_N:
+            gx = C.native().linear_grad_x(gy, wdev, N, K, C.FMT_BY_NAME[fmt], fwht_block, f16_exact,
+                                          xdt if xdt in C.DTYPE_CODE else torch.float32)
+        if gx is None:
+            gx = _grad_x(wdev, N, packed_k(K), fmt, fwht_block, gy)
+            if fwht_block:
+                gx = _fwht_last_dim(gx, fwht_block)
+            gx = gx[:, :K]
+        return gx.to(xdt), None, None, None, None, None, None, None, None, None, None
+
+
+class _AddedBias(torch.autograd.Function):
+    """y, which holds the bias already, as a function of the bias.  A node of its own because
+    autograd runs a function's whole backward for any one of its inputs: as part of
+    _PackedLinearFn, asking for the bias's gradient alone would compute grad_x too."""
+
+    @staticmethod
+    def forward(ctx, y, bias):
+        ctx.mark_dirty(y)
+        ctx.bias_dtype = bias.dtype
+        return y
+
+    @staticmethod
+    def backward(ctx, gy):
+        gb = C.native().linear_grad_bias(gy, ctx.bias_dtype) if _native_gradient(gy) else None
+        return gy, gy.sum(0).to(ctx.bias_dtype) if gb is None else gb
+
+
+def _native_gradient(gy) -> bool:
+    """Whether a native call may compute from grad_y: not where autograd records operations on
+    it (a gradient to be differentiated)."""
+    return not torch.is_grad_enabled() and type(gy) is torch.Tensor
 
 
 def _forward(x2, wdev, N, K, fmt, fwht_block, range_check, f16_exact, fp4_mfma, ws_cache):
@@ -267,7 +280,7 @@ _PLAIN = (torch.Tensor, nn.Parameter)
 
 
 def _vector_bias(bias, N: int) -> bool:
-    """Whether bias is an ordinary [N] vector, which the kernels add and _PackedLinearFn
+    """Whether bias is an ordinary [N] vector, which the kernels add and _AddedBias
     differentiates.  Any other one (a row per row of x, a single value) broadcasts against the
     [M, N] product as a torch operation."""
     return type(bias) in _PLAIN and bias.dim() == 1 and bias.shape[0] == N
@@ -320,9 +333,11 @@ def packed_linear(wdev: torch.Tensor, N: int, K: int, fmt: str, fwht_block: int,
     x2 = x.reshape(-1, K)
     if grad and x.requires_grad:
         inside = _vector_bias(bias, N)
-        y = _PackedLinearFn.apply(x2, bias if inside else None, wdev, N, K, fmt, fwht_block,
-                                  range_check, f16_exact, fp4_mfma, ws_cache)
-        if bias is not None and not inside:
+        y = _PackedLinearFn.apply(x2, bias.detach() if inside else None, wdev, N, K, fmt,
+                                  fwht_block, range_check, f16_exact, fp4_mfma, ws_cache)
+        if inside and bias_grad:
+            y = _AddedBias.apply(y, bias)
+        elif bias is not None and not inside:
             y = y + bias.to(y.dtype)
         return y.reshape(*lead, N)
     with torch.no_grad():

@@ -127,3 +127,35 @@ def test_bias_of_any_shape(dev, shape, lead):
         else:
             got = LN.packed_linear(wdev, N, K, "gf4", 0, x, bias)
             assert got.shape == ref.shape and torch.allclose(got, ref, rtol=1e-3, atol=1e-3)
+
+
+@pytest.mark.parametrize("M", [5, 40])
+def test_gradient_of_the_bias_alone(dev, M, monkeypatch):
+    """Asked for by itself, the bias's gradient decodes no weight and multiplies nothing."""
+    K, N = 256, 40
+    wdev, w = _layer(dev)
+    x = torch.randn(M, K, device=dev, requires_grad=True)
+    bias = torch.randn(N, device=dev, requires_grad=True)
+    gy = torch.randn(M, N, device=dev)
+    y = LN.packed_linear(wdev, N, K, "gf4", 0, x, bias)
+    calls = []
+    native = C.native()
+    monkeypatch.setattr(C, "_native", SimpleNamespace(
+        linear_forward=native.linear_forward, linear_grad_bias=native.linear_grad_bias,
+        linear_grad_x=lambda *a: calls.append("native") or native.linear_grad_x(*a)))
+    decode = C.dequant_device
+    monkeypatch.setattr(C, "dequant_device", lambda *a, **k: calls.append("decode") or decode(*a, **k))
+    (gb,) = torch.autograd.grad(y, bias, gy, retain_graph=True)
+    assert not calls and torch.allclose(gb, gy.sum(0), rtol=1e-5, atol=1e-5)
+    (gx,) = torch.autograd.grad(y, x, gy, retain_graph=True)
+    assert calls and torch.allclose(gx, gy @ w, rtol=1e-4, atol=1e-4)
+    both = torch.autograd.grad(y, (x, bias), gy, retain_graph=True)
+    assert torch.equal(both[0], gx) and torch.equal(both[1], gb)
+    # the gradient of the bias's gradient: d(gb . u) / d(gy) is u in every row
+    g2, u = gy.clone().requires_grad_(True), torch.randn(N, device=dev)
+    (gb,) = torch.autograd.grad(y, bias, g2, create_graph=True)
+    (c,) = torch.autograd.grad((gb * u).sum(), g2)
+    assert torch.equal(c, u.expand(M, N))
+    # the result may be changed in place, as one of y + bias may
+    z = LN.packed_linear(wdev, N, K, "gf4", 0, x, bias).mul_(2)
+    assert torch.allclose(torch.autograd.grad(z, bias, gy)[0], 2 * gb, rtol=1e-5, atol=1e-5)
