@@ -1,9 +1,10 @@
 // The packed linear layer's call path from torch: one native call per forward (and per activation
-// gradient) instead of a dozen Python, ctypes and dispatcher steps.  It checks, converts and
-// allocates exactly as linear.py's packed_linear does and launches the same kernels; what it
-// does not recognise (another dtype, a refused shape, a wrapped tensor, an active dispatch
-// mode) it leaves to packed_linear by returning None.  A decode call of a 4096^2 layer takes
-// 5 us on the GPU and took 22 us of host time through Python.
+// gradient) instead of a dozen Python, ctypes and dispatcher steps.  It launches the kernels that
+// linear.py's packed_linear launches, on x converted as there, and takes workspaces from the
+// allocator; what it does not recognise (another dtype, a refused shape, a wrapped tensor, a bias
+// that is no vector or has a forward-mode tangent, an active dispatch mode) it leaves to
+// packed_linear by returning None.  A decode call of a 4096^2 layer takes 5 us on the GPU and took
+// 22 us of host time through Python.
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -68,8 +69,10 @@ std::optional<at::Tensor> linear_forward(const at::Tensor& x, const at::Tensor& 
   if (watched() || !plain(x) || !plain(wdev) || x.device() != wdev.device() || x.dim() < 1 ||
       x.size(-1) != K || K < 1 || x.numel() == 0)
     return std::nullopt;
-  // a bias of more dimensions broadcasts against the [M, N] product, not against y's shape
-  if (bias && (!plain(*bias) || bias->device() != x.device() || bias->dim() > 1))
+  // a bias of more dimensions broadcasts against the [M, N] product, not against y's shape; one
+  // with a forward-mode tangent gives y a tangent, which only a torch operation does
+  if (bias && (!plain(*bias) || bias->device() != x.device() || bias->dim() > 1 ||
+               bias->_fw_grad(0).defined()))
     return std::nullopt;
   const int xdt = dtype_code(x.scalar_type());
   if (xdt < 0) return std::nullopt;

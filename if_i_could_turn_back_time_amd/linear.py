@@ -27,6 +27,7 @@ import copy
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd.forward_ad import unpack_dual
 
 from . import _capi as C
 
@@ -281,9 +282,10 @@ _PLAIN = (torch.Tensor, nn.Parameter)
 
 def _vector_bias(bias, N: int) -> bool:
     """Whether bias is an ordinary [N] vector, which the kernels add and _AddedBias
-    differentiates.  Any other one (a row per row of x, a single value) broadcasts against the
-    [M, N] product as a torch operation."""
-    return type(bias) in _PLAIN and bias.dim() == 1 and bias.shape[0] == N
+    differentiates.  Any other one (a row per row of x, a single value, one with a forward-mode
+    tangent) broadcasts against the [M, N] product as a torch operation."""
+    return (type(bias) in _PLAIN and bias.dim() == 1 and bias.shape[0] == N
+            and unpack_dual(bias).tangent is None)
 
 
 def _native_forward(x, wdev, N, K, fmt, fwht_block, f16_exact, fp4_mfma, bias):

@@ -5,6 +5,7 @@ from types import SimpleNamespace
 
 import pytest
 import torch
+import torch.autograd.forward_ad as fwAD
 
 from if_i_could_turn_back_time_amd import PackedWeight, QuantLinear, _capi as C
 from if_i_could_turn_back_time_amd import linear as LN
@@ -159,3 +160,24 @@ def test_gradient_of_the_bias_alone(dev, M, monkeypatch):
     # the result may be changed in place, as one of y + bias may
     z = LN.packed_linear(wdev, N, K, "gf4", 0, x, bias).mul_(2)
     assert torch.allclose(torch.autograd.grad(z, bias, gy)[0], 2 * gb, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("lead", [(5,), (2, 20)])
+@pytest.mark.parametrize("bdt", [torch.float32, torch.float16])
+def test_forward_mode_tangent_of_the_bias(dev, lead, bdt):
+    """A dual bias gives y its tangent, broadcast over x's rows, whether or not x or the bias
+    requires grad."""
+    K, N = 256, 40
+    wdev, w = _layer(dev)
+    x = torch.randn(*lead, K, device=dev)
+    bias, t = (torch.randn(N, device=dev).to(bdt) for _ in range(2))
+    plain = LN.packed_linear(wdev, N, K, "gf4", 0, x, bias)
+    for xg in (False, True):
+        for bg in (False, True):
+            for mode in (torch.enable_grad, torch.no_grad):
+                with mode(), fwAD.dual_level():
+                    b = fwAD.make_dual(bias.clone().requires_grad_(bg), t)
+                    y = LN.packed_linear(wdev, N, K, "gf4", 0, x.clone().requires_grad_(xg), b)
+                    p, ty = fwAD.unpack_dual(y)
+                    assert torch.allclose(p, plain, rtol=1e-5, atol=1e-5)
+                    assert ty is not None and torch.equal(ty, t.float().expand(*lead, N))
