@@ -65,7 +65,8 @@ void* ptr_or_null(const at::Tensor& t, size_t bytes) { return bytes ? t.data_ptr
 // F.linear(x, W, bias) for a packed W, no gradients; None where packed_linear has to decide.
 std::optional<at::Tensor> linear_forward(const at::Tensor& x, const at::Tensor& wdev, int64_t N,
                                          int64_t K, int64_t fmt, int64_t fwht_block, bool f16_exact,
-                                         bool fp4_mfma, const std::optional<at::Tensor>& bias) {
+                                         bool fp4_mfma, const std::optional<at::Tensor>& bias,
+                                         bool bf16_exact) {
   if (watched() || !plain(x) || !plain(wdev) || x.device() != wdev.device() || x.dim() < 1 ||
       x.size(-1) != K || K < 1 || x.numel() == 0)
     return std::nullopt;
@@ -86,6 +87,8 @@ std::optional<at::Tensor> linear_forward(const at::Tensor& x, const at::Tensor& 
   if (e2m1 && kdt == FB_DT_F16 && !f16_exact) return std::nullopt;
   const int64_t kp = (K + 127) / 128 * 128, M = x.numel() / K;
   if (M > kMaxGemmRows || (M > kMaxGemvBatch && kp > kMaxGemmK)) return std::nullopt;
+  // the GEMM decodes to bf16; the split of more than one GEMV batch is linear.py's
+  if (M > kMaxGemvBatch && fp4_mfma && !bf16_exact) return std::nullopt;
 
   fb_shape_t s{};
   s.N = (int32_t)N;

@@ -56,13 +56,23 @@ FP16_MAX = 65504.0
 E2M1_F16_SCALES = (104, 140)
 
 
+# The largest E8M0 byte whose E2M1 products are all exact bf16 values: 6 * 2^(s-127) is beyond
+# bf16's range from 253 on.  (The smallest, 0.5 * 2^-127, is a bf16 subnormal.)
+E2M1_BF16_SCALE_MAX = 252
+
+
+def _scales_fit(meta: torch.Tensor) -> tuple[bool, bool]:
+    """Whether an E2M1 weight of these E8M0 bytes decodes exactly to (fp16, bf16)."""
+    if meta.numel() == 0:
+        return True, True
+    lo, hi = int(meta.min()), int(meta.max())
+    return E2M1_F16_SCALES[0] <= lo and hi <= E2M1_F16_SCALES[1], hi <= E2M1_BF16_SCALE_MAX
+
+
 def e2m1_scales_fit_f16(meta: torch.Tensor) -> bool:
     """Whether every E8M0 byte of an E2M1 weight lies in ``E2M1_F16_SCALES``, i.e. the
     kernel's fp16 decode (fp16 activations) gives the exact weight values."""
-    if meta.numel() == 0:
-        return True
-    lo, hi = int(meta.min()), int(meta.max())
-    return E2M1_F16_SCALES[0] <= lo and hi <= E2M1_F16_SCALES[1]
+    return _scales_fit(meta)[0]
 
 
 def _fwht_last_dim(t: torch.Tensor, block: int) -> torch.Tensor:
@@ -100,14 +110,18 @@ def _workspace(cache: dict | None, nbytes: int, device: torch.device):
 MAX_GEMM_K = 1 << 22
 
 
-def _gemv_chunks(wdev, N, kp, fmt, fwht_block, xk, y, fp4_mfma=False, ws_cache=None):
+def _gemv_chunks(wdev, N, kp, fmt, fwht_block, xk, y, fp4_mfma=False, ws_cache=None,
+                 bf16_exact=True):
     f = C.FMT_BY_NAME[fmt]
     # More than one GEMV batch: one GEMM over all rows instead of reading and decoding the
-    # weight once per 16 rows (4096x4096, 17 rows: 9.9 -> 10.7 us; 32: 11.9 -> 11.0; 512: 187
-    # -> 28; 8192->28672, 17 rows: 65 -> 38.5).  The native FP4 option multiplies bf16 x by the
-    # exact weight there too: its two-term split of x pays a pass of its own and saves decode
-    # work that the GEMM hides.
-    if xk.shape[0] > MAX_GEMV_BATCH and kp <= MAX_GEMM_K:
+    # weight once per 16 rows (GF4, GPU time in a graph, GEMV calls -> GEMM: 4096x4096, 17 rows
+    # 10.5 -> 8.9 us, 32 rows 11.6 -> 10.1, 64 rows 22.4 -> 12.0; 1024x4096, 17 rows 7.5 -> 7.5,
+    # the closest of 9 layers of 784->300 to 8192x8192 in either format).  The native FP4 option
+    # multiplies bf16 x by the weight in bf16 there too: its two-term split of x pays a pass of
+    # its own and saves decode work that the GEMM hides (8192x8192, 17 rows: 22.4 -> 11.2).  It
+    # keeps the split where the weight has values beyond bf16's range, which the matrix cores'
+    # FP4 operands do not leave.
+    if (xk.shape[0] > MAX_GEMV_BATCH and kp <= MAX_GEMM_K and not (fp4_mfma and not bf16_exact)):
         C.gemm(wdev, xk, y, C.make_shape(N, kp, xk.shape[0], f, fwht_block,
                                          C.DTYPE_CODE[xk.dtype], C.DTYPE_CODE[y.dtype]))
         return
@@ -216,13 +230,14 @@ class _PackedLinearFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x2, bias, wdev, N, K, fmt, fwht_block, range_check, f16_exact,
-                fp4_mfma=False, ws_cache=None):
+                fp4_mfma=False, ws_cache=None, bf16_exact=True):
         y = None
         if not range_check:
-            y = _native_forward(x2, wdev, N, K, fmt, fwht_block, f16_exact, fp4_mfma, bias)
+            y = _native_forward(x2, wdev, N, K, fmt, fwht_block, f16_exact, fp4_mfma, bias,
+                                bf16_exact)
         if y is None:
             y = _forward(x2, wdev, N, K, fmt, fwht_block, range_check, f16_exact, fp4_mfma,
-                         ws_cache)
+                         ws_cache, bf16_exact)
             if bias is not None:
                 y.add_(bias.to(y.dtype))
         ctx.save_for_backward(wdev)
@@ -242,7 +257,7 @@ class _PackedLinearFn(torch.autograd.Function):
             if fwht_block:
                 gx = _fwht_last_dim(gx, fwht_block)
             gx = gx[:, :K]
-        return gx.to(xdt), None, None, None, None, None, None, None, None, None, None
+        return (gx.to(xdt), *[None] * 11)
 
 
 class _AddedBias(torch.autograd.Function):
@@ -268,12 +283,13 @@ def _native_gradient(gy) -> bool:
     return not torch.is_grad_enabled() and type(gy) is torch.Tensor
 
 
-def _forward(x2, wdev, N, K, fmt, fwht_block, range_check, f16_exact, fp4_mfma, ws_cache):
+def _forward(x2, wdev, N, K, fmt, fwht_block, range_check, f16_exact, fp4_mfma, ws_cache,
+             bf16_exact):
     """y = x2 W^T through torch and ctypes calls, for what the native call does not take."""
     xk = _kernel_input(x2, K, fmt, fwht_block, range_check, f16_exact, fp4_mfma)
     ydt = x2.dtype if x2.dtype in C.DTYPE_CODE else torch.float32
     y = torch.empty(x2.shape[0], N, dtype=ydt, device=x2.device)
-    _gemv_chunks(wdev, N, packed_k(K), fmt, fwht_block, xk, y, fp4_mfma, ws_cache)
+    _gemv_chunks(wdev, N, packed_k(K), fmt, fwht_block, xk, y, fp4_mfma, ws_cache, bf16_exact)
     return y
 
 
@@ -288,19 +304,20 @@ def _vector_bias(bias, N: int) -> bool:
             and unpack_dual(bias).tangent is None)
 
 
-def _native_forward(x, wdev, N, K, fmt, fwht_block, f16_exact, fp4_mfma, bias):
+def _native_forward(x, wdev, N, K, fmt, fwht_block, f16_exact, fp4_mfma, bias, bf16_exact):
     """The whole forward in one native call (fourbit_torch.cpp), or None where x, the weight or
     the bias is not a plain GPU tensor it takes."""
     if type(x) not in _PLAIN or (bias is not None and type(bias) not in _PLAIN):
         return None
     return C.native().linear_forward(x, wdev, N, K, C.FMT_BY_NAME[fmt], fwht_block, f16_exact,
-                                     fp4_mfma, bias)
+                                     fp4_mfma, bias, bf16_exact)
 
 
 def packed_linear(wdev: torch.Tensor, N: int, K: int, fmt: str, fwht_block: int,
                   x: torch.Tensor, bias: torch.Tensor | None = None, *,
                   range_check: bool = False, f16_exact: bool = True,
-                  fp4_mfma: bool = False, ws_cache: dict | None = None) -> torch.Tensor:
+                  fp4_mfma: bool = False, ws_cache: dict | None = None,
+                  bf16_exact: bool | None = None) -> torch.Tensor:
     """``F.linear(x, W, bias)`` for a packed 4-bit ``W [N, K]`` (device stream ``wdev``
     of a ``packed_k(K)``-wide weight): fb_gemv for up to 16 rows of x, fb_gemm for more.
 
@@ -313,14 +330,17 @@ def packed_linear(wdev: torch.Tensor, N: int, K: int, fmt: str, fwht_block: int,
     the caller owns, e.g. one per module; the native call takes its own from the allocator);
     ``f16_exact`` (E2M1 only) says whether the weight's scales decode exactly to fp16.  ``fp4_mfma``
     (unrotated E2M1 only) runs the matrix cores' native FP4 path (fb_gemv_mx) for up to 16 rows
-    (more run fb_gemm on the bf16 x and the exact weight): x as bf16, split into two MX-E4M3
-    terms, which hold a bf16 value exactly unless its 32-value block spans more than E4M3's
-    exponent range (fp16 and fp32 x are rounded to bf16 first).  No CPU path: x must be on the
-    GPU."""
+    (more run fb_gemm on the bf16 x and the weight in bf16 where ``bf16_exact``, whether the
+    weight decodes exactly to bf16, is true; it defaults to ``f16_exact``): x as bf16, split into
+    two MX-E4M3 terms, which hold a bf16 value exactly unless its 32-value block spans more than
+    E4M3's exponent range (fp16 and fp32 x are rounded to bf16 first).  No CPU path: x must be on
+    the GPU."""
+    if bf16_exact is None:
+        bf16_exact = f16_exact
     grad = torch.is_grad_enabled()
     bias_grad = grad and bias is not None and bias.requires_grad
     if not (range_check or bias_grad or (grad and x.requires_grad)):
-        y = _native_forward(x, wdev, N, K, fmt, fwht_block, f16_exact, fp4_mfma, bias)
+        y = _native_forward(x, wdev, N, K, fmt, fwht_block, f16_exact, fp4_mfma, bias, bf16_exact)
         if y is not None:
             return y
     if x.dim() == 0 or x.shape[-1] != K:
@@ -336,7 +356,8 @@ def packed_linear(wdev: torch.Tensor, N: int, K: int, fmt: str, fwht_block: int,
     if grad and x.requires_grad:
         inside = _vector_bias(bias, N)
         y = _PackedLinearFn.apply(x2, bias.detach() if inside else None, wdev, N, K, fmt,
-                                  fwht_block, range_check, f16_exact, fp4_mfma, ws_cache)
+                                  fwht_block, range_check, f16_exact, fp4_mfma, ws_cache,
+                                  bf16_exact)
         if inside and bias_grad:
             y = _AddedBias.apply(y, bias)
         elif bias is not None and not inside:
@@ -345,10 +366,11 @@ def packed_linear(wdev: torch.Tensor, N: int, K: int, fmt: str, fwht_block: int,
     with torch.no_grad():
         y = None
         if not range_check:
-            y = _native_forward(x2, wdev, N, K, fmt, fwht_block, f16_exact, fp4_mfma, None)
+            y = _native_forward(x2, wdev, N, K, fmt, fwht_block, f16_exact, fp4_mfma, None,
+                                bf16_exact)
         if y is None:
             y = _forward(x2, wdev, N, K, fmt, fwht_block, range_check, f16_exact, fp4_mfma,
-                         ws_cache)
+                         ws_cache, bf16_exact)
     if bias is not None:
         if bias_grad:
             y = y + bias.to(y.dtype)
@@ -486,6 +508,8 @@ class PackedWeight:
 class QuantLinear(nn.Linear):
     """4-bit quantized ``nn.Linear`` (reference: ``layers.py:11-45``)."""
 
+    _bf16_exact = None  # of a module pickled without it: packed_linear falls back to _f16_exact
+
     def __init__(self, linear_module: nn.Linear, bitwidth: int = 4, mask=None, *,
                  fmt: str = "gf4", hadamard=False, nthreads: int | None = None,
                  pack: bool = True, packer: str = "host", fp4_mfma: bool = False):
@@ -526,7 +550,7 @@ class QuantLinear(nn.Linear):
         self.range_check = False
         # the Python path's fb_gemv / fb_gemv_mx workspaces of this module, per (device, stream)
         self._ws_cache = {}
-        self._f16_exact = True
+        self._f16_exact = self._bf16_exact = True
         self.register_load_state_dict_post_hook(QuantLinear._rebuild_after_load)
         if pack:
             self.quantize()
@@ -589,7 +613,11 @@ class QuantLinear(nn.Linear):
         self.codes = pw.codes.to(dev)
         self.meta = pw.meta.to(dev)
         self.wdev = pw.wdev.to(dev)
-        self._f16_exact = self.fmt != "e2m1" or e2m1_scales_fit_f16(pw.meta)
+        self._set_exact(pw.meta)
+
+    def _set_exact(self, meta: torch.Tensor) -> None:
+        self._f16_exact, self._bf16_exact = (_scales_fit(meta) if self.fmt == "e2m1"
+                                             else (True, True))
 
     def _shape(self, B=1, x_dtype=torch.float16, y_dtype=torch.float16) -> C.FbShape:
         return C.make_shape(self.out_features, self.k_pack, B, C.FMT_BY_NAME[self.fmt],
@@ -663,7 +691,7 @@ class QuantLinear(nn.Linear):
         else:
             self.wdev = C.to_device_layout(self.codes.cpu(), self.meta.cpu(), shape).to(
                 self.codes.device)
-        self._f16_exact = self.fmt != "e2m1" or e2m1_scales_fit_f16(self.meta)
+        self._set_exact(self.meta)
 
     # -- reference API ------------------------------------------------------------
     def dequantized_weight(self) -> torch.Tensor:
@@ -686,7 +714,7 @@ class QuantLinear(nn.Linear):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         return packed_linear(self.wdev, self.out_features, self.in_features, self.fmt,
                              self.fwht_block, x, self.bias, range_check=self.range_check,
-                             f16_exact=self._f16_exact,
+                             f16_exact=self._f16_exact, bf16_exact=self._bf16_exact,
                              fp4_mfma=self.fp4_mfma, ws_cache=self._ws_cache)
 
     def extra_repr(self) -> str:
@@ -717,13 +745,16 @@ def fp4_mfma_shared(layers, x: torch.Tensor):
     if not x.is_cuda:
         raise RuntimeError("the packed 4-bit linear runs the HIP kernel: move the modules and "
                            "input to a ROCm GPU")
-    # more rows than a GEMV takes run the GEMM, which needs no split of x
-    if x.numel() // K > MAX_GEMV_BATCH and packed_k(K) <= MAX_GEMM_K or (
+    # more rows than a GEMV takes run the GEMM, which needs no split of x, unless a layer's weight
+    # leaves bf16
+    if (x.numel() // K > MAX_GEMV_BATCH and packed_k(K) <= MAX_GEMM_K
+            and all(q._bf16_exact for q in layers)) or (
             torch.is_grad_enabled() and (x.requires_grad or any(
                 q.bias is not None and q.bias.requires_grad for q in layers))):
         return tuple(packed_linear(q.wdev, q.out_features, K, "e2m1", 0, x, q.bias,
                                    range_check=q.range_check, f16_exact=q._f16_exact,
-                                   fp4_mfma=True, ws_cache=q._ws_cache) for q in layers)
+                                   bf16_exact=q._bf16_exact, fp4_mfma=True,
+                                   ws_cache=q._ws_cache) for q in layers)
     lead = x.shape[:-1]
     x2 = x.reshape(-1, K)
     kp = packed_k(K)

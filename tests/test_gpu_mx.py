@@ -318,3 +318,40 @@ def test_gemv_mx_two_streams_match_serial():
     for j in range(2):
         for i in range(5):
             assert torch.equal(outs[j][i], serial[j][i]), (j, i)
+
+
+@pytest.mark.parametrize("top", [252, 253, 254, 255])
+def test_fp4_option_beyond_one_batch_for_every_scale_byte(top):
+    """17 and more rows give what 16-row calls give for E8M0 bytes 0 to 255: up to 252 on the GEMM
+    (the weight is exact in bf16), from 253 on, where 4 and 6 times the scale leave bf16, on the
+    split of x in 16-row batches.  Alone and through fp4_mfma_shared."""
+    from if_i_could_turn_back_time_amd import fp4_mfma_shared
+    N, K, M = 256, 256, 40
+    g = torch.Generator().manual_seed(top)
+    lin = torch.nn.Linear(K, N, bias=False)
+    q = QuantLinear(lin, fmt="e2m1", fp4_mfma=True, pack=False).to(DEV)
+    codes = torch.randint(0, 256, (N, K // 2), generator=g, dtype=torch.uint8)
+    meta = (torch.arange(N)[:, None] % (top + 1)).expand(N, K // 32).to(torch.uint8).contiguous()
+    q.load_state_dict({"codes": codes, "meta": meta, "fb_header": q.fb_header}, strict=False)
+    assert q._bf16_exact == (top <= 252)
+    nib = torch.stack((codes & 15, codes >> 4), dim=-1).reshape(N, K).long()
+    grid = torch.tensor([0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0], dtype=torch.float64)
+    scale64 = torch.exp2(meta.double() - 127).repeat_interleave(32, dim=1)
+    w = (torch.cat((grid, -grid))[nib] * scale64).to(DEV)  # beyond fp32's range at 253 and more
+    nan_rows = (meta[:, 0] == 255).to(DEV)                 # E8M0's NaN
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).to(DEV)
+    for scale in (2.0 ** -100, 1.0, 2.0 ** 60):
+        xs = x * scale
+        with torch.no_grad():
+            ref = torch.cat([q(xs[r:r + 8]) for r in range(0, M, 8)])
+            got = [q(xs), *fp4_mfma_shared([q, q], xs)]
+        mag = xs.double().abs() @ w.abs().t()
+        # where no fp32 sum can overflow (past that, inf - inf depends on the order)
+        live = (mag < 2.0 ** 126) & ~nan_rows
+        assert bool(torch.isfinite(ref[live]).all())
+        for y in got:
+            err = (y.double() - ref.double()).abs()
+            # bf16 results: one of two neighbours (2^-7 of the value, or the smallest subnormal)
+            bound = 2 * ACC_REL * mag + 2.0 ** -7 * ref.double().abs() + 2.0 ** -133
+            assert bool((err <= bound)[live].all())
+            assert bool(torch.isnan(y[:, nan_rows]).all() and torch.isnan(ref[:, nan_rows]).all())

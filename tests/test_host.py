@@ -743,6 +743,21 @@ def test_e2m1_fp16_exact_scale_range():
     assert not PackedWeight.quantize(w, "e2m1").f16_exact
 
 
+@pytest.mark.parametrize("top", [104, 140, 141, 252, 253, 255])
+def test_e2m1_exactness_of_a_loaded_layer(top):
+    """A layer knows from the scales it loads whether they decode exactly to fp16 and to bf16
+    (6 * 2^(s-127) within bf16's range: bytes up to 252)."""
+    assert 6 * 2.0 ** (252 - 127) <= torch.finfo(torch.bfloat16).max < 6 * 2.0 ** (253 - 127)
+    lin = torch.nn.Linear(256, 16)
+    src = QuantLinear(lin, fmt="e2m1").state_dict()
+    src["meta"] = torch.full_like(src["meta"], 110)
+    src["meta"][5, 3] = top
+    q = QuantLinear(lin, fmt="e2m1", pack=False)
+    q.load_state_dict(src)
+    assert q._f16_exact == (top <= 140) and q._bf16_exact == (top <= 252)
+    assert QuantLinear(lin, fmt="gf4")._bf16_exact
+
+
 @pytest.mark.parametrize("block", [2, 16, 256, 4096])
 def test_backward_fwht_matches_oracle(block):
     """The device-side FWHT of the packed linear's backward (torch ops, any device) is
