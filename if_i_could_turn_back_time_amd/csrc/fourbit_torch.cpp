@@ -24,6 +24,7 @@ namespace {
 constexpr int64_t kMaxGemvBatch = 16;
 constexpr int64_t kMaxGemmK = 1 << 22;  // fb_gemm's limits
 constexpr int64_t kMaxGemmRows = 1 << 24;
+constexpr int64_t kMaxRotatedValues = 1 << 29;  // of x, rotated at once: a copy of 1 GiB
 // Rows of grad_y at once: bounds fb_grad_x's 16-bit terms of them, and each pass's decode of W
 // is under 1% of its products.
 constexpr int64_t kGradRows = 8192;
@@ -86,14 +87,15 @@ std::optional<at::Tensor> linear_forward(const at::Tensor& x, const at::Tensor& 
     kdt = FB_DT_BF16;
   if (e2m1 && kdt == FB_DT_F16 && !f16_exact) return std::nullopt;
   const int64_t kp = (K + 127) / 128 * 128, M = x.numel() / K;
-  if (M > kMaxGemmRows || (M > kMaxGemvBatch && kp > kMaxGemmK)) return std::nullopt;
+  if (M > INT32_MAX || (M > kMaxGemvBatch && kp > kMaxGemmK)) return std::nullopt;
   // the GEMM decodes to bf16; the split of more than one GEMV batch is linear.py's
   if (M > kMaxGemvBatch && fp4_mfma && !bf16_exact) return std::nullopt;
 
   fb_shape_t s{};
   s.N = (int32_t)N;
   s.K = (int32_t)kp;
-  s.B = (int32_t)M;
+  s.B = (int32_t)std::min(M, fwht_block ? std::min(kMaxGemmRows, kMaxRotatedValues / kp / 16 * 16)
+                                       : kMaxGemmRows);  // rows of a call
   s.group = e2m1 ? 32 : 128;
   s.fmt = (int32_t)fmt;
   s.fwht_block = (int32_t)fwht_block;
@@ -119,11 +121,16 @@ std::optional<at::Tensor> linear_forward(const at::Tensor& x, const at::Tensor& 
   sizes.back() = N;
   at::Tensor y = at::empty(sizes, x.options());
   if (M > kMaxGemvBatch) {
-    const size_t need = fb_gemm_workspace_bytes(&s);
-    const at::Tensor ws = need ? scratch(need, x) : at::Tensor();
-    check(fb_gemm(wdev.data_ptr(), xk.data_ptr(), y.data_ptr(), &s,
-                  vector_bias ? bias->data_ptr() : nullptr, bdt, ptr_or_null(ws, need), need,
-                  stream));
+    const int64_t step = s.B;
+    for (int64_t r = 0; r < M; r += step) {
+      s.B = (int32_t)std::min(step, M - r);
+      const size_t need = fb_gemm_workspace_bytes(&s);
+      const at::Tensor ws = need ? scratch(need, x) : at::Tensor();
+      check(fb_gemm(wdev.data_ptr(), static_cast<const char*>(xk.data_ptr()) + r * kp * 2,
+                    static_cast<char*>(y.data_ptr()) + r * N * y.element_size(), &s,
+                    vector_bias ? bias->data_ptr() : nullptr, bdt, ptr_or_null(ws, need), need,
+                    stream));
+    }
     if (vector_bias) return y;
   } else if (fp4_mfma) {
     const size_t need = fb_mx_workspace_bytes(&s);

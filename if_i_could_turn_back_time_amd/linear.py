@@ -108,6 +108,15 @@ def _workspace(cache: dict | None, nbytes: int, device: torch.device):
 
 # fb_gemm addresses a tile of x with 32-bit offsets: wider rows run as 16-row GEMV calls.
 MAX_GEMM_K = 1 << 22
+# Rows of x one fb_gemm call takes, and the values of x it may rotate at once (a rotated call
+# holds a 16-bit copy of its rows: 1 GiB); more rows run as several calls.
+MAX_GEMM_ROWS = 1 << 24
+MAX_ROTATED_VALUES = 1 << 29
+
+
+def gemm_rows(kp: int, fwht_block: int) -> int:
+    """Rows of x per fb_gemm call, a multiple of 16."""
+    return min(MAX_GEMM_ROWS, MAX_ROTATED_VALUES // kp // 16 * 16) if fwht_block else MAX_GEMM_ROWS
 
 
 def _gemv_chunks(wdev, N, kp, fmt, fwht_block, xk, y, fp4_mfma=False, ws_cache=None,
@@ -122,8 +131,12 @@ def _gemv_chunks(wdev, N, kp, fmt, fwht_block, xk, y, fp4_mfma=False, ws_cache=N
     # keeps the split where the weight has values beyond bf16's range, which the matrix cores'
     # FP4 operands do not leave.
     if (xk.shape[0] > MAX_GEMV_BATCH and kp <= MAX_GEMM_K and not (fp4_mfma and not bf16_exact)):
-        C.gemm(wdev, xk, y, C.make_shape(N, kp, xk.shape[0], f, fwht_block,
-                                         C.DTYPE_CODE[xk.dtype], C.DTYPE_CODE[y.dtype]))
+        step = gemm_rows(kp, fwht_block)
+        for b0 in range(0, xk.shape[0], step):
+            b1 = min(b0 + step, xk.shape[0])
+            C.gemm(wdev, xk[b0:b1], y[b0:b1],
+                   C.make_shape(N, kp, b1 - b0, f, fwht_block, C.DTYPE_CODE[xk.dtype],
+                                C.DTYPE_CODE[y.dtype]))
         return
     for b0 in range(0, xk.shape[0], MAX_GEMV_BATCH):
         b1 = min(b0 + MAX_GEMV_BATCH, xk.shape[0])
