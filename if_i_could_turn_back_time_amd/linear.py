@@ -695,12 +695,15 @@ class QuantLinear(nn.Linear):
             self.fp4_mfma = False  # the native FP4 path takes unrotated E2M1 weights only
         shape = self._shape()
         # on the GPU where the buffers are (4096x11008 GF4: 15 us instead of a copy to the host,
-        # 16 threads' permutation and a copy back, 10 ms)
+        # 16 threads' permutation and a copy back, 10 ms); views into a larger buffer, which
+        # load_state_dict(assign=True) leaves here, may start anywhere and are copied first
         if (self.codes.is_cuda and self.meta.device == self.codes.device
                 and self.codes.dtype == torch.uint8
                 and self.meta.dtype in (torch.uint8, torch.int16)
                 and self.codes.is_contiguous() and self.meta.is_contiguous()):
-            self.wdev = C.to_device_layout_gpu(self.codes, self.meta, shape)
+            codes, meta = (t if t.data_ptr() % 16 == 0 else t.clone()
+                           for t in (self.codes, self.meta))
+            self.wdev = C.to_device_layout_gpu(codes, meta, shape)
         else:
             self.wdev = C.to_device_layout(self.codes.cpu(), self.meta.cpu(), shape).to(
                 self.codes.device)

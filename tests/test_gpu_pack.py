@@ -67,3 +67,22 @@ def test_checkpoint_loads_to_the_same_stream_on_gpu_and_cpu(kw):
         q.load_state_dict(src.state_dict())
         assert q.wdev.device.type == torch.device(dev).type
         assert torch.equal(q.wdev.cpu(), src.wdev) and q._f16_exact == src._f16_exact
+
+
+@pytest.mark.parametrize("fmt", ["gf4", "e2m1"])
+@pytest.mark.parametrize("offset", [1, 2, 4, 8, 16])
+def test_checkpoint_of_views_loads_at_any_offset(fmt, offset):
+    """load_state_dict(assign=True) keeps views of one flat buffer, at addresses that are no
+    multiple of 16 (codebooks: of 2 at least)."""
+    lin = torch.nn.Linear(300, 70)
+    src = QuantLinear(lin, fmt=fmt)
+    sd = {k: v.to(DEV) for k, v in src.state_dict().items()}
+    for name in ("codes", "meta"):
+        t = sd[name]
+        at = offset * t.element_size()
+        flat = torch.zeros(at + t.numel() * t.element_size(), dtype=torch.uint8, device=DEV)
+        sd[name] = flat[at:].view(t.dtype).view(t.shape).copy_(t)
+    q = QuantLinear(lin, pack=False).to(DEV)
+    q.load_state_dict(sd, assign=True)
+    assert q.codes.data_ptr() % 16 == offset % 16
+    assert torch.equal(q.wdev.cpu(), src.wdev)
