@@ -65,6 +65,11 @@ __device__ __forceinline__ void wait_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
+// Ends a group of requests: the compiler issues no memory operation of one side on the other.
+// wait_barrier's counts are of whole groups (a chunk's x pieces and weights); inside a pipeline
+// its barriers part them, before the first one this does.
+__device__ __forceinline__ void request_group_end() { asm volatile("" ::: "memory"); }
+
 // GF4 decode of one 32-bit word (8 codes, layout order) into 4 fp16 pairs in element
 // order (e0,e1) (e2,e3) (e4,e5) (e6,e7).  tl/th: lo/hi byte-plane tables
 // {A'[0..3], A'[4..7], B'[0..3], B'[4..7]}.

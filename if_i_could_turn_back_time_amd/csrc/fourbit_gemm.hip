@@ -253,6 +253,7 @@ __global__ __launch_bounds__(kGemmWaves * 64, 2) void gemm_kernel(GemmArgs a) {
     for (int c = 0; c < D; ++c) {
       load_nib(sp0, c, nib[c]);
       stage(sp0, c, bufs[c]);
+      request_group_end();
     }
 #pragma unroll
     for (int r = 0; r < RT; ++r) {

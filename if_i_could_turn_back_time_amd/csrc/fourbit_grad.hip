@@ -288,7 +288,10 @@ __global__ __launch_bounds__(kGradWaves * 64, 2) void grad_gemm_kernel(
   if (c0 < c1) {
     load_a(c0, A[0]);
 #pragma unroll
-    for (int c = 0; c < D; ++c) stage(min(c0 + c, c1 - 1), bufs[c]);
+    for (int c = 0; c < D; ++c) {
+      stage(min(c0 + c, c1 - 1), bufs[c]);
+      request_group_end();
+    }
     for (int cb = c0; cb < c1; cb += 4) {
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
