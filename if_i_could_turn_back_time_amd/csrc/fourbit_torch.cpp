@@ -9,6 +9,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/utils/pybind.h>
 
 #include <algorithm>
@@ -199,10 +200,40 @@ std::optional<at::Tensor> linear_grad_bias(const at::Tensor& gy, at::ScalarType 
   return gb;
 }
 
+// y, which holds bias [N] already, as a function of it.  A node of its own, and one that knows
+// which gradients a backward pass asks for: autograd runs a Python function's whole backward for
+// any one of its inputs, so as an input of linear.py's _PackedLinearFn the bias's gradient alone
+// would compute gx too.
+struct AddedBias : torch::autograd::Function<AddedBias> {
+  static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& y,
+                            const at::Tensor& bias) {
+    ctx->mark_dirty({y});
+    ctx->saved_data["dtype"] = bias.scalar_type();
+    return y;
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    const at::Tensor& gy = grads[0];
+    at::Tensor gb;
+    if (ctx->needs_input_grad(1)) {
+      const at::ScalarType bt = ctx->saved_data["dtype"].toScalarType();
+      std::optional<at::Tensor> sums;
+      if (!at::GradMode::is_enabled()) sums = linear_grad_bias(gy, bt);
+      gb = sums ? *sums : gy.sum(0).to(bt);
+    }
+    return {gy, gb};
+  }
+};
+
+at::Tensor added_bias(const at::Tensor& y, const at::Tensor& bias) {
+  return AddedBias::apply(y, bias);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_fourbit_torch, m) {
   m.def("linear_forward", &linear_forward);
   m.def("linear_grad_x", &linear_grad_x);
   m.def("linear_grad_bias", &linear_grad_bias);
+  m.def("added_bias", &added_bias);
 }

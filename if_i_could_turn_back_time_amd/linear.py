@@ -262,7 +262,8 @@ class _PackedLinearFn(torch.autograd.Function):
         (wdev,) = ctx.saved_tensors
         N, K, fmt, fwht_block, xdt, f16_exact = ctx.cfg
         gx = None
-        if _native_gradient(gy) and N <= MAX_GRAD_N:
+        # not where autograd records operations on grad_y (a gradient to be differentiated)
+        if not torch.is_grad_enabled() and type(gy) is torch.Tensor and N <= MAX_GRAD_N:
             gx = C.native().linear_grad_x(gy, wdev, N, K, C.FMT_BY_NAME[fmt], fwht_block, f16_exact,
                                           xdt if xdt in C.DTYPE_CODE else torch.float32)
         if gx is None:
@@ -271,29 +272,6 @@ class _PackedLinearFn(torch.autograd.Function):
                 gx = _fwht_last_dim(gx, fwht_block)
             gx = gx[:, :K]
         return (gx.to(xdt), *[None] * 11)
-
-
-class _AddedBias(torch.autograd.Function):
-    """y, which holds the bias already, as a function of the bias.  A node of its own because
-    autograd runs a function's whole backward for any one of its inputs: as part of
-    _PackedLinearFn, asking for the bias's gradient alone would compute grad_x too."""
-
-    @staticmethod
-    def forward(ctx, y, bias):
-        ctx.mark_dirty(y)
-        ctx.bias_dtype = bias.dtype
-        return y
-
-    @staticmethod
-    def backward(ctx, gy):
-        gb = C.native().linear_grad_bias(gy, ctx.bias_dtype) if _native_gradient(gy) else None
-        return gy, gy.sum(0).to(ctx.bias_dtype) if gb is None else gb
-
-
-def _native_gradient(gy) -> bool:
-    """Whether a native call may compute from grad_y: not where autograd records operations on
-    it (a gradient to be differentiated)."""
-    return not torch.is_grad_enabled() and type(gy) is torch.Tensor
 
 
 def _forward(x2, wdev, N, K, fmt, fwht_block, range_check, f16_exact, fp4_mfma, ws_cache,
@@ -310,8 +288,8 @@ _PLAIN = (torch.Tensor, nn.Parameter)
 
 
 def _vector_bias(bias, N: int) -> bool:
-    """Whether bias is an ordinary [N] vector, which the kernels add and _AddedBias
-    differentiates.  Any other one (a row per row of x, a single value, one with a forward-mode
+    """Whether bias is an ordinary [N] vector, which the kernels add and added_bias
+    (fourbit_torch.cpp) differentiates.  Any other one (a row per row of x, a single value, one with a forward-mode
     tangent) broadcasts against the [M, N] product as a torch operation."""
     return (type(bias) in _PLAIN and bias.dim() == 1 and bias.shape[0] == N
             and unpack_dual(bias).tangent is None)
@@ -372,7 +350,7 @@ def packed_linear(wdev: torch.Tensor, N: int, K: int, fmt: str, fwht_block: int,
                                   fwht_block, range_check, f16_exact, fp4_mfma, ws_cache,
                                   bf16_exact)
         if inside and bias_grad:
-            y = _AddedBias.apply(y, bias)
+            y = C.native().added_bias(y, bias)
         elif bias is not None and not inside:
             y = y + bias.to(y.dtype)
         return y.reshape(*lead, N)

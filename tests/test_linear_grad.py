@@ -39,7 +39,7 @@ def dev(request, monkeypatch):
         monkeypatch.setattr(LN, "_forward", forward)
         monkeypatch.setattr(C, "dequant_device", _dequant_cpu)
         monkeypatch.setattr(C, "_native", SimpleNamespace(
-            linear_forward=declines, linear_grad_x=declines, linear_grad_bias=declines))
+            linear_forward=declines, linear_grad_x=declines, added_bias=C.native().added_bias))
     return request.param
 
 
@@ -142,7 +142,7 @@ def test_gradient_of_the_bias_alone(dev, M, monkeypatch):
     calls = []
     native = C.native()
     monkeypatch.setattr(C, "_native", SimpleNamespace(
-        linear_forward=native.linear_forward, linear_grad_bias=native.linear_grad_bias,
+        linear_forward=native.linear_forward, added_bias=native.added_bias,
         linear_grad_x=lambda *a: calls.append("native") or native.linear_grad_x(*a)))
     decode = C.dequant_device
     monkeypatch.setattr(C, "dequant_device", lambda *a, **k: calls.append("decode") or decode(*a, **k))
