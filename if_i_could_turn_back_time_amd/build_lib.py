@@ -141,9 +141,13 @@ def build(verbose: bool = False) -> Path:
     caller = [_hipcc(), *HIP_FLAGS, f"-I{INCLUDE}", str(C_TESTS / "abi_gpu.cpp"), "-o",
               str(C_TESTS / "abi_gpu"), f"-L{PKG}", "-l:libfourbit.so",
               "-Wl,-rpath,$ORIGIN/../../if_i_could_turn_back_time_amd"]
-    if verbose:
-        print(" ".join(caller), flush=True)
-    _run(caller)
+    # and the mask of a Jenks split at any position, which the library's entry points do not take
+    ties = [_hipcc(), *HIP_FLAGS, "-shared", str(C_TESTS / "jenks2_ties.hip"), "-o",
+            str(C_TESTS / "jenks2_ties.so")]
+    for cmd in (caller, ties):
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        _run(cmd)
     return LIB
 
 

@@ -346,8 +346,8 @@ int fb_jenks2_workspace(int64_t n, size_t* bytes);
 
 /* GPU version of fb_jenks2_host, bit-identical outputs.  w, keep, split, gvf and ws are
  * device pointers (ws 256-byte aligned, at least fb_jenks2_workspace(n) bytes); asynchronous
- * on the stream.  Non-finite values are not detected here (fb_jenks2_host rejects them with
- * FB_ERR_VALUE), so callers check first. */
+ * on the stream.  Where fb_jenks2_host rejects non-finite values with FB_ERR_VALUE, gvf comes out
+ * NaN here (finite values never give NaN) and the split, in [0, n), and the mask mean nothing. */
 int fb_jenks2_gpu(const float* w, int64_t n, uint8_t* keep, int64_t* split, double* gvf,
                   void* ws, size_t ws_bytes, void* stream);
 

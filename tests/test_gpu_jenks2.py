@@ -248,3 +248,111 @@ def test_jenks2_ssd_filters_gpu_bit_exact(dtype):
         assert np.array_equal(g.view(np.uint8), host.view(np.uint8))
         for f in range(0, nf, max(1, nf // 25)):
             assert np.array_equal(g[f], O.jenks2_ssd(w[f]).astype(npdt)), (nf, n, f)
+
+
+# ---------------------------------------------------------------- the mask at any split
+def _ties_lib():
+    import ctypes
+    from pathlib import Path
+    path = Path(__file__).resolve().parent / "c" / "jenks2_ties.so"
+    assert path.exists(), "tests/c/jenks2_ties.so is not built: run __graft_entry__.build()"
+    L = ctypes.CDLL(str(path))
+    L.ties_scratch_bytes.restype = ctypes.c_int64
+    L.ties_scratch_bytes.argtypes = [ctypes.c_int64]
+    L.ties_mask.argtypes = [ctypes.c_void_p, ctypes.c_int64] + [ctypes.c_void_p] * 5
+    return L
+
+
+def _mask_at(L, w, srt, split, shift=0):
+    n = w.size
+    wd = torch.empty(n + shift, dtype=torch.float32, device=DEV)[shift:]
+    wd.copy_(torch.from_numpy(w))
+    keep = torch.full((n + shift + 8,), 7, dtype=torch.uint8, device=DEV)
+    scratch = torch.full((L.ties_scratch_bytes(n),), 255, dtype=torch.uint8, device=DEV)
+    sd = torch.from_numpy(srt).to(DEV)
+    sp = torch.tensor([split], dtype=torch.int64, device=DEV)
+    assert L.ties_mask(wd.data_ptr(), n, sd.data_ptr(), sp.data_ptr(), keep[shift:].data_ptr(),
+                       scratch.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
+    out = keep.cpu().numpy()
+    assert (out[:shift] == 7).all() and (out[shift + n:] == 7).all()
+    return out[shift:shift + n]
+
+
+# segments of 16384 values are counted one by one; n around their edges, and many of them
+@pytest.mark.parametrize("n", [1, 2, 5, 16383, 16384, 16385, 32768, 49152 + 7, 300001])
+@pytest.mark.parametrize("kind", ["few values", "zeros", "constant", "clustered", "distinct"])
+def test_mask_of_a_split_inside_equal_values(n, kind):
+    """At every kind of position (first, inside and last of a run of equal values, -0.0 and +0.0
+    among them) the mask is that of the stable ascending order."""
+    say("mask", n, kind)
+    L = _ties_lib()
+    rng = np.random.default_rng(n)
+    if kind == "few values":
+        w = rng.integers(-2, 3, n).astype(np.float32) / 4
+        w[rng.random(n) < 0.3] = -0.0
+    elif kind == "zeros":  # nearly all zeros of either sign
+        w = np.where(rng.random(n) < 0.01, rng.standard_normal(n), 0.0).astype(np.float32)
+        w[rng.random(n) < 0.5] *= -1
+    elif kind == "constant":
+        w = np.full(n, -0.125, np.float32)
+    elif kind == "clustered":  # the equal values in a few neighbouring places
+        w = rng.standard_normal(n).astype(np.float32)
+        for c in (0, 16380, 16384, n - 3):
+            w[max(0, min(c, n)):max(0, min(c + 9, n))] = 0.5
+    else:
+        w = rng.permutation(n).astype(np.float32) - n // 2
+    order = np.argsort(w, kind="stable")
+    srt = w[order]
+    runs = np.flatnonzero(np.r_[True, srt[1:] != srt[:-1]])  # -0.0 == 0.0
+    ends = np.r_[runs[1:], n]
+    longest = np.argsort(ends - runs)[-4:]
+    splits = {0, n - 1, n // 2}
+    for r in longest:
+        a, b = int(runs[r]), int(ends[r])
+        splits |= {a, min(a + 1, b - 1), (a + b) // 2, b - 1, int(rng.integers(a, b))}
+        # the first kept one at a segment's edge in index order
+        idx = order[a:b]
+        for edge in (16383, 16384, 32767, 32768, (n - 1) // 16384 * 16384):
+            p = int(np.searchsorted(idx, edge))
+            if p < b - a:
+                splits.add(a + p)
+    for split in sorted(splits):
+        ref = np.zeros(n, np.uint8)
+        ref[order[split:]] = 1
+        assert np.array_equal(_mask_at(L, w, srt, split), ref), split
+    # the sort by key bits has -0.0 before +0.0; and pointers that allow no 4-value accesses
+    bits = np.sort(w.view(np.int32) ^ ((w.view(np.int32) >> 31) & 0x7FFFFFFF))
+    by_bits = (bits ^ ((bits >> 31) & 0x7FFFFFFF)).view(np.float32)
+    for shift in (1, 2, 3):
+        assert np.array_equal(_mask_at(L, w, by_bits, split, shift), ref)
+
+
+@pytest.mark.parametrize("n", [1, 2, 257, 65537])
+@pytest.mark.parametrize("bad", [(np.inf,), (-np.inf,), (np.inf, -np.inf), (np.nan,), (-np.nan,),
+                                 (np.inf, np.nan)])
+def test_jenks2_gpu_rejects_nonfinite(n, bad):
+    """Wherever they stand, infinities and NaN raise, as on the host; the largest finite values do
+    not."""
+    rng = np.random.default_rng(n)
+    for at in {0, n // 2, n - 1}:
+        w = rng.standard_normal(n).astype(np.float32)
+        for i, v in enumerate(bad):
+            w[(at + i) % n] = v
+        for fn in (C.jenks2_gpu, linear_mask, bias_mask):
+            with pytest.raises(RuntimeError):
+                fn(torch.from_numpy(w).to(DEV))
+        with pytest.raises(RuntimeError):
+            C.jenks2_host(torch.from_numpy(w))
+    w = np.where(rng.random(n) < 0.5, 3.4028234e38, -3.4028234e38).astype(np.float32)
+    kh, sh, gh = C.jenks2_host(torch.from_numpy(w))
+    kg, sg, gg = C.jenks2_gpu(torch.from_numpy(w).to(DEV))
+    assert sg == sh and gg == gh and torch.equal(kg.cpu(), kh)
+
+
+@pytest.mark.parametrize("n", [3, 255, 65537])
+def test_jenks2_gpu_takes_any_address(n):
+    """A view that starts 4 bytes into its buffer."""
+    w = torch.randn(n + 1) * 0.02
+    kh, sh, gh = C.jenks2_host(w[1:].contiguous())
+    kg, sg, gg = C.jenks2_gpu(w.to(DEV)[1:])
+    assert sg == sh and gg == gh and torch.equal(kg.cpu(), kh)
