@@ -42,7 +42,8 @@ EXPORTED = (
     "fb_jenks2_ssd_host", "fb_jenks2_ssd_workspace", "fb_jenks2_ssd_gpu",
     "fb_jenks2_ssd_filters_host", "fb_jenks2_ssd_filters_gpu",
     "fb_gemm", "fb_gemm_workspace_bytes", "fb_grad_x", "fb_grad_x_workspace_bytes",
-    "fb_to_device_gpu", "fb_cast_rows", "fb_add_bias", "fb_grad_bias",
+    "fb_to_device_gpu", "fb_cast_rows", "fb_add_bias", "fb_grad_bias", "fb_grad_bias_ws",
+    "fb_grad_bias_workspace_bytes",
 )
 
 
@@ -88,6 +89,8 @@ def lib() -> ctypes.CDLL:
         "fb_grad_x_workspace_bytes": (sz, [sp, i32]),
         "fb_add_bias": (ctypes.c_int, [vp, i32, i32, i32, vp, i32, vp]),
         "fb_grad_bias": (ctypes.c_int, [vp, i32, i32, i32, vp, i32, vp]),
+        "fb_grad_bias_ws": (ctypes.c_int, [vp, i32, i32, i32, vp, i32, vp, sz, vp]),
+        "fb_grad_bias_workspace_bytes": (sz, [i32, i32]),
         "fb_cast_rows": (ctypes.c_int, [vp, i32, i32, i32, vp, i32, i32, vp]),
         "fb_dequant": (ctypes.c_int, [vp, vp, i32, sp, vp]),
         "fb_quantize_gf4_gpu": (ctypes.c_int, [vp, vp, i32, i32, vp, vp, vp]),

@@ -420,9 +420,108 @@ __global__ __launch_bounds__(1024) void grad_bias_kernel(const void* __restrict_
   }
 }
 
+// The same for many rows: column sums of a run of rows per workgroup, for grad_bias_kernel (or
+// another of this) to add.  gy is read as m rows of W = q N values, so that 8 values of 16 bytes
+// (fp32: 32) per lane fill a workgroup's 512 columns whatever N is; the workgroup's waves take
+// every 4th of its R rows, and their sums are added in order through LDS.  The rows past m q, less
+// than W values, go to the sums as they are.  Bound by memory.
+template <int DT>
+__global__ __launch_bounds__(256) void grad_bias_part_kernel(const void* __restrict__ gy, int64_t m,
+                                                             int64_t W, int64_t R, int64_t tail,
+                                                             int P, int vec,
+                                                             float* __restrict__ part) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t b0 = (int64_t)blockIdx.x * 512;
+  if ((int)blockIdx.y == P) {
+    for (int64_t c = b0 + threadIdx.x; c < b0 + 512 && c < tail; c += 256)
+      part[(int64_t)P * W + c] = load_as_float(gy, m * W + c, DT);
+    return;
+  }
+  __shared__ __align__(16) float l[4][512];
+  const int64_t c0 = b0 + lane * 8;  // W % 8 == 0
+  const int64_t r0 = (int64_t)blockIdx.y * R, r1 = min(m, r0 + R);
+  float a[8] = {};
+  auto add = [&](int64_t at) {
+    if (!vec) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) a[e] += load_as_float(gy, at + e, DT);
+    } else if constexpr (DT == FB_DT_F32) {
+      const f32x4* p = reinterpret_cast<const f32x4*>(static_cast<const float*>(gy) + at);
+      const f32x4 x = p[0], y = p[1];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        a[e] += x[e];
+        a[4 + e] += y[e];
+      }
+    } else {
+      const u32x4 v = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(gy) + at);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const unsigned short h = (unsigned short)(v[e >> 1] >> (16 * (e & 1)));
+        a[e] += DT == FB_DT_F16 ? (float)__builtin_bit_cast(_Float16, h)
+                                : (float)__builtin_bit_cast(__bf16, h);
+      }
+    }
+  };
+  if (c0 < W) {
+#pragma unroll 8
+    for (int64_t r = r0 + wave; r < r1; r += 4) add(r * W + c0);
+  }
+  *reinterpret_cast<f32x4*>(&l[wave][lane * 8]) = f32x4{a[0], a[1], a[2], a[3]};
+  *reinterpret_cast<f32x4*>(&l[wave][lane * 8 + 4]) = f32x4{a[4], a[5], a[6], a[7]};
+  __syncthreads();
+  for (int c = threadIdx.x; c < 512 && b0 + c < W; c += 256)
+    part[(int64_t)blockIdx.y * W + b0 + c] = ((l[0][c] + l[1][c]) + l[2][c]) + l[3][c];
+}
+
 // ---------------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------------
+// Whether grad_bias_kernel sums a gradient by itself.  Measured (us, one launch / parts; fp16 unless
+// said): 2048 x 48 7.1 / 8.1, 4096 x 48 12.5 / 7.7, 2^18 x 48 1423 / 12 (torch's sum 25), 1024 x 4096
+// 5.6 / 7.9, 1025 x 11008 18.0 / 8.6, 65536 x 4096 545 / 93 (torch 113), 16384 x 28672 fp32 589 / 339.
+bool bias_alone(int64_t M, int64_t N) {
+  return M <= 2048 && (M <= 64 || M * N <= (6 << 20));
+}
+
+// One pass of grad_bias_part_kernel over M rows of N values.
+struct BiasParts {
+  int64_t q, m, W, R;
+  int P;
+  int64_t rows;  // of the sums it leaves
+};
+BiasParts bias_parts(int64_t M, int64_t N) {
+  BiasParts b;
+  b.q = N >= 64 ? 8 : 512 / N / 8 * 8;
+  b.m = M / b.q;
+  b.W = b.q * N;
+  // About four workgroups of 256 threads per CU, of 32 rows at least (8 per wave in flight) and
+  // 1024 at most (256 additions in a row, whatever M is).
+  const int64_t wide = (b.W + 511) / 512;
+  const int64_t fill = std::min((1024 + wide - 1) / wide, (b.m + 31) / 32);
+  b.P = (int)std::min<int64_t>(std::max(fill, (b.m + 1023) / 1024), 65000);  // the grid's y range
+  b.R = (b.m + b.P - 1) / b.P;
+  b.rows = b.P * b.q + (M - b.m * b.q);
+  return b;
+}
+
+int launch_bias_parts(const void* gy, int dt, int64_t M, int64_t N, const BiasParts& b, float* part,
+                      hipStream_t hs) {
+  const int64_t tail = (M - b.m * b.q) * N;
+  const dim3 grid((unsigned)((b.W + 511) / 512), (unsigned)(b.P + (tail ? 1 : 0)));
+  const int vec = (reinterpret_cast<uintptr_t>(gy) & 15u) == 0;
+  if (dt == FB_DT_F32)
+    hipLaunchKernelGGL(grad_bias_part_kernel<FB_DT_F32>, grid, dim3(256), 0, hs, gy, b.m, b.W, b.R,
+                       tail, b.P, vec, part);
+  else if (dt == FB_DT_F16)
+    hipLaunchKernelGGL(grad_bias_part_kernel<FB_DT_F16>, grid, dim3(256), 0, hs, gy, b.m, b.W, b.R,
+                       tail, b.P, vec, part);
+  else
+    hipLaunchKernelGGL(grad_bias_part_kernel<FB_DT_BF16>, grid, dim3(256), 0, hs, gy, b.m, b.W, b.R,
+                       tail, b.P, vec, part);
+  return hipGetLastError() == hipSuccess ? FB_OK : FB_ERR_HIP;
+}
+
 constexpr int64_t kMaxOperandBytes = 256ll << 20;  // transposed weight held at once
 constexpr int kMaxRowsW = 1 << 18;  // one span of these is 256 MiB of 16-bit operands per plane
 constexpr int64_t kMaxPartBytes = 256ll << 20;
@@ -640,6 +739,42 @@ int grad_run(const GradPlan& pl, const fb_shape_t* s, const void* wdev, const vo
 }  // namespace
 
 extern "C" {
+
+size_t fb_grad_bias_workspace_bytes(int32_t M, int32_t N) {
+  if (M < 1 || N < 1) return 0;
+  size_t bytes = 0;
+  for (int64_t rows = M; !bias_alone(rows, N);) {
+    rows = bias_parts(rows, N).rows;
+    bytes += align256((size_t)rows * N * 4);
+  }
+  return bytes;
+}
+
+int fb_grad_bias_ws(const void* gy, int32_t gy_dtype, int32_t M, int32_t N, void* gb,
+                    int32_t gb_dtype, void* ws, size_t ws_bytes, void* stream) {
+  if (!gy || !gb) return FB_ERR_NULL;
+  if (M < 1 || N < 1) return FB_ERR_SHAPE;
+  for (int32_t d : {gy_dtype, gb_dtype})
+    if (d != FB_DT_F16 && d != FB_DT_BF16 && d != FB_DT_F32) return FB_ERR_DTYPE;
+  if (reinterpret_cast<uintptr_t>(gy) & (gy_dtype == FB_DT_F32 ? 3u : 1u)) return FB_ERR_ALIGN;
+  const size_t need = fb_grad_bias_workspace_bytes(M, N);
+  if (need && !ws) return FB_ERR_NULL;
+  if (need && (reinterpret_cast<uintptr_t>(ws) & 255u)) return FB_ERR_ALIGN;
+  if (need > ws_bytes) return FB_ERR_WORKSPACE;
+  uint8_t* at = static_cast<uint8_t*>(ws);
+  int64_t rows = M;
+  while (!bias_alone(rows, N)) {
+    const BiasParts b = bias_parts(rows, N);
+    const int st = launch_bias_parts(gy, gy_dtype, rows, N, b, reinterpret_cast<float*>(at),
+                                     static_cast<hipStream_t>(stream));
+    if (st != FB_OK) return st;
+    gy = at;
+    gy_dtype = FB_DT_F32;
+    rows = b.rows;
+    at += align256((size_t)rows * N * 4);
+  }
+  return fb_grad_bias(gy, gy_dtype, (int32_t)rows, N, gb, gb_dtype, stream);
+}
 
 int fb_grad_bias(const void* gy, int32_t gy_dtype, int32_t M, int32_t N, void* gb,
                  int32_t gb_dtype, void* stream) {

@@ -195,8 +195,11 @@ std::optional<at::Tensor> linear_grad_bias(const at::Tensor& gy, at::ScalarType 
   c10::DeviceGuard guard(gy.device());
   const at::Tensor g = gy.contiguous();
   at::Tensor gb = at::empty({gy.size(1)}, gy.options().dtype(bt));
-  check(fb_grad_bias(g.data_ptr(), gdt, (int32_t)gy.size(0), (int32_t)gy.size(1), gb.data_ptr(),
-                     bdt, stream_of(gy)));
+  const int32_t M = (int32_t)gy.size(0), N = (int32_t)gy.size(1);
+  const size_t need = fb_grad_bias_workspace_bytes(M, N);
+  const at::Tensor ws = need ? scratch(need, gy) : at::Tensor();
+  check(fb_grad_bias_ws(g.data_ptr(), gdt, M, N, gb.data_ptr(), bdt, ptr_or_null(ws, need), need,
+                        stream_of(gy)));
   return gb;
 }
 

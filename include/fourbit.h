@@ -282,6 +282,14 @@ int fb_grad_x(const void* wdev, const void* gy, void* gx, const fb_shape_t* s, i
 int fb_grad_bias(const void* gy, int32_t gy_dtype, int32_t M, int32_t N, void* gb,
                  int32_t gb_dtype, void* stream);
 
+/* fb_grad_bias for any number of rows: many (more than 2048, or more than 6 Mi values) are summed in
+ * parts side by side (fp32, a fixed order), which need a device workspace ws, 256-byte aligned, of
+ * fb_grad_bias_workspace_bytes(M, N) bytes (0: none used).  Its contents need no initialisation;
+ * calls that share it must not overlap. */
+int fb_grad_bias_ws(const void* gy, int32_t gy_dtype, int32_t M, int32_t N, void* gb,
+                    int32_t gb_dtype, void* ws, size_t ws_bytes, void* stream);
+size_t fb_grad_bias_workspace_bytes(int32_t M, int32_t N);
+
 /* Workspace bytes of fb_grad_x for this shape on the current device (0: a shape it does not
  * take). */
 size_t fb_grad_x_workspace_bytes(const fb_shape_t* s, int32_t f16_exact);

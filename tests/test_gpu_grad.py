@@ -141,6 +141,48 @@ def test_grad_bias(gdt, M, N):
     assert gq.dtype == q.bias.dtype and torch.equal(gq, gb)
 
 
+@pytest.mark.parametrize("gdt", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N", [
+    (2048, 48), (2049, 48), (2049, 1), (3071, 1), (3073, 2), (4095, 7), (4099, 63), (4096, 64),
+    (4103, 65), (9000, 300), (70001, 513), (1 << 18, 48), ((1 << 20) + 3, 1), (1 << 20, 24),
+    (12345, 4096), (64, 98305), (65, 98305), (600, 11008), (1537, 4099)])
+def test_grad_bias_of_many_rows(gdt, M, N):
+    """More than 2048 rows, or 6 Mi values, are summed in parts: at most 256 additions in a row in
+    the first pass, 8 in the others and 96 in the last, so at most 400 roundings whatever M is."""
+    print("grad bias", gdt, M, N, flush=True)
+    buf = torch.full((M * N + 8192,), float("nan"), dtype=gdt, device=DEV)
+    for shift in (4096, 4097):  # 16-byte aligned or not, NaN around
+        gy = buf[shift:shift + M * N].view(M, N)
+        gy.normal_()
+        gb = C.native().linear_grad_bias(gy, torch.float32)
+        ref = gy.double().sum(0)
+        assert bool(((gb.double() - ref).abs() <= 400 * 2.0 ** -24 * gy.double().abs().sum(0)).all())
+        assert torch.equal(gb, C.native().linear_grad_bias(gy, torch.float32))
+        half = C.native().linear_grad_bias(gy, torch.float16)
+        assert torch.equal(half, gb.half())
+        gy.fill_(float("nan"))
+
+
+def test_grad_bias_workspace_contract():
+    L = C.lib()
+    assert L.fb_grad_bias_workspace_bytes(2048, 300) == 0 == L.fb_grad_bias_workspace_bytes(0, 1)
+    assert L.fb_grad_bias_workspace_bytes(64, 1 << 20) == 0 < L.fb_grad_bias_workspace_bytes(65, 1 << 20)
+    need = L.fb_grad_bias_workspace_bytes(5000, 300)
+    gy = torch.randn(5000, 300, device=DEV)
+    gb = torch.empty(300, device=DEV)
+    ws = torch.empty(need + 256, dtype=torch.uint8, device=DEV)
+    s = torch.cuda.current_stream().cuda_stream
+
+    def rc(ws_ptr, nbytes, g=gy.data_ptr(), dt=C.DT_F32, M=5000):
+        return L.fb_grad_bias_ws(g, dt, M, 300, gb.data_ptr(), C.DT_F32, ws_ptr, nbytes, s)
+
+    assert rc(None, 0) == -1 and rc(ws.data_ptr() + 16, need) == -7
+    assert rc(ws.data_ptr(), need - 1) == -8
+    assert rc(ws.data_ptr(), need, g=None) == -1 and rc(ws.data_ptr(), need, dt=3) == -5
+    assert rc(ws.data_ptr(), need, g=gy.data_ptr() + 2) == -7 and rc(None, 0, M=0) == -2
+    assert rc(ws.data_ptr(), need) == 0 and rc(None, 0, M=2048) == 0
+
+
 @pytest.mark.parametrize("ydt", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,N", [(1, 300), (3, 77), (16, 4096)])
 def test_gemv_bias_is_the_in_place_add(ydt, M, N):
