@@ -242,8 +242,11 @@ class _PackedLinearFn(torch.autograd.Function):
     operations on W decoded in chunks of row tiles (``_grad_x``)."""
 
     @staticmethod
-    def forward(ctx, x2, bias, wdev, N, K, fmt, fwht_block, range_check, f16_exact,
-                fp4_mfma=False, ws_cache=None, bf16_exact=True):
+    def forward(ctx, x2, constants):
+        """``constants``: bias, then packed_linear's arguments from wdev on, as one tuple (autograd
+        looks at each argument of its own, 0.2 us apiece)."""
+        (bias, wdev, N, K, fmt, fwht_block, range_check, f16_exact, fp4_mfma, ws_cache,
+         bf16_exact) = constants
         y = None
         if not range_check:
             y = _native_forward(x2, wdev, N, K, fmt, fwht_block, f16_exact, fp4_mfma, bias,
@@ -271,7 +274,7 @@ class _PackedLinearFn(torch.autograd.Function):
             if fwht_block:
                 gx = _fwht_last_dim(gx, fwht_block)
             gx = gx[:, :K]
-        return (gx.to(xdt), *[None] * 11)
+        return gx.to(xdt), None
 
 
 def _forward(x2, wdev, N, K, fmt, fwht_block, range_check, f16_exact, fp4_mfma, ws_cache,
@@ -346,9 +349,8 @@ def packed_linear(wdev: torch.Tensor, N: int, K: int, fmt: str, fwht_block: int,
     x2 = x.reshape(-1, K)
     if grad and x.requires_grad:
         inside = _vector_bias(bias, N)
-        y = _PackedLinearFn.apply(x2, bias.detach() if inside else None, wdev, N, K, fmt,
-                                  fwht_block, range_check, f16_exact, fp4_mfma, ws_cache,
-                                  bf16_exact)
+        y = _PackedLinearFn.apply(x2, (bias if inside else None, wdev, N, K, fmt, fwht_block,
+                                       range_check, f16_exact, fp4_mfma, ws_cache, bf16_exact))
         if inside and bias_grad:
             y = C.native().added_bias(y, bias)
         elif bias is not None and not inside:
