@@ -19,7 +19,7 @@
 //    tiles are separate scheduling regions, so that the instruction stream alternates the two
 //    (left to itself the compiler groups them, and a wave then waits for its own MFMAs).
 // What bounds it: E2M1 runs at the matrix cores' power-limited rate (8192 -> 28672, M = 2048:
-// 635 us, 1515 TFLOP/s; the library's bf16 GEMM of 8192^3 reaches 1418 on the same card; one
+// 621 to 635 us, 1,515 to 1,549 TFLOP/s; the library's bf16 GEMM of 8192^3 reaches 1418 on the same card; one
 // workgroup of wider staging per CU: 737 us); GF4 issues nearly as many cycles of decode and MFMA
 // instructions as its MFMAs take (964 us, 998 TFLOP/s; 16-row GEMV calls: 4840 us; one workgroup
 // per CU: 1006).  Small M is bound by latency and the x fill of each CU; the K range is then
@@ -411,9 +411,10 @@ __global__ __launch_bounds__(256) void cast_rows_kernel(const void* __restrict__
 // ---------------------------------------------------------------------------------
 // Tile shapes the plan chooses from, with the time in us that a span (512 K-values) of one
 // tile takes on a CU when one workgroup runs there and when two do (both done).  Fitted to
-// 6,000 timings of every shape and part count over M = 17..2048 on 4096^2, 8192^2, 4096 ->
-// 11008, 11008 -> 4096 and 8192 -> 28672; the plan it picks is within 1.1% (geometric mean; 12%
-// at worst) of the best one timed.  A table rather than a formula because the costs follow no
+// timings of every shape and part count over M = 17..2048 on 4096^2, 8192^2, 4096 -> 11008,
+// 11008 -> 4096 and 8192 -> 28672.  Timed again with every shape and part count on those and on
+// 1024^2 and 896 -> 300 (126 cases, profiles/gemm_plan_vs_all_tiles.md): the plan it picks is
+// 0.6% (geometric mean; 9.4% at worst) from the best.  A table rather than a formula because the costs follow no
 // simple one: small tiles are bound by latency and the x fill, GF4's wide ones by instruction
 // issue (RT = 4 does not fit two workgroups' registers there), E2M1's by the MFMAs.
 struct GemmShape {

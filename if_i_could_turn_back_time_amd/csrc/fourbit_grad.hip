@@ -530,9 +530,11 @@ constexpr int kMaxParts = 8;
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 
 // Tile shapes with the time in us that a chunk (128 contraction values) of one tile takes on a
-// CU when one workgroup runs there and when two do.  Fitted to 2,900 timings of these and of six
-// other shapes at every part count, over M = 17..1024, 1 to 6 term pairs and 5 layers of 1024 ->
-// 2048 to 8192^2; the plan it picks is within 2.9% (geometric mean; 19% at worst) of the best.
+// CU when one workgroup runs there and when two do.  Fitted to timings of these and of six other
+// shapes at every part count, over M = 17..1024, 1 to 6 term pairs and 5 layers of 1024 -> 2048 to
+// 8192^2.  Timed again with every shape and part count (80 cases of 4096^2 to 8192 -> 28672,
+// profiles/gemm_plan_vs_all_tiles.md): the whole call on the plan it picks is 1.6% (geometric
+// mean; 11.6% at worst) from the best.
 struct GradShape {
   int rt, ct;
   float one, two;
