@@ -1,8 +1,8 @@
 // The packed linear layer's call path from torch: one native call per forward (and per activation
 // gradient) instead of a dozen Python, ctypes and dispatcher steps.  It launches the kernels that
 // linear.py's packed_linear launches, on x converted as there, and takes workspaces from the
-// allocator; what it does not recognise (another dtype, a refused shape, a wrapped tensor, a bias
-// that is no vector or has a forward-mode tangent, an active dispatch mode) it leaves to
+// allocator; what it does not recognise (another dtype, a refused shape, a wrapped tensor or one
+// with a forward-mode tangent, a bias that is no vector, an active dispatch mode) it leaves to
 // packed_linear by returning None.  A decode call of a 4096^2 layer takes 5 us on the GPU and took
 // 22 us of host time through Python.
 #include <ATen/ATen.h>
@@ -39,15 +39,16 @@ int dtype_code(at::ScalarType t) {
 }
 
 // A plain dense GPU tensor whose memory this code may read: no functorch wrapper, fake or
-// functional tensor, and nobody watching the operators.
+// functional tensor, and no forward-mode tangent, which only torch operations carry on.
 bool plain(const at::Tensor& t) {
   const auto ks = t.key_set();
-  return t.is_cuda() && t.layout() == at::kStrided && t.has_storage() &&
+  return !t._fw_grad(0).defined() && t.is_cuda() && t.layout() == at::kStrided && t.has_storage() &&
          !ks.has(c10::DispatchKey::Python) && !ks.has(c10::DispatchKey::Functionalize) &&
          !ks.has(c10::DispatchKey::FuncTorchBatched) &&
          !ks.has(c10::DispatchKey::FuncTorchGradWrapper) && !t.is_neg() && !t.is_conj();
 }
 
+// Whether somebody watches the operators.
 bool watched() {
   return c10::impl::TorchDispatchModeTLS::any_modes_set() ||
          c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer) ||
@@ -72,10 +73,8 @@ std::optional<at::Tensor> linear_forward(const at::Tensor& x, const at::Tensor& 
   if (watched() || !plain(x) || !plain(wdev) || x.device() != wdev.device() || x.dim() < 1 ||
       x.size(-1) != K || K < 1 || x.numel() == 0)
     return std::nullopt;
-  // a bias of more dimensions broadcasts against the [M, N] product, not against y's shape; one
-  // with a forward-mode tangent gives y a tangent, which only a torch operation does
-  if (bias && (!plain(*bias) || bias->device() != x.device() || bias->dim() > 1 ||
-               bias->_fw_grad(0).defined()))
+  // a bias of more dimensions broadcasts against the [M, N] product, not against y's shape
+  if (bias && (!plain(*bias) || bias->device() != x.device() || bias->dim() > 1))
     return std::nullopt;
   const int xdt = dtype_code(x.scalar_type());
   if (xdt < 0) return std::nullopt;

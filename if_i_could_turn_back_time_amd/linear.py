@@ -292,8 +292,8 @@ _PLAIN = (torch.Tensor, nn.Parameter)
 
 def _vector_bias(bias, N: int) -> bool:
     """Whether bias is an ordinary [N] vector, which the kernels add and added_bias
-    (fourbit_torch.cpp) differentiates.  Any other one (a row per row of x, a single value, one with a forward-mode
-    tangent) broadcasts against the [M, N] product as a torch operation."""
+    (fourbit_torch.cpp) differentiates.  Any other one (a row per row of x, a single value, one
+    with a forward-mode tangent) broadcasts against the [M, N] product as a torch operation."""
     return (type(bias) in _PLAIN and bias.dim() == 1 and bias.shape[0] == N
             and unpack_dual(bias).tangent is None)
 

@@ -181,3 +181,29 @@ def test_forward_mode_tangent_of_the_bias(dev, lead, bdt):
                     p, ty = fwAD.unpack_dual(y)
                     assert torch.allclose(p, plain, rtol=1e-5, atol=1e-5)
                     assert ty is not None and torch.equal(ty, t.float().expand(*lead, N))
+
+
+@pytest.mark.parametrize("M", [5, 40])
+@pytest.mark.parametrize("block", [0, 256])
+@pytest.mark.parametrize("xdt", [torch.float32, torch.float16])
+def test_forward_mode_tangent_of_the_gradient(dev, M, block, xdt):
+    """A backward pass over a dual grad_y (forward over reverse, with a tangent from behind the
+    layer) gives the gradients' tangents: those of grad_y's tangent."""
+    K, N = 256, 40
+    if dev == "cpu":
+        xdt = torch.float32
+    wdev, w = _layer(dev, fwht_block=block)
+    x = torch.randn(M, K, device=dev, dtype=xdt, requires_grad=True)
+    bias = torch.randn(N, device=dev, requires_grad=True)
+    gy, t = (torch.randn(M, N, device=dev, dtype=xdt) for _ in range(2))
+    y = LN.packed_linear(wdev, N, K, "gf4", block, x, bias)
+    want = torch.autograd.grad(y, (x, bias), gy, retain_graph=True)
+    want_t = torch.autograd.grad(y, (x, bias), t, retain_graph=True)
+    with fwAD.dual_level():
+        got = torch.autograd.grad(y, (x, bias), fwAD.make_dual(gy, t))
+        for g, a, b in zip(got, want, want_t):
+            p, gt = fwAD.unpack_dual(g)
+            assert gt is not None
+            # the torch form rounds the bias's sum to grad_y's type first
+            assert torch.allclose(p, a, rtol=2e-3, atol=2e-3)
+            assert torch.allclose(gt, b, rtol=2e-3, atol=2e-3)
